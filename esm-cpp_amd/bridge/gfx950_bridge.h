@@ -72,7 +72,7 @@ bool RopeApplyVarlen(float* x, const float* cos, const float* sin, const int* cu
                      int num_heads, int head_dim);
 
 // esm::kernels::AttentionVarlen (kernels.h:119-121): the split-fp16 MFMA
-// kernel at head_dim 64 (fp32-level results), the scalar fp32 kernel for any
+// kernel at head_dim 64 (fp32-level results), the fp32 MFMA kernel for any
 // other head_dim <= 128.
 bool AttentionVarlen(const float* q, const float* k, const float* v, const int* cu_seqlens, int batch_size,
                      int num_heads, int head_dim, float* out);

@@ -203,7 +203,7 @@ hipError_t launch_attention_x3(const uint32_t* q, int ldq, const uint16_t* kh, c
 // (planes != null: hi at [r * ld_out + c], lo d elements further).
 hipError_t launch_pack_x3(const float* x, int ld_x, int rows, int d, float scale, uint32_t* words, uint16_t* planes,
                           int ld_out, hipStream_t s);
-// Exact fp32 path for any head_dim <= 128 (one thread per query).
+// Exact fp32 path for any head_dim <= 128 (fp32 MFMA, softmax sum in double).
 hipError_t launch_attention_f32(const float* q, const float* k, const float* v,
                                 int ld, int head_dim, const int* cu_seqlens,
                                 const AttnWork* work, int num_work, float* out,

@@ -52,7 +52,7 @@ enum {
  * [M,K] input, 1 when all zero); PER_TOKEN uses one such scale per row. */
 enum { ESM_GFX950_ACT_PER_TENSOR = 0, ESM_GFX950_ACT_PER_TOKEN = 1 };
 
-/* Attention arithmetic for esm_gfx950_attention_varlen. FP32: scalar fp32
+/* Attention arithmetic for esm_gfx950_attention_varlen. FP32: fp32 MFMA
  * kernel in the reference's operation order. BF16_MFMA: q/k rounded to bf16,
  * v and the probabilities to fp16, on MFMA. F16X3_MFMA: fp32 inputs, every
  * operand split into fp16 hi + lo and each product formed by three fp16
@@ -66,7 +66,7 @@ enum { ESM_GFX950_ATTN_FP32 = 0, ESM_GFX950_ATTN_BF16_MFMA = 1, ESM_GFX950_ATTN_
  * fp16, single fp16 MFMAs; BF16: Q/K as bf16. Those two halve the Q/K/V
  * traffic but round every attention operand once (about 3e-4 off the logit
  * correlation of a W8A8 network, whose int8 rounding amplifies any
- * perturbation). FP32: fp32 Q/K/V and the scalar fp32 kernel. */
+ * perturbation). FP32: fp32 Q/K/V and the fp32 MFMA kernel. */
 enum {
   ESM_GFX950_ATTN_MODE_FP16 = 0,
   ESM_GFX950_ATTN_MODE_BF16 = 1,

@@ -209,3 +209,35 @@ def test_cu_seqlens_validation(dev):
         dev.attention_varlen(x, x, x, np.array([1, 4], np.int32), H, dh, x)
     with pytest.raises(eg.Gfx950Error, match="non-decreasing"):
         dev.attention_varlen(x, x, x, np.array([0, 3, 2], np.int32), H, dh, x)
+
+
+class _Offset:
+    """A device array's data from element `first` on."""
+
+    def __init__(self, arr, first):
+        self.ptr = type(arr.ptr)(arr.ptr.value + first * arr.dtype.itemsize)
+
+
+@pytest.mark.parametrize("dh,shift", [(4, 0), (6, 0), (16, 0), (16, 1), (20, 0), (32, 0), (36, 1), (64, 0), (100, 0),
+                                      (128, 0)])
+def test_fp32_path_block_edges(dev, oracle, dh, shift):
+    """Lengths around the 16-key blocks and 64-query tiles, head widths around
+    the padded ones, operands off a 16-byte boundary; an infinite V in the
+    last key of a partial block reaches only what its weights reach. The
+    bound is the scores' rounding: q is scaled, |score| < 8, so an exponential
+    moves by at most 8 * 2^-24 * dh / 4 relative, under 1e-5 at dh 128."""
+    H, lengths = 3, [1, 15, 16, 17, 63, 64, 65, 129]
+    r = rng(dh + shift)
+    cu = cu_from_lengths(lengths)
+    T = int(cu[-1])
+    q, k, v = _qkv(r, T, H, dh)
+    v[cu[4] - 1, 1, dh - 1] = np.inf  # the last key of the 17-token sequence
+    pad = np.zeros(shift, np.float32)
+    arrs = [dev.array(np.concatenate([pad, x.ravel()])) for x in (q, k, v)]
+    out = dev.empty((T * H * dh + shift,), np.float32)
+    dev.attention_varlen(*(_Offset(a, shift) for a in arrs), cu, H, dh, _Offset(out, shift), eg.ATTN_FP32)
+    got = out.numpy()[shift:].reshape(T, H * dh)
+    want = oracle.attention_varlen(q, k, v, cu, H, dh)
+    assert np.array_equal(np.isinf(got), np.isinf(want)) and np.isinf(want).sum() == 17
+    fine = np.isfinite(want)
+    np.testing.assert_allclose(got[fine], want[fine], rtol=1e-5, atol=1e-5)
