@@ -170,4 +170,30 @@ __device__ __forceinline__ uint32_t quant_pack4(float4 v, float inv) {
   return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
 }
 
+constexpr int kGroupM = 8;  // row tiles walked together
+
+__device__ __forceinline__ int xcd_remap(int id, int num) {
+  constexpr int X = 8;
+  const int per = num / X, rem = num % X;
+  const int xcd = id % X, local = id / X;
+  return xcd * per + min(xcd, rem) + local;
+}
+
+// Output tile of GEMM workgroup `id`: ids are first spread so that each XCD
+// (workgroup id mod 8) owns a contiguous range, then walked in groups of
+// kGroupM row tiles so consecutive tiles on one XCD share W columns and A rows
+// in that XCD's L2.
+__device__ __forceinline__ void tile_origin_of(int id, int M, int N, int BM, int BN, int* m0, int* n0) {
+  const int tiles_m = (M + BM - 1) / BM;
+  const int tiles_n = (N + BN - 1) / BN;
+  const int pid = xcd_remap(id, tiles_m * tiles_n);
+  const int per_group = kGroupM * tiles_n;
+  const int group = pid / per_group;
+  const int first_m = group * kGroupM;
+  const int gsize = min(tiles_m - first_m, kGroupM);
+  const int in_group = pid - group * per_group;
+  *m0 = (first_m + in_group % gsize) * BM;
+  *n0 = (in_group / gsize) * BN;
+}
+
 }  // namespace esm_gfx950

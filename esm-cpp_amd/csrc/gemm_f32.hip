@@ -7,11 +7,18 @@
 // Products are exact fp32 products accumulated in fp32, so results differ
 // from the sequential reference sum only by summation order.
 //
-// Tiling: 128x128 workgroup tile, four waves of 64x64, 32-wide K stages in
-// LDS (row pitch 36 floats). Within a stage, lane group g (lane / 16) owns
-// the eight consecutive k values [8g, 8g+8): MFMA step j multiplies A and W
-// at k = 8g + j for every lane group, which keeps A and W consistent and
-// lets each lane fetch its k values with two 16-byte LDS reads.
+// Three kernels (launch_gemm_f32 picks):
+//   - gemm_f32_tile_kernel: aligned rows with K % 32 == 0; LDS tiles of 32x32
+//     to 128x64, direct global -> LDS stage loads;
+//   - gemm_f32_skinny_kernel: grids too small for that one (and the decoder's
+//     N <= 48): eight waves split K, operands straight into registers;
+//   - gemm_f32_kernel: any other shape (128x128 tiles through registers).
+//
+// gemm_f32_kernel's tiling: 128x128 workgroup tile, four waves of 64x64,
+// 32-wide K stages in LDS (row pitch 36 floats). Within a stage, lane group g
+// (lane / 16) owns the eight consecutive k values [8g, 8g+8): MFMA step j
+// multiplies A and W at k = 8g + j for every lane group, which keeps A and W
+// consistent and lets each lane fetch its k values with two 16-byte LDS reads.
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -278,72 +285,301 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_x3_kernel(const GemmX3Args p
   }
 }
 
-// ---- Narrow fp32 GEMM, N <= 48 (the tied decoder, d -> 33 logits): one wave
-// per 16 rows covers all 48 (padded) columns with v_mfma_f32_16x16x4f32.
-// Lane (r, g) = (lane % 16, lane / 16) loads a float4 of row r of A at
-// k = k0 + 4g and of rows r, r + 16, r + 32 of W; MFMA step j then multiplies
-// A[r][k0 + 4g + j] with W[c][k0 + 4g + j] for every lane group g, which sums
-// all 16 k of the stage over the four steps. W (N x K, 169 KB for the ESM
-// decoder) is re-read from L2 by every wave. K % 16 == 0.
-__global__ __launch_bounds__(256) void gemm_narrow_kernel(const GemmF32Args p) {
-  const int lane = threadIdx.x & 63;
-  const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
-  if (row0 >= p.M) return;
-  const int r = lane & 15, g = lane >> 4;
-  const float* arow = p.A + static_cast<size_t>(min(row0 + r, p.M - 1)) * p.lda + 4 * g;
-  const float* wrow[3];
-  bool wok[3];
+// ---- Tiled fp32 GEMM (K % 32 == 0, 16-byte aligned rows): 2 x 2 waves of
+// 16 MB x 16 NB outputs, a 32 MB x 32 NB workgroup tile.
+//
+// Staging is the INT8 kernel's: K advances 128 bytes (32 floats) a stage, one
+// global_load_lds_dwordx4 per 8 rows x 128 bytes, chunk c of row r at c ^ r
+// within its 1 KB block, two or three stage buffers and one barrier a stage.
+// A lane reads 16 bytes, k = 16 h + 4 lg .. + 4 of row lr, per half h of the
+// stage; MFMA step j multiplies k = 16 h + 4 lg + j. The operands are swapped
+// (W rows in the M dimension), so a lane's four accumulators are four
+// consecutive columns of one row and go out as one 16-byte store.
+//
+// v_mfma_f32_16x16x4_f32 takes 32 cycles for 512 operand bytes, so neither LDS
+// nor the stage loads bound the loop; what does is the matrix rate times how
+// evenly the tiles fall on the CUs (f32_tile_of). 1280 x 1280 at 7,777 rows:
+// 303 us with 128x128 tiles staged through registers, 199 here (128 TFLOP/s;
+// 165 us at the rate of a large fp32 library product); at 66 rows and K = N =
+// 320, 33 -> 4.8 us.
+template <int MB, int NB>
+struct F32Tile {
+  static constexpr int BM = 32 * MB, BN = 32 * NB;
+  static constexpr int kBlocks = (BM + BN) / 8;  // 1 KB blocks per stage
+  static constexpr int kPer = kBlocks / 4;       // per wave
+  static constexpr int kStage = kBlocks * 1024;
+  // More buffers only cost resident workgroups (1280 x 1280 at 1,000 rows,
+  // 32x32 tiles: 33 us with three, 39 with five).
+  static constexpr int kNStage = kStage <= 16384 ? 3 : 2;
+  // A single 16x16 block per wave would be one chain of dependent MFMAs, 52
+  // cycles each instead of the 32 they occupy the matrix core: its halves of a
+  // stage go to two accumulators.
+  static constexpr int kChains = MB * NB == 1 ? 2 : 1;
+};
+
+// One 16-byte-per-lane global -> LDS load, as in the INT8 kernel: uniform
+// base, 32-bit lane offset, LDS byte address in M0; awaited by the explicit
+// vmcnt before the barrier that publishes the stage.
+__device__ __forceinline__ void f32_dma16(const void* base, uint32_t off, uint32_t lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0v)
+               : "memory", "m0");
+#endif
+}
+
+// Output of four consecutive columns of one row, the epilogue applied.
+template <int EPI>
+__device__ __forceinline__ void f32_store4(const GemmF32Args& p, int row, int col, f32x4 v, bool vec_c) {
+  if (row >= p.M || col >= p.N) return;
+  float* dst = p.C + static_cast<size_t>(row) * p.ldc + col;
+  const int n = min(4, p.N - col);
 #pragma unroll
-  for (int nb = 0; nb < 3; ++nb) {
-    const int c = nb * 16 + r;
-    wok[nb] = c < p.N;
-    wrow[nb] = p.W + static_cast<size_t>(min(c, p.N - 1)) * p.ldw + 4 * g;
+  for (int e = 0; e < 4; ++e) {
+    v[e] += p.bias && e < n ? p.bias[col + e] : 0.0f;
+    if constexpr (EPI == kF32Gelu) v[e] = gelu_erf(v[e]);
   }
-  f32x4 acc[3];
+  if (vec_c && n == 4) {
+    if constexpr (EPI == kF32Resid) v = *reinterpret_cast<const f32x4*>(dst) + v;
+    *reinterpret_cast<f32x4*>(dst) = v;
+  } else {
 #pragma unroll
-  for (int nb = 0; nb < 3; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
-  f32x4 a = *reinterpret_cast<const f32x4*>(arow);
-  f32x4 b[3];
+    for (int e = 0; e < 4; ++e)
+      if (e < n) dst[e] = EPI == kF32Resid ? dst[e] + v[e] : v[e];
+  }
+}
+
+template <int MB, int NB, int EPI>
+__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p, bool vec_c) {
+  using TL = F32Tile<MB, NB>;
+  constexpr int BM = TL::BM, BN = TL::BN, kPer = TL::kPer, kStage = TL::kStage, kNStage = TL::kNStage;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kNStage * kStage];
+  int m0, n0;
+  tile_origin_of(blockIdx.x, p.M, p.N, BM, BN, &m0, &n0);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+  const int lr = lane & 15, lg = lane >> 4;
+
+  // Blocks wave * kPer .. of a stage: [0, BM / 8) are A row groups, the rest
+  // W row groups; rows past the edge re-read the last valid row.
+  uint32_t goff[kPer];
 #pragma unroll
-  for (int nb = 0; nb < 3; ++nb) b[nb] = *reinterpret_cast<const f32x4*>(wrow[nb]);
-  for (int k0 = 0; k0 < p.K; k0 += 16) {
-    f32x4 an = a, bn[3] = {b[0], b[1], b[2]};
-    if (k0 + 16 < p.K) {
-      an = *reinterpret_cast<const f32x4*>(arow + k0 + 16);
+  for (int i = 0; i < kPer; ++i) {
+    const int b = wave * kPer + i;
+    const int r = lane >> 3, c = (lane & 7) ^ r;
+    const bool is_a = b < BM / 8;
+    const int row = is_a ? min(m0 + b * 8 + r, p.M - 1) : min(n0 + (b - BM / 8) * 8 + r, p.N - 1);
+    goff[i] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(is_a ? p.lda : p.ldw) + c * 4) * 4u;
+  }
+  const uint32_t lds0 = static_cast<uint32_t>(
+      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)smem));
+  auto load_stage = [&](int kt, int buf) {
 #pragma unroll
-      for (int nb = 0; nb < 3; ++nb) bn[nb] = *reinterpret_cast<const f32x4*>(wrow[nb] + k0 + 16);
+    for (int i = 0; i < kPer; ++i)
+      f32_dma16((wave * kPer + i < BM / 8 ? p.A : p.W) + kt * 32, goff[i],
+                lds0 + static_cast<uint32_t>(buf * kStage + (wave * kPer + i) * 1024));
+  };
+  const int nk = p.K / 32;
+#pragma unroll
+  for (int st = 0; st < kNStage - 1; ++st)
+    if (st < nk) load_stage(st, st);
+
+  constexpr int kChains = TL::kChains;
+  f32x4 acc[kChains][MB][NB];
+#pragma unroll
+  for (int x = 0; x < kChains; ++x)
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[x][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Row R's chunk c of a stage: block R / 8, slot c ^ (R % 8).
+  const int arow = wm * 16 * MB + lr, wrow = BM + wn * 16 * NB + lr;
+  auto frag = [&](const uint8_t* st, int R, int h) {
+    return *reinterpret_cast<const f32x4*>(st + (R >> 3) * 1024 + (R & 7) * 128 + (((4 * h + lg) ^ (R & 7)) << 4));
+  };
+  int buf = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    // Stage kt has landed (this wave's loads, then everyone's behind the
+    // barrier), and every wave is done with stage kt - 1, whose buffer
+    // receives stage kt + kNStage - 1.
+    if (kNStage == 3 && kt + 1 < nk)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPer) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt + kNStage - 1 < nk) load_stage(kt + kNStage - 1, buf == 0 ? kNStage - 1 : buf - 1);
+    const uint8_t* st = smem + buf * kStage;
+    buf = buf + 1 == kNStage ? 0 : buf + 1;
+    // The chains of a single-block wave advance together; otherwise one half
+    // of the stage at a time keeps fewer fragments live.
+#pragma unroll
+    for (int h0 = 0; h0 < 2; h0 += kChains) {
+      f32x4 fa[kChains][MB], fw[kChains][NB];
+#pragma unroll
+      for (int x = 0; x < kChains; ++x) {
+#pragma unroll
+        for (int i = 0; i < MB; ++i) fa[x][i] = frag(st, arow + 16 * i, h0 + x);
+#pragma unroll
+        for (int j = 0; j < NB; ++j) fw[x][j] = frag(st, wrow + 16 * j, h0 + x);
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int x = 0; x < kChains; ++x)
+#pragma unroll
+          for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+              acc[x][i][j] =
+                  __builtin_amdgcn_mfma_f32_16x16x4f32(fw[x][j][e], fa[x][i][e], acc[x][i][j], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      f32x4 v = acc[0][i][j];
+      if constexpr (kChains == 2) v += acc[1][i][j];
+      f32_store4<EPI>(p, m0 + wm * 16 * MB + 16 * i + lr, n0 + wn * 16 * NB + 16 * j + 4 * lg, v, vec_c);
+    }
+}
+
+// ---- Skinny fp32 GEMM (K % 16 == 0): a 16 MB x 16 NB output tile whose K is
+// split over the workgroup's eight waves. Each wave loads its 16-wide K steps
+// straight into registers (lane (lr, lg): k = 16 s + 4 lg .. + 4 of row lr), CH
+// steps in flight at once, and the waves' sums meet in LDS in wave order. It
+// is for grids of few tiles, where one wave's walk over all of K, a load
+// latency per step, is what the launch takes.
+constexpr int kSkinnyWaves = 8;
+template <int MB, int NB, int CH, int EPI>
+__global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_f32_skinny_kernel(const GemmF32Args p, bool vec_c) {
+  __shared__ f32x4 part[kSkinnyWaves][MB * NB][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int m0 = blockIdx.x * 16 * MB, n0 = blockIdx.y * 16 * NB;
+  const float* arow[MB];
+  const float* wrow[NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i) arow[i] = p.A + static_cast<size_t>(min(m0 + 16 * i + lr, p.M - 1)) * p.lda + 4 * lg;
+#pragma unroll
+  for (int j = 0; j < NB; ++j) wrow[j] = p.W + static_cast<size_t>(min(n0 + 16 * j + lr, p.N - 1)) * p.ldw + 4 * lg;
+  f32x4 acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = p.K / 16;
+  const int s0 = steps * wave / kSkinnyWaves, s1 = steps * (wave + 1) / kSkinnyWaves;
+  for (int s = s0; s < s1; s += CH) {
+    f32x4 fa[CH][MB], fw[CH][NB];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int k0 = 16 * min(s + u, s1 - 1);  // past the range: its last step again, unused
+#pragma unroll
+      for (int i = 0; i < MB; ++i) fa[u][i] = *reinterpret_cast<const f32x4*>(arow[i] + k0);
+#pragma unroll
+      for (int j = 0; j < NB; ++j) fw[u][j] = *reinterpret_cast<const f32x4*>(wrow[j] + k0);
     }
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int u = 0; u < CH; ++u)
+      if (s + u < s1) {
 #pragma unroll
-      for (int nb = 0; nb < 3; ++nb)
-        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], wok[nb] ? b[nb][j] : 0.0f, acc[nb], 0, 0, 0);
-    a = an;
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-    for (int nb = 0; nb < 3; ++nb) b[nb] = bn[nb];
+          for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[u][j][e], fa[u][i][e], acc[i][j], 0, 0, 0);
+      }
   }
-  // Output element i of block nb in lane (r, g): row row0 + 4g + i, column nb*16 + r.
 #pragma unroll
-  for (int nb = 0; nb < 3; ++nb) {
-    const int col = nb * 16 + r;
-    if (col >= p.N) continue;
-    const float bias = p.bias ? p.bias[col] : 0.0f;
+  for (int i = 0; i < MB; ++i)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int row = row0 + 4 * g + i;
-      if (row < p.M) p.C[static_cast<size_t>(row) * p.ldc + col] = acc[nb][i] + bias;
+    for (int j = 0; j < NB; ++j) part[wave][i * NB + j][lane] = acc[i][j];
+  __syncthreads();
+  // Wave w finishes block w.
+  if (wave >= MB * NB) return;
+  f32x4 v = part[0][wave][lane];
+#pragma unroll
+  for (int w = 1; w < kSkinnyWaves; ++w) v += part[w][wave][lane];
+  f32_store4<EPI>(p, m0 + 16 * (wave / NB) + lr, n0 + 16 * (wave % NB) + 4 * lg, v, vec_c);
+}
+
+}  // namespace
+
+namespace {
+
+bool f32_vec_c(const GemmF32Args& p) { return p.ldc % 4 == 0 && reinterpret_cast<uintptr_t>(p.C) % 16 == 0; }
+
+// One EPI of a kernel template instantiated for each fp32 epilogue.
+#define ESM_F32_EPI(KERNEL, ...)                                                              \
+  switch (epi) {                                                                              \
+    case kF32Store: hipLaunchKernelGGL((KERNEL<__VA_ARGS__, kF32Store>), grid, block, 0, s, p, vec_c); break; \
+    case kF32Gelu: hipLaunchKernelGGL((KERNEL<__VA_ARGS__, kF32Gelu>), grid, block, 0, s, p, vec_c); break;   \
+    case kF32Resid: hipLaunchKernelGGL((KERNEL<__VA_ARGS__, kF32Resid>), grid, block, 0, s, p, vec_c); break; \
+    default: return hipErrorInvalidValue;                                                     \
+  }                                                                                           \
+  return hipGetLastError()
+
+template <int MB, int NB>
+hipError_t launch_f32_tile(const GemmF32Args& p, int epi, hipStream_t s) {
+  using TL = F32Tile<MB, NB>;
+  const bool vec_c = f32_vec_c(p);
+  const dim3 grid(((p.M + TL::BM - 1) / TL::BM) * ((p.N + TL::BN - 1) / TL::BN)), block(256);
+  ESM_F32_EPI(gemm_f32_tile_kernel, MB, NB);
+}
+
+template <int MB, int NB, int CH>
+hipError_t launch_f32_skinny(const GemmF32Args& p, int epi, hipStream_t s) {
+  const bool vec_c = f32_vec_c(p);
+  const dim3 grid((p.M + 16 * MB - 1) / (16 * MB), (p.N + 16 * NB - 1) / (16 * NB)), block(kSkinnyWaves * 64);
+  ESM_F32_EPI(gemm_f32_skinny_kernel, MB, NB, CH);
+}
+
+bool f32_skinny_ok(const GemmF32Args& p) {
+  return p.K > 0 && p.K % 16 == 0 && p.lda % 4 == 0 && p.ldw % 4 == 0;
+}
+
+// The stage loads take 16-byte aligned rows and 32-bit lane offsets.
+bool f32_tile_ok(const GemmF32Args& p) {
+  constexpr uint64_t kLimit = 1ull << 32;
+  return p.K > 0 && p.K % 32 == 0 && p.lda % 4 == 0 && p.ldw % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.W)) % 16 == 0 &&
+         static_cast<uint64_t>(p.M) * p.lda * 4 <= kLimit && static_cast<uint64_t>(p.N) * p.ldw * 4 <= kLimit;
+}
+
+// Index into {32x32, 64x64, 128x64}: the tile whose grid takes the least
+// time, (the most tiles any CU gets + 1/2) x the tile's outputs x its cost per
+// output. The costs are those of many rounds (2560 x 2560 at 16,000 rows:
+// 1,727 / 1,529 / 1,498 us); the half tile is the last round, in which a CU's
+// few remaining workgroups leave its matrix cores waiting. It follows the
+// measured order at 1280 x 1280: 33 / 44 / 48 us at 1,000 rows, 56 / 62 / 79 at
+// 1,768, 94 / 84 / 81 at 3,000, 224 / 199 / 230 at 7,777, 457 / 393 / 389 at
+// 16,000. (64x32 and 128x128 tiles were never more than 8% faster.)
+int f32_tile_of(int M, int N) {
+  static constexpr int kBM[3] = {32, 64, 128}, kBN[3] = {32, 64, 64};
+  static constexpr double kCost[3] = {1.17, 1.02, 1.0};
+  const int cus = device_cus();
+  int best = 0;
+  double best_t = 0.0;
+  for (int t = 0; t < 3; ++t) {
+    const long tiles = static_cast<long>((M + kBM[t] - 1) / kBM[t]) * ((N + kBN[t] - 1) / kBN[t]);
+    const double c = (static_cast<double>((tiles + cus - 1) / cus) + 0.5) * kBM[t] * kBN[t] * kCost[t];
+    if (t == 0 || c < best_t) {
+      best = t;
+      best_t = c;
     }
   }
+  return best;
 }
 
 }  // namespace
 
 hipError_t launch_gemm_narrow(const GemmF32Args& p, hipStream_t s) {
   if (p.M <= 0 || p.N <= 0) return hipSuccess;
-  if (p.N > 48 || p.K <= 0 || p.K % 16 != 0 || p.lda % 4 != 0 || p.ldw % 4 != 0) return hipErrorInvalidValue;
-  const int waves = (p.M + 15) / 16;
-  hipLaunchKernelGGL(gemm_narrow_kernel, dim3((waves + 3) / 4), dim3(256), 0, s, p);
-  return hipGetLastError();
+  if (p.N > 48 || !f32_skinny_ok(p)) return hipErrorInvalidValue;
+  // 32 rows a workgroup halve the reads of W once there are enough of them.
+  if (p.M > 4096) return launch_f32_skinny<2, 3, 4>(p, kF32Store, s);
+  return launch_f32_skinny<1, 3, 5>(p, kF32Store, s);
 }
 
 hipError_t launch_gemm_x3(const GemmX3Args& p, int epi, hipStream_t s) {
@@ -362,6 +598,19 @@ hipError_t launch_gemm_x3(const GemmX3Args& p, int epi, hipStream_t s) {
 
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epi, hipStream_t s) {
   if (p.M <= 0 || p.N <= 0) return hipSuccess;
+  // At most one 16x16-tile workgroup a CU and a K long enough to be worth
+  // splitting: N = 320 at 66 rows takes 6.4 / 6.5 / 6.6 / 6.7 us skinny for K
+  // = 320 / 480 / 960 / 1280 against 4.8 / 6.0 / 9.7 / 12.2 in 32x32 tiles; a
+  // second round of workgroups (301 rows) 11.4 against 12.4 at K = 1280.
+  const long tiles16 = static_cast<long>((p.M + 15) / 16) * ((p.N + 15) / 16);
+  if (f32_skinny_ok(p) && p.K >= 512 && tiles16 <= device_cus()) return launch_f32_skinny<1, 1, 10>(p, epi, s);
+  if (f32_tile_ok(p)) {
+    switch (f32_tile_of(p.M, p.N)) {
+      case 0: return launch_f32_tile<1, 1>(p, epi, s);
+      case 1: return launch_f32_tile<2, 2>(p, epi, s);
+      default: return launch_f32_tile<4, 2>(p, epi, s);
+    }
+  }
   const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
   const dim3 grid(tiles), block(kThreads);
   const bool vec = (p.K % 4 == 0) && (p.lda % 4 == 0) && (p.ldw % 4 == 0);

@@ -102,6 +102,39 @@ def test_linear_f32(dev, oracle, M, N, K):
     assert np.all(np.abs(got - want) <= 1e-4 * (1 + np.abs(want)))
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 512), (16, 16, 528), (17, 33, 1024), (65, 47, 1280), (1, 4, 32), (31, 33, 64), (33, 31, 96), (64, 64, 32),
+    (65, 130, 320), (1000, 333, 64), (2049, 1030, 96), (4133, 640, 128), (9000, 322, 32),
+])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_linear_f32_tile_edges(dev, M, N, K, shift):
+    """Edges of the K-split tiles (16 x 16, K steps of 16) and of the 32x32,
+    64x64 and 128x64 tiles, an N that is no multiple of 4, one stage and odd
+    stage counts; shift 1 moves every operand off its 16-byte boundary (the
+    general kernel). Bound: a sum of K products, each rounding at most 2^-24 of
+    the sum of magnitudes, 2^-24 * K * sum |a w| at worst."""
+    r = rng(M + N + K)
+    A = r.uniform(-1, 1, size=(M, K)).astype(np.float32)
+    W = r.uniform(-1, 1, size=(N, K)).astype(np.float32)
+    b = r.uniform(-1, 1, size=N).astype(np.float32) if (M + N) % 2 else None
+
+    def at(x):
+        a = dev.array(np.concatenate([np.zeros(shift, np.float32), x.ravel()]))
+        a.ptr = type(a.ptr)(a.ptr.value + 4 * shift)
+        keep.append(a)
+        return a
+
+    keep = []
+    out = at(np.full((M, N), np.nan, np.float32))
+    dev.linear_f32(at(A), at(W), at(b) if b is not None else None, out, M, N, K)
+    for a in keep:
+        a.ptr = type(a.ptr)(a.ptr.value - 4 * shift)
+    got = out.numpy()[shift:].reshape(M, N)
+    A64, W64 = A.astype(np.float64), W.astype(np.float64)
+    want = A64 @ W64.T + (0 if b is None else b)
+    assert np.all(np.abs(got - want) <= 2.0**-24 * K * (np.abs(A64) @ np.abs(W64).T + 1))
+
+
 def test_linear_f32_known_answer(dev):
     """Reference tests/cpp/test_kernels.cpp:88-111."""
     A = np.array([[1, 2, 3], [4, 5, 6]], np.float32)
