@@ -249,7 +249,8 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
 //
 // Every operand is split into hi + lo fp16 parts (hi = fp16(x), lo =
 // fp16(x - hi): 22 significant bits together), written by the QKV GEMM
-// epilogue after RoPE (or by launch_pack_x3 for the op-level entry), and each
+// epilogue after RoPE (or by this kernel from fp32 rows, for the op-level
+// entry), and each
 // product uses three MFMAs: hi*hi + lo*hi + hi*lo (the dropped lo*lo term is
 // below 2^-22 relative). Q comes multiplied by a power of two (q_prescale) so
 // the lo parts of the small pre-scaled Q stay normal fp16; the factor is
@@ -357,11 +358,24 @@ __device__ __forceinline__ void split8(const float (&p)[8], f16x8* hi, f16x8* lo
 // batches keep the unconditional rescale: there the leaner loop ran as fast
 // in isolation, but beside the second sequence group's kernels the
 // configuration-4 forward got 1% slower.
-template <bool LONG>
-__global__ __launch_bounds__(256, 4) void attn_x3_kernel(
+//
+// F32: Q, K and V arrive as fp32 rows (the op-level entry) and are split here,
+// into the same operands bit for bit: thread (row, c) of a chunk loads the
+// eight dims of the row's 16-byte plane chunk c (4 c .. + 4 and 32 + 4 c .. +
+// 4) of K and V while the previous chunk is computed, and writes their hi and
+// lo parts to the other buffer after it. A packing pass would write and
+// re-read every operand: 64 sequences around 120 tokens (20 heads) took 76 us
+// in three packing launches plus 35 here, 41 us without them. The 16
+// registers of the chunk in flight leave three workgroups a CU.
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // any fp32 address
+
+template <bool LONG, bool F32>
+__global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
     const uint32_t* __restrict__ q, int ldq, const uint16_t* __restrict__ kh, const uint16_t* __restrict__ kl,
-    const uint16_t* __restrict__ vh, const uint16_t* __restrict__ vl, int ldp, float s2, const int* __restrict__ cu,
-    const AttnWork* __restrict__ work, float* __restrict__ out, int ld_out, float* __restrict__ part_max) {
+    const uint16_t* __restrict__ vh, const uint16_t* __restrict__ vl, int ldp, const float* __restrict__ fq,
+    const float* __restrict__ fk, const float* __restrict__ fv, int ldf, float q_prescale, float s2,
+    const int* __restrict__ cu, const AttnWork* __restrict__ work, float* __restrict__ out, int ld_out,
+    float* __restrict__ part_max) {
   // Two chunk buffers, each [K hi | K lo | V hi | V lo] planes of 64 rows x
   // 128 bytes.
   __shared__ __attribute__((aligned(1024))) uint8_t sbuf[2 * kChunkBytes];
@@ -408,23 +422,75 @@ __global__ __launch_bounds__(256, 4) void attn_x3_kernel(
   // block qb, positions [lg*8, lg*8+8) and [32+lg*8, 32+lg*8+8). The Q words
   // are loaded first and chunk 0 right behind them, so both round trips
   // overlap.
-  uint4 qw[2][2][2];
-#pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
-    const int qi = min(qbase + qb * 16 + lr, L - 1);
-    const uint32_t* qp = q + static_cast<size_t>(start + qi) * ldq + hoff;
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      qw[qb][half][0] = *reinterpret_cast<const uint4*>(qp + half * 32 + lg * 8);
-      qw[qb][half][1] = *reinterpret_cast<const uint4*>(qp + half * 32 + lg * 8 + 4);
-    }
-  }
-  load_chunk(0, 0);
   f16x8 qh[2][2], ql[2][2];
+  f32x4u kr[2], vr[2];  // F32: the next chunk's dims of this thread
+  // F32: this thread's row and 16-byte plane chunk of a key chunk.
+  const int crow = tid >> 3, cc = tid & 7;
+  auto load_f32 = [&](int kc) {
+    const size_t at = static_cast<size_t>(start + kc + min(crow, min(KCX, L - kc) - 1)) * ldf + hoff + 4 * cc;
+    kr[0] = *reinterpret_cast<const f32x4u*>(fk + at);
+    kr[1] = *reinterpret_cast<const f32x4u*>(fk + at + 32);
+    vr[0] = *reinterpret_cast<const f32x4u*>(fv + at);
+    vr[1] = *reinterpret_cast<const f32x4u*>(fv + at + 32);
+  };
+  auto store_f32 = [&](int buf) {
+    uint8_t* row = sbuf + buf * kChunkBytes + crow * 128;
+    uint32_t h[4], l[4];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+    for (int j = 0; j < 4; ++j) split_pair(kr[0][j], kr[1][j], &h[j], &l[j]);
+    const int ko = (cc ^ swz_k(crow)) << 4;
+    *reinterpret_cast<uint4*>(row + ko) = make_uint4(h[0], h[1], h[2], h[3]);
+    *reinterpret_cast<uint4*>(row + kPlaneBytes + ko) = make_uint4(l[0], l[1], l[2], l[3]);
 #pragma unroll
-    for (int half = 0; half < 2; ++half) unpack8(qw[qb][half][0], qw[qb][half][1], &qh[qb][half], &ql[qb][half]);
+    for (int j = 0; j < 4; ++j) split_pair(vr[0][j], vr[1][j], &h[j], &l[j]);
+    const int vo = (cc ^ swz_v(crow)) << 4;
+    *reinterpret_cast<uint4*>(row + 2 * kPlaneBytes + vo) = make_uint4(h[0], h[1], h[2], h[3]);
+    *reinterpret_cast<uint4*>(row + 3 * kPlaneBytes + vo) = make_uint4(l[0], l[1], l[2], l[3]);
+  };
+  if constexpr (F32) {
+    // Positions 32 half + 8 lg .. + 8 are dims 16 half + 4 lg .. + 4 and those
+    // + 32, paired.
+    f32x4u x[2][2][2];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      const float* qp = fq + static_cast<size_t>(start + min(qbase + qb * 16 + lr, L - 1)) * ldf + hoff + 4 * lg;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        x[qb][half][0] = *reinterpret_cast<const f32x4u*>(qp + 16 * half);
+        x[qb][half][1] = *reinterpret_cast<const f32x4u*>(qp + 16 * half + 32);
+      }
+    }
+    load_f32(0);
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          split_pair(x[qb][half][0][j] * q_prescale, x[qb][half][1][j] * q_prescale, &h[j], &l[j]);
+        qh[qb][half] = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4*>(h));
+        ql[qb][half] = __builtin_bit_cast(f16x8, *reinterpret_cast<const uint4*>(l));
+      }
+    store_f32(0);
+  } else {
+    uint4 qw[2][2][2];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+      const int qi = min(qbase + qb * 16 + lr, L - 1);
+      const uint32_t* qp = q + static_cast<size_t>(start + qi) * ldq + hoff;
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        qw[qb][half][0] = *reinterpret_cast<const uint4*>(qp + half * 32 + lg * 8);
+        qw[qb][half][1] = *reinterpret_cast<const uint4*>(qp + half * 32 + lg * 8 + 4);
+      }
+    }
+    load_chunk(0, 0);
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+      for (int half = 0; half < 2; ++half) unpack8(qw[qb][half][0], qw[qb][half][1], &qh[qb][half], &ql[qb][half]);
+  }
 
   f32x4 o[2][4];
 #pragma unroll
@@ -454,7 +520,12 @@ __global__ __launch_bounds__(256, 4) void attn_x3_kernel(
     // everyone's and retires the previous chunk's reads of the other buffer,
     // which then receives the next chunk, in flight during this one.
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (kc0 + KCX < L) load_chunk(kc0 + KCX, buf ^ 1);
+    if (kc0 + KCX < L) {
+      if constexpr (F32)
+        load_f32(kc0 + KCX);
+      else
+        load_chunk(kc0 + KCX, buf ^ 1);
+    }
     if (!active) return;
     const uint8_t* sKh = sbuf + buf * kChunkBytes;
     const uint8_t* sKl = sKh + kPlaneBytes;
@@ -567,7 +638,12 @@ __global__ __launch_bounds__(256, 4) void attn_x3_kernel(
 
   // Whole chunks, then the sequence's partial last chunk (if any).
   int kc0 = 0, buf = 0;
-  for (; kc0 + KCX <= L; kc0 += KCX, buf ^= 1) chunk(kc0, KCX, buf, std::true_type{});
+  for (; kc0 + KCX <= L; kc0 += KCX, buf ^= 1) {
+    chunk(kc0, KCX, buf, std::true_type{});
+    // The other buffer's last reads ended before this chunk's barrier.
+    if constexpr (F32)
+      if (kc0 + KCX < L) store_f32(buf ^ 1);
+  }
   if (kc0 < L) {
     chunk(kc0, L - kc0, buf, std::false_type{});
     buf ^= 1;
@@ -614,28 +690,6 @@ __global__ __launch_bounds__(256, 4) void attn_x3_kernel(
   if (part_max) {
     m = wave_max(m);
     if (lane == 0) part_max[blockIdx.x * 4 + wave] = m;
-  }
-}
-
-// fp32 rows -> the split-fp16 kernel's operand layout (head_dim 64, positions
-// 0, 32, 1, 33, ... within each head): planes == 0, split words (x * scale)
-// at out_w[r * ld_out + c]; planes != 0, fp16 hi parts at out_h[r * ld_out +
-// c] and lo parts d elements further.
-__global__ void pack_x3_kernel(const float* __restrict__ x, int ld_x, int rows, int d, float scale, int planes,
-                               uint32_t* __restrict__ out_w, uint16_t* __restrict__ out_h, int ld_out) {
-  const size_t total = static_cast<size_t>(rows) * d;
-  for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < total;
-       i += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const size_t r = i / d;
-    const int c = static_cast<int>(i % d);
-    const int pos = c & 63, dim = (c & ~63) + (pos >> 1) + ((pos & 1) << 5);
-    const uint32_t wv = split_f16_word(x[r * ld_x + dim] * scale);
-    if (planes) {
-      out_h[r * ld_out + c] = static_cast<uint16_t>(wv & 0xffffu);
-      out_h[r * ld_out + d + c] = static_cast<uint16_t>(wv >> 16);
-    } else {
-      out_w[r * ld_out + c] = wv;
-    }
   }
 }
 
@@ -847,23 +901,25 @@ hipError_t launch_attention_x3(const uint32_t* q, int ldq, const uint16_t* kh, c
   if (num_work <= 0) return hipSuccess;
   const float s2 = kLog2e / q_prescale;
   if (max_len > kAttnLongSeq)
-    hipLaunchKernelGGL(attn_x3_kernel<true>, dim3(num_work), dim3(256), 0, s, q, ldq, kh, kl, vh, vl, ldp, s2,
-                       cu_seqlens, work, out, ld_out, part_max);
+    hipLaunchKernelGGL((attn_x3_kernel<true, false>), dim3(num_work), dim3(256), 0, s, q, ldq, kh, kl, vh, vl, ldp,
+                       nullptr, nullptr, nullptr, 0, q_prescale, s2, cu_seqlens, work, out, ld_out, part_max);
   else
-    hipLaunchKernelGGL(attn_x3_kernel<false>, dim3(num_work), dim3(256), 0, s, q, ldq, kh, kl, vh, vl, ldp, s2,
-                       cu_seqlens, work, out, ld_out, part_max);
+    hipLaunchKernelGGL((attn_x3_kernel<false, false>), dim3(num_work), dim3(256), 0, s, q, ldq, kh, kl, vh, vl, ldp,
+                       nullptr, nullptr, nullptr, 0, q_prescale, s2, cu_seqlens, work, out, ld_out, part_max);
   return hipGetLastError();
 }
 
-hipError_t launch_pack_x3(const float* x, int ld_x, int rows, int d, float scale, uint32_t* words, uint16_t* planes,
-                          int ld_out, hipStream_t s) {
-  const size_t n = static_cast<size_t>(rows) * d;
-  if (n == 0) return hipSuccess;
-  if (d % 64 != 0 || (words == nullptr) == (planes == nullptr)) return hipErrorInvalidValue;
-  size_t g = (n + 255) / 256;
-  if (g > 65536) g = 65536;
-  hipLaunchKernelGGL(pack_x3_kernel, dim3(static_cast<unsigned>(g)), dim3(256), 0, s, x, ld_x, rows, d, scale,
-                     planes ? 1 : 0, words, planes, ld_out);
+hipError_t launch_attention_x3_f32(const float* q, const float* k, const float* v, int ld, float q_prescale,
+                                   const int* cu_seqlens, const AttnWork* work, int num_work, float* out, int ld_out,
+                                   int max_len, hipStream_t s) {
+  if (num_work <= 0) return hipSuccess;
+  const float s2 = kLog2e / q_prescale;
+  if (max_len > kAttnLongSeq)
+    hipLaunchKernelGGL((attn_x3_kernel<true, true>), dim3(num_work), dim3(256), 0, s, nullptr, 0, nullptr, nullptr,
+                       nullptr, nullptr, 0, q, k, v, ld, q_prescale, s2, cu_seqlens, work, out, ld_out, nullptr);
+  else
+    hipLaunchKernelGGL((attn_x3_kernel<false, true>), dim3(num_work), dim3(256), 0, s, nullptr, 0, nullptr, nullptr,
+                       nullptr, nullptr, 0, q, k, v, ld, q_prescale, s2, cu_seqlens, work, out, ld_out, nullptr);
   return hipGetLastError();
 }
 

@@ -754,28 +754,17 @@ extern "C" int esm_gfx950_attention_varlen(esm_gfx950_ctx* ctx, const float* q, 
     return ctx->fail(ESM_GFX950_INVALID_ARGUMENT, "attention_varlen: unknown precision");
   ESM_REQUIRE(ctx, head_dim == kHeadDimMfma, "attention_varlen: the MFMA path needs head_dim == 64");
   if (precision == ESM_GFX950_ATTN_F16X3_MFMA) {
-    // Pack the fp32 operands into split-fp16 words (Q times kQPrescale), then
-    // run the split-fp16 kernel.
-    const size_t n = static_cast<size_t>(T) * ld;
-    const size_t wbytes = align_up(n * 4, 256);
+    // The kernel splits the fp32 operands itself (Q times kQPrescale).
     int* d_cu;
     AttnWork* d_work;
     int nwork;
-    ESM_TRY(stage_attention_meta(ctx, cu_seqlens, batch_size, num_heads, kAttnMfmaQTile, 3 * wbytes, &d_cu, &d_work,
-                                 &nwork, true));
-    char* base = static_cast<char*>(ctx->scratch);
-    auto* qw = reinterpret_cast<uint32_t*>(base);
-    auto* kp = reinterpret_cast<uint16_t*>(base + wbytes);      // [T, 2 ld]: hi | lo
-    auto* vp = reinterpret_cast<uint16_t*>(base + 2 * wbytes);
-    ESM_HIP(ctx, launch_pack_x3(q, ld, T, ld, kQPrescale, qw, nullptr, ld, ctx->stream));
-    ESM_HIP(ctx, launch_pack_x3(k, ld, T, ld, 1.0f, nullptr, kp, 2 * ld, ctx->stream));
-    ESM_HIP(ctx, launch_pack_x3(v, ld, T, ld, 1.0f, nullptr, vp, 2 * ld, ctx->stream));
+    ESM_TRY(stage_attention_meta(ctx, cu_seqlens, batch_size, num_heads, kAttnMfmaQTile, 0, &d_cu, &d_work, &nwork,
+                                 true));
     int max_len = 0;
     for (int b = 0; b < batch_size; ++b) max_len = std::max(max_len, cu_seqlens[b + 1] - cu_seqlens[b]);
     int slot;
     ESM_TRY(ctx->time_begin("attention", &slot));
-    ESM_HIP(ctx, launch_attention_x3(qw, ld, kp, kp + ld, vp, vp + ld, 2 * ld, kQPrescale, d_cu, d_work, nwork, out,
-                                     ld, max_len, ctx->stream));
+    ESM_HIP(ctx, launch_attention_x3_f32(q, k, v, ld, kQPrescale, d_cu, d_work, nwork, out, ld, max_len, ctx->stream));
     ESM_TRY(ctx->time_end(slot));
     ESM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return ESM_GFX950_OK;

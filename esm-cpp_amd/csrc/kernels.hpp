@@ -198,11 +198,12 @@ hipError_t launch_attention_x3(const uint32_t* q, int ldq, const uint16_t* kh, c
                                const uint16_t* vl, int ldp, float q_prescale, const int* cu_seqlens,
                                const AttnWork* work, int num_work, float* out, int ld_out, int max_len,
                                hipStream_t s, float* part_max = nullptr);
-// fp32 [rows, d] (row stride ld_x, d % 64 == 0) -> that layout: split words
-// of x * scale (words != null, row stride ld_out words) or hi / lo planes
-// (planes != null: hi at [r * ld_out + c], lo d elements further).
-hipError_t launch_pack_x3(const float* x, int ld_x, int rows, int d, float scale, uint32_t* words, uint16_t* planes,
-                          int ld_out, hipStream_t s);
+// The same attention on fp32 q, k, v rows (token t, head h at base + t * ld +
+// h * 64), split inside the kernel: the results of splitting them into that
+// layout first, bit for bit.
+hipError_t launch_attention_x3_f32(const float* q, const float* k, const float* v, int ld, float q_prescale,
+                                   const int* cu_seqlens, const AttnWork* work, int num_work, float* out, int ld_out,
+                                   int max_len, hipStream_t s);
 // Exact fp32 path for any head_dim <= 128 (fp32 MFMA, softmax sum in double).
 hipError_t launch_attention_f32(const float* q, const float* k, const float* v,
                                 int ld, int head_dim, const int* cu_seqlens,

@@ -241,3 +241,27 @@ def test_fp32_path_block_edges(dev, oracle, dh, shift):
     assert np.array_equal(np.isinf(got), np.isinf(want)) and np.isinf(want).sum() == 17
     fine = np.isfinite(want)
     np.testing.assert_allclose(got[fine], want[fine], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("lengths", [[1, 31, 32, 33], [64, 127, 128, 129], [257, 2, 288]])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_x3_splits_any_fp32_rows(dev, oracle, lengths, shift):
+    """The fp32-input entry splits its operands inside the kernel: lengths
+    around the 32-key chunks and 128-query tiles, short and long variants,
+    operands off a 16-byte boundary (the same bits as aligned ones). Bar as
+    the other split-fp16 tests'."""
+    H = 3
+    r = rng(sum(lengths))
+    cu = cu_from_lengths(lengths)
+    T = int(cu[-1])
+    q, k, v = _qkv(r, T, H, 64)
+    want = oracle.attention_varlen(q, k, v, cu, H, 64)
+    outs = []
+    for off in (0, shift):
+        pad = np.zeros(off, np.float32)
+        arrs = [dev.array(np.concatenate([pad, x.ravel()])) for x in (q, k, v)]
+        out = dev.empty((T, H * 64), np.float32)
+        dev.attention_varlen(*(_Offset(a, off) for a in arrs), cu, H, 64, out, eg.ATTN_F16X3_MFMA)
+        outs.append(out.numpy())
+    assert np.array_equal(outs[0], outs[1])
+    np.testing.assert_allclose(outs[0], want, rtol=1e-5, atol=1e-5)
