@@ -8,6 +8,8 @@
 // src/quant/pack.cpp:119-147, GeluRef src/kernels/gelu.cpp:30-35,
 // ResidualAddInplaceRef / ScaleInplaceRef src/kernels/residual.cpp:23-29,
 // RopeApplyVarlenRef src/kernels/rope.cpp:47-70, Embed src/model.cpp:737-778.
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -122,25 +124,51 @@ __device__ __forceinline__ float ln_row(float* __restrict__ x, const float* __re
       // may be) receives this row's new scale.
       const float as = split.a_scale[row];
       const size_t plane = static_cast<size_t>(rows) * d;
+      // Every plane's loads are issued before the first sum: a loop over the
+      // planes waits out one load latency per plane and chunk (301 rows, four
+      // planes: 12.4 against 7.2 us).
+      int4 acc[NV];
+      auto sum_planes = [&](auto count) {
+        constexpr int S = decltype(count)::value;
+        int4 t[S][NV];
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+#pragma unroll
+          for (int j = 0; j < NV; ++j) {
+            const int c = (j * 64 + lane) * 4;
+            t[k][j] = *reinterpret_cast<const int4*>(split.planes + k * plane + static_cast<size_t>(row) * d +
+                                                     (c < d ? c : 0));
+          }
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+          acc[j] = t[0][j];
+#pragma unroll
+          for (int k = 1; k < S; ++k) {
+            acc[j].x += t[k][j].x;
+            acc[j].y += t[k][j].y;
+            acc[j].z += t[k][j].z;
+            acc[j].w += t[k][j].w;
+          }
+        }
+      };
+      if (split.splits == 2)
+        sum_planes(std::integral_constant<int, 2>{});
+      else if (split.splits == 3)
+        sum_planes(std::integral_constant<int, 3>{});
+      else if (split.splits == 4)
+        sum_planes(std::integral_constant<int, 4>{});
+      else
+        sum_planes(std::integral_constant<int, 1>{});
 #pragma unroll
       for (int j = 0; j < NV; ++j) {
         const int c = (j * 64 + lane) * 4;
         const int cc = c < d ? c : 0;
-        const int32_t* src = split.planes + static_cast<size_t>(row) * d + cc;
-        int4 acc = *reinterpret_cast<const int4*>(src);
-        for (int k = 1; k < split.splits; ++k) {
-          const int4 t = *reinterpret_cast<const int4*>(src + k * plane);
-          acc.x += t.x;
-          acc.y += t.y;
-          acc.z += t.z;
-          acc.w += t.w;
-        }
         const float4 ws = *reinterpret_cast<const float4*>(split.w_scale + cc);
         const float4 bs = split.bias ? *reinterpret_cast<const float4*>(split.bias + cc) : make_float4(0.f, 0.f, 0.f, 0.f);
-        r[j].x = c < d ? __builtin_fmaf(static_cast<float>(acc.x), as * ws.x, bs.x) : 0.0f;
-        r[j].y = c < d ? __builtin_fmaf(static_cast<float>(acc.y), as * ws.y, bs.y) : 0.0f;
-        r[j].z = c < d ? __builtin_fmaf(static_cast<float>(acc.z), as * ws.z, bs.z) : 0.0f;
-        r[j].w = c < d ? __builtin_fmaf(static_cast<float>(acc.w), as * ws.w, bs.w) : 0.0f;
+        r[j].x = c < d ? __builtin_fmaf(static_cast<float>(acc[j].x), as * ws.x, bs.x) : 0.0f;
+        r[j].y = c < d ? __builtin_fmaf(static_cast<float>(acc[j].y), as * ws.y, bs.y) : 0.0f;
+        r[j].z = c < d ? __builtin_fmaf(static_cast<float>(acc[j].z), as * ws.z, bs.z) : 0.0f;
+        r[j].w = c < d ? __builtin_fmaf(static_cast<float>(acc[j].w), as * ws.w, bs.w) : 0.0f;
       }
     } else {
       load_row_vec<NV>(resid + static_cast<size_t>(row) * d, d, lane, r);
@@ -166,7 +194,10 @@ __device__ __forceinline__ float ln_row(float* __restrict__ x, const float* __re
 // QUANT: int8 codes and the row's scale; the scale from the row's own
 // maximum (per-token), or with tensor_absmax from that device value, each
 // code then quant_i8 as the per-tensor quantisation kernel forms it.
-template <int NV, bool QUANT, bool SPLIT = false>
+// MAX (never with QUANT): the forms with a per-tensor absmax, kept apart
+// because the next row's registers would cost the plain LayerNorm half its
+// waves (123 -> 73 registers at 1280 columns, 218 -> 142 at 2560).
+template <int NV, bool QUANT, bool SPLIT = false, bool MAX = false>
 __global__ __launch_bounds__(256) void layernorm_vec_kernel(
     float* __restrict__ x, const float* __restrict__ resid, const float* __restrict__ gamma,
     const float* __restrict__ beta, float eps, float* __restrict__ out,
@@ -175,7 +206,7 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   float4 v[NV];
-  if (!QUANT && tensor_absmax && !SPLIT && !resid && !out) {
+  if (MAX && !resid && !out) {
     // The maximum alone: the wave's next row is loaded while this one is
     // reduced, so each wave keeps a row's loads in flight.
     float am = 0.f;
@@ -193,7 +224,7 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(
     block_atomic_max_nonneg(tensor_absmax, am);
     return;
   }
-  if (!QUANT && tensor_absmax) {
+  if constexpr (MAX) {
     float am = 0.f;
     for (int base = blockIdx.x * kRowsPerBlock; base < rows; base += gridDim.x * kRowsPerBlock) {
       const int row = base + wave;
@@ -754,12 +785,18 @@ hipError_t launch_layernorm(float* x, const float* resid, const float* gamma, co
   // bounded grid: one atomic per block.
   if (tensor_absmax && d % 4 == 0 && d <= 2560 && g.x > kReduceBlocks) g.x = kReduceBlocks;
   if (!out && !(tensor_absmax && d % 4 == 0 && d <= 2560)) return hipErrorInvalidValue;
-  if (d % 4 == 0 && d <= 1280) {
-    hipLaunchKernelGGL((layernorm_vec_kernel<5, false>), g, b, 0, s, x, resid, gamma, beta, eps, out, rows, d,
-                       tensor_absmax, nullptr, 0, nullptr, round16);
-  } else if (d % 4 == 0 && d <= 2560) {
-    hipLaunchKernelGGL((layernorm_vec_kernel<10, false>), g, b, 0, s, x, resid, gamma, beta, eps, out, rows, d,
-                       tensor_absmax, nullptr, 0, nullptr, round16);
+  if (d % 4 == 0 && d <= 2560) {
+#define ESM_LN(NV, MAX)                                                                                              \
+  hipLaunchKernelGGL((layernorm_vec_kernel<NV, false, false, MAX>), g, b, 0, s, x, resid, gamma, beta, eps, out,    \
+                     rows, d, tensor_absmax, nullptr, 0, nullptr, round16)
+    if (d <= 512 && !tensor_absmax) {
+      ESM_LN(2, false);
+    } else if (d <= 1280) {
+      if (tensor_absmax) ESM_LN(5, true); else ESM_LN(5, false);
+    } else {
+      if (tensor_absmax) ESM_LN(10, true); else ESM_LN(10, false);
+    }
+#undef ESM_LN
   } else {
     hipLaunchKernelGGL(layernorm_any_kernel, g, b, 0, s, x, resid, gamma, beta, eps, out, rows, d, tensor_absmax,
                        round16);
@@ -803,7 +840,7 @@ hipError_t launch_layernorm_quant_split(float* x, const SplitResid& r, const flo
                                         float eps, int rows, int d, int8_t* q, int ldq, float* scales,
                                         hipStream_t s, int round16) {
   if (rows <= 0 || d <= 0) return hipSuccess;
-  if (d % 4 != 0 || d > 2560 || r.splits < 1 || !r.planes || !r.a_scale || !r.w_scale) return hipErrorInvalidValue;
+  if (d % 4 != 0 || d > 2560 || r.splits < 1 || r.splits > 4 || !r.planes || !r.a_scale || !r.w_scale) return hipErrorInvalidValue;
   const dim3 g = rows_grid(rows), b(256);
   if (d <= 1280) {
     hipLaunchKernelGGL((layernorm_vec_kernel<5, true, true>), g, b, 0, s, x, nullptr, gamma, beta, eps, nullptr, rows,
