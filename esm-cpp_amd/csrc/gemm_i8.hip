@@ -352,34 +352,29 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_i8_kernel(const GemmI8Args
 namespace v3 {
 
 constexpr int WAVES_M = 2;  // waves down the tile
-constexpr int BN = 256;     // tile width
 constexpr int BK = 128;
 
-// Tile height: BLK_M 32x32 row blocks per wave, BM = 64 * BLK_M rows (1: 64,
-// 2: 128, 4: 256, 5: 320). For grids that fill the CUs the launcher picks the
-// height that needs the fewer rows' worth of workgroup rounds (a 256-row grid
-// that spills a few tiles into one more round often fits in fewer rounds as
-// 320-row tiles), 320 on a tie; small-M grids take shorter tiles so that
-// more CUs share the rows (gemm_i8_tile_rows).
-// Wave layout: BLK_N 32x32 column blocks per wave, WAVES_N = 8 / BLK_N waves
-// across the 256 columns. Every launch uses BLK_N 2: eight waves, two per
-// SIMD. (BLK_N 4, four waves of 128x128 with the accumulators in AGPRs, reads
-// 29% fewer LDS bytes per MFMA but ran 11-27% slower: one wave per SIMD
-// leaves the matrix core idle at every barrier and LDS wait.)
-template <int BLK_M_, int BLK_N_ = 2>
+// Tile: BLK_M 32x32 row blocks per wave, BM = 64 * BLK_M rows (1: 64, 2: 128,
+// 3: 192, 4: 256, 5: 320), and WAVES_N waves of two column blocks, BN = 64 *
+// WAVES_N columns. Which tile a launch takes: best_tile.
+// Every launch uses two column blocks a wave: two waves per SIMD. (BLK_N 4,
+// four waves of 128x128 with the accumulators in AGPRs, reads 29% fewer LDS
+// bytes per MFMA but ran 11-27% slower: one wave per SIMD leaves the matrix
+// core idle at every barrier and LDS wait.)
+template <int BLK_M_, int BLK_N_ = 2, int WAVES_N_ = 4>
 struct Tile {
   static constexpr int BLK_M = BLK_M_, BLK_N = BLK_N_;
-  static constexpr int WAVES_N = 8 / BLK_N;
+  static constexpr int WAVES_N = WAVES_N_;
+  static constexpr int BN = WAVES_N * BLK_N * 32;
   static constexpr int kWaves = WAVES_M * WAVES_N;
   static constexpr int kThreads = kWaves * 64;
-  static_assert(WAVES_N * BLK_N * 32 == BN, "waves x blocks must cover the 256 tile columns");
   static constexpr int BM = WAVES_M * BLK_M * 32;
   static constexpr int kBlocks = (BM + BN) / 8;  // 1 KB blocks per stage
   static constexpr int kPer = kBlocks / kWaves;
-  static constexpr int kStage = kBlocks * 1024;  // 64 KB (BM 256) / 72 KB (BM 320)
-  // Stage buffers: three for the short tiles (40 / 48 KB each), so the loads
-  // run two stages ahead of the MFMAs; the tall tiles' two fill the LDS.
-  static constexpr int kNStage = BLK_M <= 2 ? 3 : 2;
+  static constexpr int kStage = kBlocks * 1024;  // 16 KB (64x64) to 72 KB (320x256)
+  // Stage buffers: three or four for the small tiles, so the loads run two or
+  // three stages ahead of the MFMAs; the tall tiles' two fill the LDS.
+  static constexpr int kNStage = kStage <= 24 * 1024 ? 4 : kStage <= 48 * 1024 ? 3 : 2;
   // RoPE cos / sin rows of a tile staged in LDS, transposed: [32 dims][BM
   // rows + pad], so that a lane reads four consecutive rows of one dim at once.
   static constexpr int kRopeTPitch = BM + 4;
@@ -466,12 +461,12 @@ constexpr int kBufNT = 2;  // buffer access aux bits: non-temporal
 // weights, p.q_scale == 1, so the product would be exact anyway).
 // kEpiQkvSplit: the Q columns' weight scales and bias arrive already
 // multiplied by p.q_prescale (see the kernel's scale staging).
-template <int BLK_M, int BLK_N, int EPI, bool FULL, int WHICH, bool QS = true>
+template <int BLK_M, int BLK_N, int WAVES_N, int EPI, bool FULL, int WHICH, bool QS = true>
 __device__ __forceinline__ void qkv_head(const GemmI8Args& p, const i32x16 (&acc)[BLK_M][BLK_N], int g, int hc,
                                          int wr0, int lr0, int l32, const float* s_as, const float (&ws)[BLK_N],
                                          const float (&bs)[BLK_N], const float* s_cosT, const float* s_sinT, int m0,
                                          int n0) {
-  constexpr int kRopeTPitch = Tile<BLK_M, BLK_N>::kRopeTPitch;
+  constexpr int kRopeTPitch = Tile<BLK_M, BLK_N, WAVES_N>::kRopeTPitch;
   const uint32_t ldc = p.ldc;
   const uint32_t dm = p.d_model;
   // Row offsets: the lane's first row (lr0) times the stride once; the rest
@@ -574,7 +569,7 @@ __device__ __forceinline__ void qkv_head(const GemmI8Args& p, const i32x16 (&acc
 // MAX: also reduce |out| into p.row_absmax / p.tensor_absmax (whichever is set).
 // c_i32: the int32 output (kEpiI32), p.C_i32 or, for a split-K launch, the
 // split's own plane of it.
-template <int BLK_M, int BLK_N, int EPI, bool FULL, bool MAX>
+template <int BLK_M, int BLK_N, int WAVES_N, int EPI, bool FULL, bool MAX>
 __device__ __forceinline__ void epilogue32(const GemmI8Args& p, const i32x16 (&acc)[BLK_M][BLK_N], int wm, int wn,
                                            int l32, int hi, const float* s_as, const float* s_ws,
                                            const float* s_bs, const float* s_cosT, const float* s_sinT, int m0,
@@ -617,14 +612,14 @@ __device__ __forceinline__ void epilogue32(const GemmI8Args& p, const i32x16 (&a
         if (!FULL && n0 + hc >= p.N) break;
         const int which = (n0 + hc) / p.d_model;
         if (which == 0 && p.q_scale == 1.0f)
-          qkv_head<BLK_M, BLK_N, EPI, FULL, 0, false>(p, acc, g, hc, wr0, lr0, l32, s_as, ws, bs, s_cosT, s_sinT, m0,
+          qkv_head<BLK_M, BLK_N, WAVES_N, EPI, FULL, 0, false>(p, acc, g, hc, wr0, lr0, l32, s_as, ws, bs, s_cosT, s_sinT, m0,
                                                       n0);
         else if (which == 0)
-          qkv_head<BLK_M, BLK_N, EPI, FULL, 0>(p, acc, g, hc, wr0, lr0, l32, s_as, ws, bs, s_cosT, s_sinT, m0, n0);
+          qkv_head<BLK_M, BLK_N, WAVES_N, EPI, FULL, 0>(p, acc, g, hc, wr0, lr0, l32, s_as, ws, bs, s_cosT, s_sinT, m0, n0);
         else if (which == 1)
-          qkv_head<BLK_M, BLK_N, EPI, FULL, 1>(p, acc, g, hc, wr0, lr0, l32, s_as, ws, bs, s_cosT, s_sinT, m0, n0);
+          qkv_head<BLK_M, BLK_N, WAVES_N, EPI, FULL, 1>(p, acc, g, hc, wr0, lr0, l32, s_as, ws, bs, s_cosT, s_sinT, m0, n0);
         else
-          qkv_head<BLK_M, BLK_N, EPI, FULL, 2>(p, acc, g, hc, wr0, lr0, l32, s_as, ws, bs, s_cosT, s_sinT, m0, n0);
+          qkv_head<BLK_M, BLK_N, WAVES_N, EPI, FULL, 2>(p, acc, g, hc, wr0, lr0, l32, s_as, ws, bs, s_cosT, s_sinT, m0, n0);
       }
       return;
     } else if constexpr (EPI == kEpiF32R24) {
@@ -787,18 +782,18 @@ __device__ __forceinline__ void epilogue32(const GemmI8Args& p, const i32x16 (&a
         }
       if constexpr (MAX) {
         // One atomic per workgroup (every wave reaches this point).
-        if (p.tensor_absmax) block_atomic_max_nonneg<Tile<BLK_M, BLK_N>::kWaves>(p.tensor_absmax, tmax);
+        if (p.tensor_absmax) block_atomic_max_nonneg<Tile<BLK_M, BLK_N, WAVES_N>::kWaves>(p.tensor_absmax, tmax);
       }
     }
   }
 }
 
-template <int BLK_M, int BLK_N, int EPI>
-__global__ __launch_bounds__((Tile<BLK_M, BLK_N>::kThreads), 1) void gemm_i8_v3_kernel(const GemmI8Args p) {
-  using TL = Tile<BLK_M, BLK_N>;
-  constexpr int BM = TL::BM, kPer = TL::kPer, kStage = TL::kStage, kRopeTPitch = TL::kRopeTPitch;
+template <int BLK_M, int BLK_N, int WAVES_N, int EPI>
+__global__ __launch_bounds__((Tile<BLK_M, BLK_N, WAVES_N>::kThreads), 1) void gemm_i8_v3_kernel(const GemmI8Args p) {
+  using TL = Tile<BLK_M, BLK_N, WAVES_N>;
+  constexpr int BM = TL::BM, BN = TL::BN, kPer = TL::kPer, kStage = TL::kStage, kRopeTPitch = TL::kRopeTPitch;
   constexpr int kNStage = TL::kNStage;
-  constexpr int kThreads = TL::kThreads, WAVES_N = TL::WAVES_N;
+  constexpr int kThreads = TL::kThreads;
   __shared__ __attribute__((aligned(1024))) int8_t smem[kNStage * kStage];
   __shared__ float s_as[BM], s_ws[BN], s_bs[BN];
   __shared__ int s_pos[BM];
@@ -846,25 +841,13 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N>::kThreads), 1) void gemm_i8_v3_
   }
   auto gbase = [&](int i) { return wave * kPer + i < BM / 8 ? pA : pW; };
   const uint32_t ldst = lds_addr(smem) + static_cast<uint32_t>(wave * kPer * 1024);
-  // Stage 0 first, so that its loads and the scale loads below are in flight
-  // together.
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) dma16_async_so(gbase(i), goff[i], ldst + i * 1024);
-
-  // kEpiF32R24: whether a value of the tile can be NaN (a scale or bias not
-  // finite, or a scale above 2^60, so that a product of two could overflow).
-  // Each wave's verdict goes to LDS here and is combined before the
-  // epilogue.
-  __shared__ int s_risk[TL::kWaves];
-  if constexpr (EPI != kEpiI32) {
-    // Per-row activation scales and per-column weight scales / bias of the
-    // tile, read once here instead of per element in the epilogue, every
-    // item's loads issued before the first LDS write. The epilogue (and the
-    // RoPE staging) read them after the main loop's barriers, each of which
-    // follows an lgkmcnt(0) wait, so no barrier of their own is needed.
-    constexpr int kItems = (BM + BN + kThreads - 1) / kThreads;
-    float va[kItems], vb[kItems];
-    int vp[kItems];
+  // Per-row activation scales and per-column weight scales / bias of the
+  // tile, read once here instead of per element in the epilogue, every item's
+  // loads issued before the first LDS write (stage_scales).
+  constexpr int kItems = (BM + BN + kThreads - 1) / kThreads;
+  float va[kItems], vb[kItems];
+  int vp[kItems];
+  auto load_scales = [&]() {
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
       const int t = threadIdx.x + k * kThreads;
@@ -884,6 +867,13 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N>::kThreads), 1) void gemm_i8_v3_
         }
       }
     }
+  };
+  // kEpiF32R24: whether a value of the tile can be NaN (a scale or bias not
+  // finite, or a scale above 2^60, so that a product of two could overflow).
+  // Each wave's verdict goes to LDS here and is combined before the
+  // epilogue.
+  __shared__ int s_risk[TL::kWaves];
+  auto stage_scales = [&]() {
     int risk = 0;
 #pragma unroll
     for (int k = 0; k < kItems; ++k) {
@@ -910,6 +900,31 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N>::kThreads), 1) void gemm_i8_v3_
     if constexpr (EPI == kEpiF32R24) {
       const bool wave_risk = __builtin_amdgcn_ballot_w64(risk != 0) != 0;
       if (lane == 0) s_risk[wave] = wave_risk;
+    }
+  };
+  auto load_stage = [&](int st, int buf) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) dma16_async_so(gbase(i) + st * BK, goff[i], ldst + buf * kStage + i * 1024);
+  };
+  // Tall tiles (two buffers): stage 0 first, so that its loads and the scale
+  // loads are in flight together, and the scales staged behind them; the
+  // epilogue (and the RoPE staging) read them after the main loop's barriers,
+  // each of which follows an lgkmcnt(0) wait, so no barrier of their own is
+  // needed. Small tiles (kEarly), whose few stages are mostly load latency:
+  // all free buffers' stages go out at once behind the scale loads, and the
+  // scales stay in registers until the main loop is over (staging them first
+  // would wait for every load in flight).
+  constexpr bool kEarly = kNStage > 2;
+  if constexpr (kEarly) {
+    if constexpr (EPI != kEpiI32) load_scales();
+#pragma unroll
+    for (int st = 0; st < kNStage - 1; ++st)
+      if (st < nk) load_stage(st, st);
+  } else {
+    load_stage(0, 0);
+    if constexpr (EPI != kEpiI32) {
+      load_scales();
+      stage_scales();
     }
   }
 
@@ -970,14 +985,22 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N>::kThreads), 1) void gemm_i8_v3_
     if constexpr (kReads > kPairs) __builtin_amdgcn_sched_group_barrier(0x100, kReads - kPairs, 0);
   };
   i32x4 fa0[BLK_M], fb0[BLK_N], fa1[BLK_M], fb1[BLK_N];
-  asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-  // Stages 1 .. kNStage - 1 go to the free buffers.
-#pragma unroll
-  for (int st = 1; st < kNStage; ++st) {
-    if (st < nk) {
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) dma16_async_so(gbase(i) + st * BK, goff[i], ldst + st * kStage + i * 1024);
-    }
+  // Waits until at most `ahead` later stages' loads are in flight (vector
+  // memory operations complete in order), then the barrier.
+  auto wait_stage = [&](int ahead) {
+    if (kNStage > 3 && ahead >= 2)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kPer) : "memory");
+    else if (kNStage > 2 && ahead >= 1)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPer) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  };
+  if constexpr (kEarly) {
+    wait_stage(min(kNStage - 2, nk - 1));
+    if (kNStage - 1 < nk) load_stage(kNStage - 1, kNStage - 1);
+  } else {
+    wait_stage(0);
+    if (1 < nk) load_stage(1, 1);
   }
   read_frags(smem, 0, fa0, fb0);
   static_assert(kSub == 4, "the sub-step rotation below assumes four 32-byte sub-steps per stage");
@@ -1002,23 +1025,14 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N>::kThreads), 1) void gemm_i8_v3_
     interleave();
     // Stage kt + 1 has landed (own loads, then the barrier for everyone
     // else's) and every wave has finished reading stage kt, whose buffer
-    // then receives stage kt + kNStage. With three buffers stage kt + 2's
-    // loads, issued one iteration earlier, may still be in flight: vector
-    // memory operations complete in order, so waiting until at most those
-    // kPer remain means stage kt + 1's have landed. The body has no other
-    // branch: the last iteration reads sub-step 0 of a stale buffer into
-    // fa0 / fb0 and never uses it (a branch around those reads would split
-    // the last sub-step's MFMAs over two blocks, and the accumulators'
-    // copies at the join spill).
-    if (kNStage == 3 && kt + 2 < nk)
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPer) : "memory");
-    else
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (kt + kNStage < nk) {
-      const uint32_t dst = ldst + bcur * kStage;
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) dma16_async_so(gbase(i) + (kt + kNStage) * BK, goff[i], dst + i * 1024);
-    }
+    // then receives stage kt + kNStage. With more than two buffers the loads
+    // of stages kt + 2 .. kt + kNStage - 1 may still be in flight. The body
+    // has no other branch: the last iteration reads sub-step 0 of a stale
+    // buffer into fa0 / fb0 and never uses it (a branch around those reads
+    // would split the last sub-step's MFMAs over two blocks, and the
+    // accumulators' copies at the join spill).
+    wait_stage(min(kNStage - 2, nk - 2 - kt));
+    if (kt + kNStage < nk) load_stage(kt + kNStage, bcur);
     read_frags(smem + bnext * kStage, 0, fa0, fb0);
     mfmas(fa1, fb1);
     interleave();
@@ -1026,6 +1040,10 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N>::kThreads), 1) void gemm_i8_v3_
   };
   stage(0, std::true_type{});
   for (int kt = 1; kt < nk; ++kt) stage(kt, std::false_type{});
+  if constexpr (kEarly && EPI != kEpiI32) {
+    stage_scales();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  }
 
   const float* s_cosT = nullptr;
   const float* s_sinT = nullptr;
@@ -1083,17 +1101,17 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N>::kThreads), 1) void gemm_i8_v3_
   const bool full = m0 + BM <= p.M && n0 + BN <= p.N;
   if (kMaxable && (p.row_absmax || p.tensor_absmax)) {
     if (full)
-      epilogue32<BLK_M, BLK_N, EPI, true, kMaxable>(p, acc, wm, wn, l32, hi, s_as, s_ws, s_bs, s_cosT, s_sinT, m0, n0,
+      epilogue32<BLK_M, BLK_N, WAVES_N, EPI, true, kMaxable>(p, acc, wm, wn, l32, hi, s_as, s_ws, s_bs, s_cosT, s_sinT, m0, n0,
           c_i32, nan_risk);
     else
-      epilogue32<BLK_M, BLK_N, EPI, false, kMaxable>(p, acc, wm, wn, l32, hi, s_as, s_ws, s_bs, s_cosT, s_sinT, m0, n0,
+      epilogue32<BLK_M, BLK_N, WAVES_N, EPI, false, kMaxable>(p, acc, wm, wn, l32, hi, s_as, s_ws, s_bs, s_cosT, s_sinT, m0, n0,
           c_i32, nan_risk);
   } else {
     if (full)
-      epilogue32<BLK_M, BLK_N, EPI, true, false>(p, acc, wm, wn, l32, hi, s_as, s_ws, s_bs, s_cosT, s_sinT, m0, n0,
+      epilogue32<BLK_M, BLK_N, WAVES_N, EPI, true, false>(p, acc, wm, wn, l32, hi, s_as, s_ws, s_bs, s_cosT, s_sinT, m0, n0,
           c_i32, nan_risk);
     else
-      epilogue32<BLK_M, BLK_N, EPI, false, false>(p, acc, wm, wn, l32, hi, s_as, s_ws, s_bs, s_cosT, s_sinT, m0, n0,
+      epilogue32<BLK_M, BLK_N, WAVES_N, EPI, false, false>(p, acc, wm, wn, l32, hi, s_as, s_ws, s_bs, s_cosT, s_sinT, m0, n0,
           c_i32, nan_risk);
   }
 }
@@ -1166,32 +1184,33 @@ hipError_t launch_v1(const GemmI8Args& p, int epi, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int BLK_M, int BLK_N = 2>
+template <int BLK_M, int WAVES_N = 4>
 hipError_t launch_v3_tile(const GemmI8Args& p, int epi, hipStream_t s) {
   using namespace v3;
-  constexpr int BM = Tile<BLK_M, BLK_N>::BM;
+  using TL = Tile<BLK_M, 2, WAVES_N>;
+  constexpr int BM = TL::BM, BN = TL::BN;
   const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-  const dim3 grid(tiles * (epi == kEpiI32 ? std::max(p.splits, 1) : 1)), block(Tile<BLK_M, BLK_N>::kThreads);
+  const dim3 grid(tiles * (epi == kEpiI32 ? std::max(p.splits, 1) : 1)), block(TL::kThreads);
   switch (epi) {
-    case kEpiI32: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiI32>), grid, block, 0, s, p); break;
-    case kEpiF32: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiF32>), grid, block, 0, s, p); break;
-    case kEpiF32Gelu: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiF32Gelu>), grid, block, 0, s, p); break;
-    case kEpiF32Resid: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiF32Resid>), grid, block, 0, s, p); break;
-    case kEpiQkvRope: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiQkvRope>), grid, block, 0, s, p); break;
-    case kEpiF32GeluQ: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiF32GeluQ>), grid, block, 0, s, p); break;
+    case kEpiI32: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiI32>), grid, block, 0, s, p); break;
+    case kEpiF32: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiF32>), grid, block, 0, s, p); break;
+    case kEpiF32Gelu: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiF32Gelu>), grid, block, 0, s, p); break;
+    case kEpiF32Resid: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiF32Resid>), grid, block, 0, s, p); break;
+    case kEpiQkvRope: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiQkvRope>), grid, block, 0, s, p); break;
+    case kEpiF32GeluQ: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiF32GeluQ>), grid, block, 0, s, p); break;
     case kEpiF32GeluAs:
-      hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiF32GeluAs>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiF32GeluAs>), grid, block, 0, s, p);
       break;
     case kEpiF32GeluX86:
-      hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiF32GeluX86>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiF32GeluX86>), grid, block, 0, s, p);
       break;
     case kEpiQkvRopeF32:
-      hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiQkvRopeF32>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiQkvRopeF32>), grid, block, 0, s, p);
       break;
-    case kEpiQkvSplit: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiQkvSplit>), grid, block, 0, s, p); break;
+    case kEpiQkvSplit: hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiQkvSplit>), grid, block, 0, s, p); break;
     case kEpiF32R24:
       if (p.N % 64 != 0 || !p.C_f16 || !p.C_u8 || p.ldc % 2 != 0) return hipErrorInvalidValue;
-      hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, BLK_N, kEpiF32R24>), grid, block, 0, s, p);
+      hipLaunchKernelGGL((gemm_i8_v3_kernel<BLK_M, 2, WAVES_N, kEpiF32R24>), grid, block, 0, s, p);
       break;
     default: return hipErrorInvalidValue;
   }
@@ -1216,99 +1235,119 @@ int device_cus() {
 
 namespace {
 
-long tiles_of(int M, int N, int BM) {
-  return static_cast<long>((M + BM - 1) / BM) * ((N + v3::BN - 1) / v3::BN);
+// The pipelined kernel's tiles. 64 .. 320: rows of a tile 256 columns wide,
+// but 64 is 64x64; kTile128x128 is 128x128.
+constexpr int kTile128x128 = 1128;
+
+// A launch's estimated time in microseconds: whole rounds of workgroups over
+// the CUs at t = fixed + per_stage * stages each, and a last, partly filled
+// round at sparse * t plus the rest in proportion to its workgroups (a round
+// that leaves CUs idle runs at a higher clock and with less L2 contention).
+// The constants are fitted to launches of N x K = 1280..10240 x 1280..10240 at
+// 30..9,000 rows; at 5120 x 1280 and 4,099 rows, for one, it gives 39 / 36 / 44
+// / 49 us for 128, 192, 256 and 320 rows, measured 40.5 / 37.5 / 42.2 / 50.4.
+struct TileCost {
+  int code, rows, cols, per_cu;
+  double fixed, per_stage, sparse;
+};
+constexpr TileCost kTileCosts[] = {
+    // 64x64: two share a CU; alone a workgroup takes 3.8 + 0.24 a stage. At
+    // 301 rows 6.2 us (N = K = 1280), 13.1 (K = 5120); the 64x256 tile it
+    // replaced took 8.2 and 21.9.
+    {64, 64, 64, 2, 3.0, 0.42, 0.72},
+    // 128x128: the same rows and stage bytes per column as 64x256, no slower
+    // anywhere: 8.3 against 8.6 us at 2,048 rows (N = K = 1280).
+    {kTile128x128, 128, 128, 1, 3.6, 0.42, 1.0},
+    {128, 128, 256, 1, 4.0, 0.95, 0.75},
+    {192, 192, 256, 1, 6.0, 1.28, 0.72},
+    {256, 256, 256, 1, 9.0, 1.55, 0.68},
+    {320, 320, 256, 1, 13.0, 1.6, 0.72},
+};
+
+long tiles_of(int M, int N, const TileCost& c) {
+  return static_cast<long>((M + c.rows - 1) / c.rows) * ((N + c.cols - 1) / c.cols);
 }
 
-// Workgroup rounds times tile height: the rows' worth of tile time the grid
-// needs when every round costs one tile's time.
-long tile_cost(int M, int N, int BM, int cus) { return (tiles_of(M, N, BM) + cus - 1) / cus * BM; }
+double tile_time(const TileCost& c, long workgroups, int stages, int cus) {
+  const double t = c.fixed + c.per_stage * stages;
+  const long slots = static_cast<long>(cus) * c.per_cu;
+  const long whole = workgroups / slots, rest = workgroups % slots;
+  const double last = rest ? t * (c.sparse + (1.0 - c.sparse) * static_cast<double>(rest) / slots) : 0.0;
+  return static_cast<double>(whole) * t + last;
+}
+
+// The tile with the least estimated time for `splits` ranges of K.
+const TileCost& best_tile(int M, int N, int stages, int splits, int cus, bool tall_ok, double* t) {
+  const TileCost* best = nullptr;
+  for (const TileCost& c : kTileCosts) {
+    if (c.rows == 320 && !tall_ok) continue;
+    const double x = tile_time(c, tiles_of(M, N, c) * splits, (stages + splits - 1) / splits, cus);
+    if (!best || x < *t) {
+      best = &c;
+      *t = x;
+    }
+  }
+  return *best;
+}
+
+// A launch that fills its share of the CUs (a concurrent sequence group's
+// share, or all of them) is counted over the whole device: concurrent
+// launches fill each other's last rounds.
+int counted_cus(int M, int N, int cus) {
+  const int all = device_cus();
+  if (cus <= 0) return all;
+  const long tiles256 = static_cast<long>((M + 255) / 256) * ((N + 255) / 256);
+  return tiles256 >= cus ? all : cus;
+}
 
 }  // namespace
 
 int gemm_i8_tile_rows(int M, int N, int K, int epi, int cus) {
   const int forced = g_tile_rows.load(std::memory_order_relaxed);
   if (forced != 0) return forced;
-  const int all = device_cus();
-  if (cus <= 0) cus = all;
-  // Ties go to 320 rows: at equal rounds the taller tile re-reads less of
-  // A and W (fc1 at config 4: 270 vs 282 us). The erff GELU and bf16/fp32
-  // RoPE epilogues stay at 256 rows: at BLK_M = 5 they exceed 256 VGPRs. The
-  // split-word QKV epilogue spills 72 bytes there too, but runs faster at
-  // 320 rows all the same (216 vs 224 us at config 4). Rounds are counted
-  // over the whole device: concurrent launches fill each other's last round.
+  // The erff GELU and bf16/fp32 RoPE epilogues stay at 256 rows: at BLK_M = 5
+  // they exceed 256 VGPRs. The split-word QKV epilogue spills 72 bytes there
+  // too, but runs faster at 320 rows all the same (216 vs 224 us at
+  // config 4).
   const bool tall_ok =
       epi == kEpiI32 || epi == kEpiF32 || epi == kEpiF32Resid || epi == kEpiQkvSplit || epi == kEpiF32R24 ||
       epi == kEpiF32GeluAs;
-  if (tiles_of(M, N, 256) >= cus)
-    return tall_ok && tile_cost(M, N, 320, all) <= tile_cost(M, N, 256, all) ? 320 : 256;
-  // The 256-row grid leaves CUs idle (one workgroup per CU): shorter tiles
-  // spread the rows over more CUs. Estimated time of a grid = rounds x
-  // (stages + fixed cost) x the per-stage time of the tile height, the
-  // per-stage times relative to the 256-row tile's.
-  static constexpr int kRows[3] = {64, 128, 256};
-  static constexpr double kStage[3] = {0.45, 0.62, 1.0};
-  constexpr double kFixed = 3.0;  // prologue + epilogue, in stages
-  const double stages = K / v3::BK + kFixed;
-  int best = 256;
-  double best_t = 0.0;
-  for (int i = 2; i >= 0; --i) {
-    const long rounds = (tiles_of(M, N, kRows[i]) + cus - 1) / cus;
-    const double t = static_cast<double>(rounds) * stages * kStage[i];
-    if (i == 2 || t < best_t * 0.97) {
-      best = kRows[i];
-      best_t = t;
-    }
-  }
-  return best;
+  double t = 0.0;
+  return best_tile(M, N, K / v3::BK, 1, counted_cus(M, N, cus), tall_ok, &t).code;
 }
 
 namespace {
 
 std::atomic<int> g_split_k{0};
 
-// Estimated time, in units of one 256-row tile's K stage (about 2 us here),
-// of a grid of `tiles` workgroups on `cus` CUs running `stages` K stages each
-// at tile height rows (64, 128 or 256), as in gemm_i8_tile_rows.
-double grid_units(long tiles, int stages, int rows, int cus) {
-  const double per = rows == 64 ? 0.45 : rows == 128 ? 0.62 : 1.0;
-  const long rounds = (tiles + cus - 1) / cus;
-  return static_cast<double>(rounds) * (stages + 3.0) * per;
-}
-
 }  // namespace
 
 int gemm_i8_split_k(int M, int N, int K, int cus, bool fused, int* rows) {
-  const int all = device_cus();
-  if (cus <= 0) cus = all;
   *rows = gemm_i8_tile_rows(M, N, K, kEpiF32, cus);
   const int forced = g_split_k.load(std::memory_order_relaxed);
   if (forced == 1 || N % 4 != 0) return 1;
   const int nk = K / v3::BK;
   if (forced >= 2) return nk >= forced ? forced : 1;
-  if (*rows == 320 || tiles_of(M, N, *rows) >= cus) return 1;
-  // The dequant pass reads S int32 planes and writes the fp32 result: at
-  // about 4 TB/s plus a launch, in the same units. Fused into the reader, it
-  // costs the S - 1 planes read beyond the fp32 result it replaces.
-  constexpr double kUnitUs = 2.05;
-  auto pass_units = [&](int S) {
-    if (fused) return (S - 1.0) * static_cast<double>(M) * N * 4.0 / 4.0e6 / kUnitUs;
-    const double bytes = (S + 1.0) * static_cast<double>(M) * N * 4.0;
-    return (bytes / 4.0e6 + 4.0) / kUnitUs;
-  };
-  double best = grid_units(tiles_of(M, N, *rows), nk, *rows, cus);
-  int best_s = 1, best_rows = *rows;
-  static constexpr int kRows[3] = {64, 128, 256};
-  for (int r : kRows)
-    for (int S = 2; S <= 4 && nk / S >= 4; ++S) {
-      const double t = grid_units(tiles_of(M, N, r) * S, (nk + S - 1) / S, r, cus) + pass_units(S);
-      if (t < best * 0.9) {
-        best = t;
-        best_s = S;
-        best_rows = r;
-      }
+  if (g_tile_rows.load(std::memory_order_relaxed) != 0) return 1;
+  const int n = counted_cus(M, N, cus);
+  double best = 0.0;
+  const TileCost& one = best_tile(M, N, nk, 1, n, true, &best);
+  if (tiles_of(M, N, one) >= n) return 1;
+  // The dequant pass reads S int32 planes and reads and writes the fp32
+  // result at about 4 TB/s, after a launch; fused into the LayerNorm that
+  // reads the result, the planes' reads and 1.5 us more.
+  const double plane = static_cast<double>(M) * N * 4.0 / 4.0e6;
+  int best_s = 1;
+  for (int S = 2; S <= 4 && nk / S >= 4; ++S) {
+    double t = 0.0;
+    const TileCost& c = best_tile(M, N, nk, S, n, true, &t);
+    t += fused ? S * plane + 1.5 : (S + 2) * plane + 4.0;
+    if (t < best * 0.95) {
+      best = t;
+      best_s = S;
+      *rows = c.code;
     }
-  *rows = best_rows;
+  }
   return best_s;
 }
 
@@ -1322,7 +1361,9 @@ namespace {
 
 hipError_t launch_v3_rows(const GemmI8Args& p, int epi, int rows, hipStream_t s) {
   switch (rows) {
-    case 64: return launch_v3_tile<1>(p, epi, s);
+    case 64: return launch_v3_tile<1, 1>(p, epi, s);
+    case kTile128x128: return launch_v3_tile<2, 2>(p, epi, s);
+    case 192: return launch_v3_tile<3>(p, epi, s);
     case 128: return launch_v3_tile<2>(p, epi, s);
     case 320: return launch_v3_tile<5>(p, epi, s);
     default: return launch_v3_tile<4>(p, epi, s);

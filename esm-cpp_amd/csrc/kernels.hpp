@@ -87,35 +87,34 @@ struct GemmI8Args {
   size_t splitk_ws_elems = 0;
 };
 
-// Picks the pipelined 256- or 320-row-tile kernel when gemm_i8_pipelined_ok(p) (K a
+// Picks the pipelined kernel when gemm_i8_pipelined_ok(p) (K a
 // multiple of 128, 16-byte aligned rows, M*lda and N*ldw at most 2^32 bytes),
-// else the general 256x128 kernel.
+// else the general 256x128-tile kernel.
 hipError_t launch_gemm_i8(const GemmI8Args& p, int epilogue, hipStream_t s);
 bool gemm_i8_pipelined_ok(const GemmI8Args& p);
 // variant 1: general kernel; 2: pipelined kernel (fails on shapes it cannot take).
 hipError_t launch_gemm_i8_variant(const GemmI8Args& p, int epilogue, int variant, hipStream_t s);
 // Row height of the pipelined kernel's tile for every later launch in the
-// process: 64, 128, 256, 320, or 0 to pick per launch (gemm_i8_tile_rows).
-// False for other values.
+// process: 64 (64x64), 128, 256, 320 (256 columns wide), or 0 to pick per
+// launch (gemm_i8_tile_rows). False for other values.
 bool set_gemm_tile_rows(int rows);
-// The pipelined kernel's tile height for an M x N x K launch with epilogue
-// epi on `cus` CUs (0: the current device's): grids of at least one 256-row
-// workgroup per CU take 256 or 320 rows, whichever needs the fewer rows'
-// worth of workgroup rounds (320 on a tie, for the epilogues that fit it);
-// smaller grids take 64, 128 or 256 rows by an estimate of their time.
+// The pipelined kernel's tile for an M x N x K launch with epilogue epi on
+// `cus` CUs (0: the current device's): the one with the least estimated time
+// (64x64, 128x128, or 128, 192, 256 or 320 rows by 256 columns), as the code
+// launch_gemm_i8_partials takes.
 int gemm_i8_tile_rows(int M, int N, int K, int epi, int cus);
 // Compute units of the current device (queried once per device; 256 if the
 // query fails).
 int device_cus();
 // K splits of a kEpiF32 launch with a workspace (1: none): grids that leave
 // CUs idle split K when the estimated time of the split grid plus its dequant
-// pass beats the unsplit one's. *rows receives the tile height to use.
+// pass beats the unsplit one's. *rows receives the tile code to use.
 // fused: the partial planes are summed by the kernel that reads the result
 // (launch_layernorm_quant_split) instead of a pass of their own, which then
 // costs only that kernel's extra reads.
 int gemm_i8_split_k(int M, int N, int K, int cus, bool fused, int* rows);
 // The kEpiI32 split-K grid alone: p.C_i32 receives `splits` [M, p.ldc] planes
-// of partial sums (p.ldc >= N), at tile height rows.
+// of partial sums (p.ldc >= N), with tile code rows.
 hipError_t launch_gemm_i8_partials(const GemmI8Args& p, int splits, int rows, hipStream_t s);
 // Process-wide override of gemm_i8_split_k for later launches: 0 automatic,
 // 1 never, 2..4 that many splits wherever a launch qualifies (workspace large

@@ -311,3 +311,39 @@ def test_linear_i8_gelu_quant_r24_rejects_bad_shapes(dev):
     with pytest.raises(eg.Gfx950Error):
         dev.linear_i8_gelu_quant_r24(dA, 208, da, w, None, 4, dh, dl, dq, 64, ds)
     w.free()
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 64, 128), (70, 130, 128), (70, 130, 256), (63, 65, 384), (65, 63, 512), (130, 70, 640), (300, 1280, 768),
+    (301, 5120, 1280), (1000, 130, 1280),   # 64x64, one to ten stages in four buffers
+    (2048, 1280, 1280), (1990, 1210, 5120), (1025, 3900, 256),  # 128x128
+    (4099, 5120, 1280), (2500, 3840, 1280), (4001, 2510, 2560),  # 192 rows
+    (9001, 5121, 384),
+])
+def test_automatic_tile_edges(dev, M, N, K):
+    """The tile that a launch picks by itself, at ragged edges and few K
+    stages: the dequantised output equals the 256-row tile's bit for bit, and
+    the edge rows equal the closed form fma(acc, a_scale * w_scale, bias)."""
+    r = rng(M + N + K)
+    A = r.integers(-127, 128, size=(M, K), dtype=np.int8)
+    W = r.integers(-127, 128, size=(N, K), dtype=np.int8)
+    s = r.uniform(0.001, 0.02, size=N).astype(np.float32)
+    a_s = r.uniform(0.001, 0.02, size=M).astype(np.float32)
+    b = r.standard_normal(N).astype(np.float32)
+    w = dev.weight_i8(W, s)
+    dA, ds, db = dev.array(A), dev.array(a_s), dev.array(b)
+    outs = []
+    for rows in (0, 256):
+        eg.set_gemm_tile_rows(rows)
+        try:
+            out = dev.array(np.full((M, N), np.nan, np.float32))
+            dev.linear_i8_q(dA, K, ds, w, db, out, M)
+            outs.append(out.numpy())
+        finally:
+            eg.set_gemm_tile_rows(0)
+    w.free()
+    assert np.array_equal(outs[0], outs[1])
+    for m in sorted({0, M // 2, max(0, M - 2), M - 1}):
+        acc = (W.astype(np.int64) @ A[m].astype(np.int64)).astype(np.float32)  # |acc| < 2^24: exact
+        want = acc.astype(np.float64) * (a_s[m] * s).astype(np.float64) + b
+        np.testing.assert_allclose(outs[0][m], want, rtol=2.0**-23, atol=0)
