@@ -929,10 +929,10 @@ struct esm_gfx950_model {
   std::vector<DevLayer> layers;
   float *final_ln_w = nullptr, *final_ln_b = nullptr;
   float *lm_dense_w = nullptr, *lm_dense_b = nullptr;
-  // lm head dense weight as split-fp16 planes of W * 2^shift (null when
+  // lm head dense weight as split-fp16 rows of W * 2^shift (null when
   // d % 32 != 0) and whether the forward uses them (split-fp16 GEMM) or the
   // fp32 weight (fp32 MFMA).
-  uint16_t *lm_w_hi = nullptr, *lm_w_lo = nullptr;
+  uint16_t* lm_w_split = nullptr;
   float lm_w_unscale = 1.0f;
   bool lm_dense_split = false;
   float *lm_ln_w = nullptr, *lm_ln_b = nullptr;
@@ -1006,9 +1006,10 @@ int upload_f(esm_gfx950_ctx* ctx, esm_gfx950_model* m, const T* src, size_t n, T
 
 // Concatenates the given linears along N into one device weight.
 // part0_scale multiplies part 0's per-channel scales and bias (int8 only).
-// W [N, K] fp32 as the two fp16 planes of the split-fp16 GEMM: hi = fp16(x),
-// lo = fp16(x - hi) of x = W * 2^shift, with the shift putting max|W| in
-// [2^13, 2^14) so that the lo parts of small weights stay normal fp16.
+// W [N, K] fp32 as the split-fp16 GEMM's rows (per 32 k, the hi then the lo
+// parts): hi = fp16(x), lo = fp16(x - hi) of x = W * 2^shift, with the shift
+// putting max|W| in [2^13, 2^14) so that the lo parts of small weights stay
+// normal fp16.
 int upload_split(esm_gfx950_ctx* ctx, esm_gfx950_model* m, const float* w, int N, int K) {
   const size_t n = static_cast<size_t>(N) * K;
   float amax = 0.0f;
@@ -1019,16 +1020,16 @@ int upload_split(esm_gfx950_ctx* ctx, esm_gfx950_model* m, const float* w, int N
     std::frexp(amax, &e);  // amax in [2^(e-1), 2^e)
     shift = std::min(100, std::max(-100, 14 - e));
   }
-  std::vector<uint16_t> hi(n), lo(n);
+  std::vector<uint16_t> split(2 * n);
   for (size_t i = 0; i < n; ++i) {
     const float x = std::ldexp(w[i], shift);
     const _Float16 h = static_cast<_Float16>(x);
     const _Float16 l = static_cast<_Float16>(x - static_cast<float>(h));
-    hi[i] = __builtin_bit_cast(uint16_t, h);
-    lo[i] = __builtin_bit_cast(uint16_t, l);
+    const size_t at = (i / 32) * 64 + i % 32;  // K % 32 == 0: pieces do not cross rows
+    split[at] = __builtin_bit_cast(uint16_t, h);
+    split[at + 32] = __builtin_bit_cast(uint16_t, l);
   }
-  ESM_TRY(upload_f(ctx, m, hi.data(), n, &m->lm_w_hi));
-  ESM_TRY(upload_f(ctx, m, lo.data(), n, &m->lm_w_lo));
+  ESM_TRY(upload_f(ctx, m, split.data(), split.size(), &m->lm_w_split));
   m->lm_w_unscale = std::ldexp(1.0f, -shift);
   return ESM_GFX950_OK;
 }
@@ -1258,7 +1259,7 @@ extern "C" int esm_gfx950_model_set_numerics(esm_gfx950_ctx* ctx, esm_gfx950_mod
 
 extern "C" int esm_gfx950_model_set_lm_dense_split(esm_gfx950_ctx* ctx, esm_gfx950_model* model, int enabled) {
   if (!ctx || !model) return ESM_GFX950_INVALID_ARGUMENT;
-  ESM_REQUIRE(ctx, !enabled || model->lm_w_hi, "model_set_lm_dense_split: hidden size is not a multiple of 32");
+  ESM_REQUIRE(ctx, !enabled || model->lm_w_split, "model_set_lm_dense_split: hidden size is not a multiple of 32");
   model->lm_dense_split = enabled != 0;
   return ESM_GFX950_OK;
 }
@@ -2206,10 +2207,23 @@ int forward_part(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const esm_gfx95
     return ESM_GFX950_OK;
   }
   // (Last residual +) final LN and lm head: dense -> GELU -> LN -> tied
-  // decoder + bias (reference src/model.cpp:1181-1239).
-  ESM_HIP(ctx, launch_layernorm(a.hidden, pending, m->final_ln_w, m->final_ln_b, c.layer_norm_eps, a.ln, T, d,
-                                nullptr, s));
-  if (cap) ESM_TRY(capture(m->layers.size(), a.ln));
+  // decoder + bias (reference src/model.cpp:1181-1239). For the split-fp16
+  // dense the LayerNorm writes its output already split; where the fp32 output
+  // is wanted too, or the row is wider than that kernel's, a pass splits it.
+  const uint16_t* split_a = nullptr;
+  if (m->lm_dense_split && !cap && !pending && d <= 2560) {
+    ESM_HIP(ctx, launch_layernorm_x3(a.hidden, nullptr, m->final_ln_w, m->final_ln_b, c.layer_norm_eps,
+                                     reinterpret_cast<uint16_t*>(a.ln), T, d, s));
+    split_a = reinterpret_cast<const uint16_t*>(a.ln);
+  } else {
+    ESM_HIP(ctx, launch_layernorm(a.hidden, pending, m->final_ln_w, m->final_ln_b, c.layer_norm_eps, a.ln, T, d,
+                                  nullptr, s));
+    if (cap) ESM_TRY(capture(m->layers.size(), a.ln));
+    if (m->lm_dense_split) {
+      ESM_HIP(ctx, launch_split_rows(a.ln, Td, reinterpret_cast<uint16_t*>(a.attn), s));
+      split_a = reinterpret_cast<const uint16_t*>(a.attn);
+    }
+  }
   DevLinear dense;
   dense.w32 = m->lm_dense_w;
   dense.bias = m->lm_dense_b;
@@ -2219,11 +2233,8 @@ int forward_part(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const esm_gfx95
   ESM_TRY(ctx->time_begin("lm_dense", &slot));
   if (m->lm_dense_split) {
     GemmX3Args x;
-    x.A = a.ln;
-    x.lda = d;
-    x.w_hi = m->lm_w_hi;
-    x.w_lo = m->lm_w_lo;
-    x.ldw = d;
+    x.A = split_a;
+    x.W = m->lm_w_split;
     x.w_unscale = m->lm_w_unscale;
     x.bias = m->lm_dense_b;
     x.C = a.lm_a;

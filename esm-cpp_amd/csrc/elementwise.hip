@@ -197,7 +197,9 @@ __device__ __forceinline__ float ln_row(float* __restrict__ x, const float* __re
 // MAX (never with QUANT): the forms with a per-tensor absmax, kept apart
 // because the next row's registers would cost the plain LayerNorm half its
 // waves (123 -> 73 registers at 1280 columns, 218 -> 142 at 2560).
-template <int NV, bool QUANT, bool SPLIT = false, bool MAX = false>
+// X3 (with neither): out receives the split-fp16 GEMM's A rows instead of fp32,
+// per 32 columns 64 bytes of hi parts and 64 bytes of lo parts.
+template <int NV, bool QUANT, bool SPLIT = false, bool MAX = false, bool X3 = false>
 __global__ __launch_bounds__(256) void layernorm_vec_kernel(
     float* __restrict__ x, const float* __restrict__ resid, const float* __restrict__ gamma,
     const float* __restrict__ beta, float eps, float* __restrict__ out,
@@ -271,6 +273,20 @@ __global__ __launch_bounds__(256) void layernorm_vec_kernel(
       }
       for (int c = d + lane; c < ldq; c += 64) qr[c] = 0;
       if (lane == 0) scales[row] = scale;
+    }
+  } else if constexpr (X3) {
+    uint8_t* orow = reinterpret_cast<uint8_t*>(out) + static_cast<size_t>(row) * d * 4;
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      const int c = (j * 64 + lane) * 4;
+      if (c < d) {
+        uint2 h, l;
+        split_pair(v[j].x, v[j].y, &h.x, &l.x);
+        split_pair(v[j].z, v[j].w, &h.y, &l.y);
+        uint8_t* piece = orow + (c >> 5) * 128 + (c & 31) * 2;
+        *reinterpret_cast<uint2*>(piece) = h;
+        *reinterpret_cast<uint2*>(piece + 64) = l;
+      }
     }
   } else {
     if (out) {
@@ -754,6 +770,21 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const int* __restrict__
   }
 }
 
+// Four values per thread as the split-fp16 GEMM's rows (n a multiple of 32).
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, size_t n,
+                                                         uint16_t* __restrict__ out) {
+  for (size_t i = (blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x) * 4; i < n;
+       i += static_cast<size_t>(gridDim.x) * blockDim.x * 4) {
+    const float4 v = *reinterpret_cast<const float4*>(x + i);
+    uint2 h, l;
+    split_pair(v.x, v.y, &h.x, &l.x);
+    split_pair(v.z, v.w, &h.y, &l.y);
+    uint16_t* piece = out + (i >> 5) * 64 + (i & 31);
+    *reinterpret_cast<uint2*>(piece) = h;
+    *reinterpret_cast<uint2*>(piece + 32) = l;
+  }
+}
+
 __global__ void cast_kernel(const float* __restrict__ x, size_t n, uint16_t* __restrict__ out,
                             int to_bf16) {
   for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < n;
@@ -801,6 +832,28 @@ hipError_t launch_layernorm(float* x, const float* resid, const float* gamma, co
     hipLaunchKernelGGL(layernorm_any_kernel, g, b, 0, s, x, resid, gamma, beta, eps, out, rows, d, tensor_absmax,
                        round16);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_layernorm_x3(float* x, const float* resid, const float* gamma, const float* beta, float eps,
+                               uint16_t* out, int rows, int d, hipStream_t s) {
+  if (rows <= 0 || d <= 0) return hipSuccess;
+  if (d % 32 != 0 || d > 2560 || !out) return hipErrorInvalidValue;
+  const dim3 g = rows_grid(rows), b(256);
+  float* o = reinterpret_cast<float*>(out);
+  if (d <= 1280)
+    hipLaunchKernelGGL((layernorm_vec_kernel<5, false, false, false, true>), g, b, 0, s, x, resid, gamma, beta, eps, o,
+                       rows, d, nullptr, nullptr, 0, nullptr, 0);
+  else
+    hipLaunchKernelGGL((layernorm_vec_kernel<10, false, false, false, true>), g, b, 0, s, x, resid, gamma, beta, eps,
+                       o, rows, d, nullptr, nullptr, 0, nullptr, 0);
+  return hipGetLastError();
+}
+
+hipError_t launch_split_rows(const float* x, size_t n, uint16_t* out, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  if (n % 32 != 0) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(split_rows_kernel, grid_for(n / 4), dim3(256), 0, s, x, n, out);
   return hipGetLastError();
 }
 

@@ -19,6 +19,9 @@
 // (lane / 16) owns the eight consecutive k values [8g, 8g+8): MFMA step j
 // multiplies A and W at k = 8g + j for every lane group, which keeps A and W
 // consistent and lets each lane fetch its k values with two 16-byte LDS reads.
+#include <algorithm>
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 
@@ -146,145 +149,6 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const GemmF32Args
   }
 }
 
-// ---- Split-fp16 GEMM (fp32 accuracy on fp16 MFMA), same 128x128 tile and
-// wave layout as above on v_mfma_f32_16x16x32_f16: each lane holds eight
-// consecutive k of one row for A and W, so one MFMA covers a 32-wide K stage.
-// A (fp32) is split into hi / lo fp16 planes while it is staged in LDS; W's
-// planes come split. LDS rows are 64 bytes (four 16-byte chunks), chunk c of
-// row r stored at position c ^ ((r / 4) mod 4): the 16-byte fragment reads
-// of 16 rows at one chunk then cover all 64 banks once, and so do the stage
-// writes of four consecutive rows (an 80-byte padded pitch kept the reads
-// conflict-free but made every write pass conflict).
-constexpr int kX3Pitch = 64;                    // bytes per 32-half row
-constexpr int kX3Plane = 128 * kX3Pitch;        // one 128-row plane
-constexpr int kX3Stage = 4 * kX3Plane;          // A hi, A lo, W hi, W lo
-
-// Byte offset of 16-byte chunk c of row r in a plane.
-__device__ __forceinline__ int x3_off(int r, int c) { return r * kX3Pitch + ((c ^ ((r >> 2) & 3)) << 4); }
-
-__device__ __forceinline__ uint2 pack_f16x4(float a, float b, float c, float d) {
-  return make_uint2(static_cast<uint32_t>(f32_to_f16_bits(a)) | (static_cast<uint32_t>(f32_to_f16_bits(b)) << 16),
-                    static_cast<uint32_t>(f32_to_f16_bits(c)) | (static_cast<uint32_t>(f32_to_f16_bits(d)) << 16));
-}
-
-// One K stage of the tile from global memory: A 128 rows x 32 floats (four
-// float4 per thread), W planes 128 rows x 32 halves each (two 16-byte pieces
-// per plane per thread). Rows past the edge re-read the last valid row;
-// their results are never stored.
-__device__ __forceinline__ void x3_load(const GemmX3Args& p, int m0, int n0, int k0, f32x4 (&ra)[4],
-                                        i32x4 (&rh)[2], i32x4 (&rl)[2]) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int idx = t + kThreads * i;
-    const int row = min(m0 + (idx >> 3), p.M - 1);
-    ra[i] = *reinterpret_cast<const f32x4*>(p.A + static_cast<size_t>(row) * p.lda + k0 + (idx & 7) * 4);
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int idx = t + kThreads * i;
-    const int row = min(n0 + (idx >> 2), p.N - 1);
-    const size_t off = static_cast<size_t>(row) * p.ldw + k0 + (idx & 3) * 8;
-    rh[i] = *reinterpret_cast<const i32x4*>(p.w_hi + off);
-    rl[i] = *reinterpret_cast<const i32x4*>(p.w_lo + off);
-  }
-}
-
-// The stage into LDS: A split into hi / lo planes, W planes as loaded.
-__device__ __forceinline__ void x3_store(uint8_t* st, const f32x4 (&ra)[4], const i32x4 (&rh)[2],
-                                         const i32x4 (&rl)[2]) {
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int idx = t + kThreads * i;
-    const int off = x3_off(idx >> 3, (idx & 7) >> 1) + (idx & 1) * 8;
-    const f32x4 x = ra[i];
-    const float hx = f16_bits_to_f32(f32_to_f16_bits(x[0])), hy = f16_bits_to_f32(f32_to_f16_bits(x[1]));
-    const float hz = f16_bits_to_f32(f32_to_f16_bits(x[2])), hw = f16_bits_to_f32(f32_to_f16_bits(x[3]));
-    *reinterpret_cast<uint2*>(st + off) = pack_f16x4(hx, hy, hz, hw);
-    *reinterpret_cast<uint2*>(st + kX3Plane + off) = pack_f16x4(x[0] - hx, x[1] - hy, x[2] - hz, x[3] - hw);
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int idx = t + kThreads * i;
-    const int off = x3_off(idx >> 2, idx & 3);
-    *reinterpret_cast<i32x4*>(st + 2 * kX3Plane + off) = rh[i];
-    *reinterpret_cast<i32x4*>(st + 3 * kX3Plane + off) = rl[i];
-  }
-}
-
-template <int EPI>
-__global__ __launch_bounds__(kThreads, 2) void gemm_x3_kernel(const GemmX3Args p) {
-  __shared__ __attribute__((aligned(16))) uint8_t smem[2 * kX3Stage];
-  const int tiles_n = (p.N + BN - 1) / BN;
-  const int m0 = (blockIdx.x / tiles_n) * BM;
-  const int n0 = (blockIdx.x % tiles_n) * BN;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int lr = lane & 15, lg = lane >> 4;
-
-  f32x4 ra[4];
-  i32x4 rh[2], rl[2];
-  f32x4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int nk = p.K / 32;
-  x3_load(p, m0, n0, 0, ra, rh, rl);
-  x3_store(smem, ra, rh, rl);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const uint8_t* cur = smem + (kt & 1) * kX3Stage;
-    const bool more = kt + 1 < nk;
-    if (more) x3_load(p, m0, n0, (kt + 1) * 32, ra, rh, rl);
-    f16x8 ah[4], al[4], bh[4], bl[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ao = x3_off(wm * 64 + i * 16 + lr, lg);
-      const int bo = x3_off(wn * 64 + i * 16 + lr, lg);
-      ah[i] = *reinterpret_cast<const f16x8*>(cur + ao);
-      al[i] = *reinterpret_cast<const f16x8*>(cur + kX3Plane + ao);
-      bh[i] = *reinterpret_cast<const f16x8*>(cur + 2 * kX3Plane + bo);
-      bl[i] = *reinterpret_cast<const f16x8*>(cur + 3 * kX3Plane + bo);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int n = 0; n < 4; ++n) {
-        f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bh[n], acc[i][n], 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], bh[n], c, 0, 0, 0);
-        acc[i][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bl[n], c, 0, 0, 0);
-      }
-    if (more) x3_store(smem + ((kt + 1) & 1) * kX3Stage, ra, rh, rl);
-    __syncthreads();
-  }
-
-  const int rb0 = m0 + wm * 64, cb0 = n0 + wn * 64;
-#pragma unroll
-  for (int n = 0; n < 4; ++n) {
-    const int col = cb0 + n * 16 + lr;
-    if (col >= p.N) continue;
-    const float b = p.bias ? p.bias[col] : 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = rb0 + i * 16 + lg * 4 + r;
-        if (row >= p.M) continue;
-        float v = __builtin_fmaf(acc[i][n][r], p.w_unscale, b);
-        if constexpr (EPI == kF32Gelu) v = gelu_erf(v);
-        float* dst = p.C + static_cast<size_t>(row) * p.ldc + col;
-        if constexpr (EPI == kF32Resid) {
-          *dst += v;
-        } else {
-          *dst = v;
-        }
-      }
-  }
-}
-
 // ---- Tiled fp32 GEMM (K % 32 == 0, 16-byte aligned rows): 2 x 2 waves of
 // 16 MB x 16 NB outputs, a 32 MB x 32 NB workgroup tile.
 //
@@ -298,10 +162,20 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_x3_kernel(const GemmX3Args p
 //
 // v_mfma_f32_16x16x4_f32 takes 32 cycles for 512 operand bytes, so neither LDS
 // nor the stage loads bound the loop; what does is the matrix rate times how
-// evenly the tiles fall on the CUs (f32_tile_of). 1280 x 1280 at 7,777 rows:
+// evenly the tiles fall on the CUs (tile_of). 1280 x 1280 at 7,777 rows:
 // 303 us with 128x128 tiles staged through registers, 199 here (128 TFLOP/s;
 // 165 us at the rate of a large fp32 library product); at 66 rows and K = N =
 // 320, 33 -> 4.8 us.
+// X3: the split-fp16 GEMM on the same stages. A row of A or W holds, for each
+// 32 k, 64 bytes of hi parts and 64 bytes of lo parts (GemmX3Args), so a
+// 128-byte piece is again one K stage: chunk lg is a lane's eight hi halves, k
+// = 8 lg .. + 8, and chunk 4 + lg its lo halves, the operands of one
+// v_mfma_f32_16x16x32_f16 each; three of them per 16x16 block and stage (hi hi
+// + lo hi + hi lo). They take 48 cycles where the fp32 MFMAs take 256, so here
+// the stage traffic bounds the loop and the tiles want to be large. With A
+// split while it was staged through registers (128x128 tiles, 64-byte rows) the
+// ESM-2 650M lm dense took 58 / 62 / 409 us at 301 / 2,048 / 31,107 rows; 15 /
+// 35 / 359 here.
 template <int MB, int NB>
 struct F32Tile {
   static constexpr int BM = 32 * MB, BN = 32 * NB;
@@ -329,14 +203,16 @@ __device__ __forceinline__ void f32_dma16(const void* base, uint32_t off, uint32
 }
 
 // Output of four consecutive columns of one row, the epilogue applied.
-template <int EPI>
+// X3: the sums are first multiplied by c_unscale, in one rounding with the bias.
+template <int EPI, bool X3>
 __device__ __forceinline__ void f32_store4(const GemmF32Args& p, int row, int col, f32x4 v, bool vec_c) {
   if (row >= p.M || col >= p.N) return;
   float* dst = p.C + static_cast<size_t>(row) * p.ldc + col;
   const int n = min(4, p.N - col);
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    v[e] += p.bias && e < n ? p.bias[col + e] : 0.0f;
+    const float b = p.bias && e < n ? p.bias[col + e] : 0.0f;
+    v[e] = X3 ? __builtin_fmaf(v[e], p.c_unscale, b) : v[e] + b;
     if constexpr (EPI == kF32Gelu) v[e] = gelu_erf(v[e]);
   }
   if (vec_c && n == 4) {
@@ -349,7 +225,7 @@ __device__ __forceinline__ void f32_store4(const GemmF32Args& p, int row, int co
   }
 }
 
-template <int MB, int NB, int EPI>
+template <bool X3, int MB, int NB, int EPI>
 __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p, bool vec_c) {
   using TL = F32Tile<MB, NB>;
   constexpr int BM = TL::BM, BN = TL::BN, kPer = TL::kPer, kStage = TL::kStage, kNStage = TL::kNStage;
@@ -384,7 +260,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
   for (int st = 0; st < kNStage - 1; ++st)
     if (st < nk) load_stage(st, st);
 
-  constexpr int kChains = TL::kChains;
+  constexpr int kChains = X3 ? 1 : TL::kChains;
   f32x4 acc[kChains][MB][NB];
 #pragma unroll
   for (int x = 0; x < kChains; ++x)
@@ -394,8 +270,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
       for (int j = 0; j < NB; ++j) acc[x][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // Row R's chunk c of a stage: block R / 8, slot c ^ (R % 8).
   const int arow = wm * 16 * MB + lr, wrow = BM + wn * 16 * NB + lr;
+  using Frag = std::conditional_t<X3, f16x8, f32x4>;
   auto frag = [&](const uint8_t* st, int R, int h) {
-    return *reinterpret_cast<const f32x4*>(st + (R >> 3) * 1024 + (R & 7) * 128 + (((4 * h + lg) ^ (R & 7)) << 4));
+    return *reinterpret_cast<const Frag*>(st + (R >> 3) * 1024 + (R & 7) * 128 + (((4 * h + lg) ^ (R & 7)) << 4));
   };
   int buf = 0;
   for (int kt = 0; kt < nk; ++kt) {
@@ -409,8 +286,31 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
     if (kt + kNStage - 1 < nk) load_stage(kt + kNStage - 1, buf == 0 ? kNStage - 1 : buf - 1);
     const uint8_t* st = smem + buf * kStage;
     buf = buf + 1 == kNStage ? 0 : buf + 1;
+    if constexpr (X3) {
+      f16x8 ah[MB], al[MB], wh[NB], wl[NB];
+#pragma unroll
+      for (int i = 0; i < MB; ++i) {
+        ah[i] = frag(st, arow + 16 * i, 0);
+        al[i] = frag(st, arow + 16 * i, 1);
+      }
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        wh[j] = frag(st, wrow + 16 * j, 0);
+        wl[j] = frag(st, wrow + 16 * j, 1);
+      }
+#pragma unroll
+      for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], ah[i], acc[0][i][j], 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], al[i], c, 0, 0, 0);
+          acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[j], ah[i], c, 0, 0, 0);
+        }
+      continue;
+    }
     // The chains of a single-block wave advance together; otherwise one half
     // of the stage at a time keeps fewer fragments live.
+    if constexpr (!X3)
 #pragma unroll
     for (int h0 = 0; h0 < 2; h0 += kChains) {
       f32x4 fa[kChains][MB], fw[kChains][NB];
@@ -439,7 +339,7 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
     for (int j = 0; j < NB; ++j) {
       f32x4 v = acc[0][i][j];
       if constexpr (kChains == 2) v += acc[1][i][j];
-      f32_store4<EPI>(p, m0 + wm * 16 * MB + 16 * i + lr, n0 + wn * 16 * NB + 16 * j + 4 * lg, v, vec_c);
+      f32_store4<EPI, X3>(p, m0 + wm * 16 * MB + 16 * i + lr, n0 + wn * 16 * NB + 16 * j + 4 * lg, v, vec_c);
     }
 }
 
@@ -501,7 +401,7 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_f32_skinny_kernel(cons
   f32x4 v = part[0][wave][lane];
 #pragma unroll
   for (int w = 1; w < kSkinnyWaves; ++w) v += part[w][wave][lane];
-  f32_store4<EPI>(p, m0 + 16 * (wave / NB) + lr, n0 + 16 * (wave % NB) + 4 * lg, v, vec_c);
+  f32_store4<EPI, false>(p, m0 + 16 * (wave / NB) + lr, n0 + 16 * (wave % NB) + 4 * lg, v, vec_c);
 }
 
 }  // namespace
@@ -520,12 +420,12 @@ bool f32_vec_c(const GemmF32Args& p) { return p.ldc % 4 == 0 && reinterpret_cast
   }                                                                                           \
   return hipGetLastError()
 
-template <int MB, int NB>
+template <bool X3, int MB, int NB>
 hipError_t launch_f32_tile(const GemmF32Args& p, int epi, hipStream_t s) {
   using TL = F32Tile<MB, NB>;
   const bool vec_c = f32_vec_c(p);
   const dim3 grid(((p.M + TL::BM - 1) / TL::BM) * ((p.N + TL::BN - 1) / TL::BN)), block(256);
-  ESM_F32_EPI(gemm_f32_tile_kernel, MB, NB);
+  ESM_F32_EPI(gemm_f32_tile_kernel, X3, MB, NB);
 }
 
 template <int MB, int NB, int CH>
@@ -547,29 +447,45 @@ bool f32_tile_ok(const GemmF32Args& p) {
          static_cast<uint64_t>(p.M) * p.lda * 4 <= kLimit && static_cast<uint64_t>(p.N) * p.ldw * 4 <= kLimit;
 }
 
-// Index into {32x32, 64x64, 128x64}: the tile whose grid takes the least
-// time, (the most tiles any CU gets + 1/2) x the tile's outputs x its cost per
-// output. The costs are those of many rounds (2560 x 2560 at 16,000 rows:
-// 1,727 / 1,529 / 1,498 us); the half tile is the last round, in which a CU's
-// few remaining workgroups leave its matrix cores waiting. It follows the
-// measured order at 1280 x 1280: 33 / 44 / 48 us at 1,000 rows, 56 / 62 / 79 at
-// 1,768, 94 / 84 / 81 at 3,000, 224 / 199 / 230 at 7,777, 457 / 393 / 389 at
-// 16,000. (64x32 and 128x128 tiles were never more than 8% faster.)
-int f32_tile_of(int M, int N) {
-  static constexpr int kBM[3] = {32, 64, 128}, kBN[3] = {32, 64, 64};
-  static constexpr double kCost[3] = {1.17, 1.02, 1.0};
+// Tiles 0 .. n - 1 of {32x32, 64x64, 128x64, 128x128}: the one whose grid
+// takes the least time, (the most tiles any CU gets + 1/2) x the tile's
+// outputs x its cost per output. The costs are those of many rounds; the half
+// tile is the last round, in which a CU's few remaining workgroups leave its
+// matrix cores waiting.
+int tile_of(int M, int N, int n, const double* cost) {
+  static constexpr int kBM[4] = {32, 64, 128, 128}, kBN[4] = {32, 64, 64, 128};
   const int cus = device_cus();
   int best = 0;
   double best_t = 0.0;
-  for (int t = 0; t < 3; ++t) {
+  for (int t = 0; t < n; ++t) {
     const long tiles = static_cast<long>((M + kBM[t] - 1) / kBM[t]) * ((N + kBN[t] - 1) / kBN[t]);
-    const double c = (static_cast<double>((tiles + cus - 1) / cus) + 0.5) * kBM[t] * kBN[t] * kCost[t];
+    const double c = (static_cast<double>((tiles + cus - 1) / cus) + 0.5) * kBM[t] * kBN[t] * cost[t];
     if (t == 0 || c < best_t) {
       best = t;
       best_t = c;
     }
   }
   return best;
+}
+
+// fp32: 2560 x 2560 at 16,000 rows takes 1,727 / 1,529 / 1,498 us. The choice
+// follows the measured order at 1280 x 1280: 33 / 44 / 48 us at 1,000 rows, 56 /
+// 62 / 79 at 1,768, 94 / 84 / 81 at 3,000, 224 / 199 / 230 at 7,777, 457 / 393 /
+// 389 at 16,000. (64x32 and 128x128 tiles were never more than 8% faster.)
+constexpr double kF32Cost[3] = {1.17, 1.02, 1.0};
+
+// Split-fp16, bound by the stage traffic: 1280 x 1280 takes 15 / 21 / 35 / 48 us
+// at 301 rows, 45 / 35 / 38 / 50 at 2,048, 148 / 103 / 91 / 110 at 7,562, - / 423
+// / 376 / 359 at 31,107; 2560 x 2560 at 7,562 rows 617 / 358 / 339 / 305.
+constexpr double kX3Cost[4] = {2.2, 1.18, 1.07, 1.0};
+
+hipError_t launch_x3_tile(const GemmF32Args& p, int epi, hipStream_t s) {
+  switch (tile_of(p.M, p.N, 4, kX3Cost)) {
+    case 0: return launch_f32_tile<true, 1, 1>(p, epi, s);
+    case 1: return launch_f32_tile<true, 2, 2>(p, epi, s);
+    case 2: return launch_f32_tile<true, 4, 2>(p, epi, s);
+    default: return launch_f32_tile<true, 4, 4>(p, epi, s);
+  }
 }
 
 }  // namespace
@@ -582,18 +498,30 @@ hipError_t launch_gemm_narrow(const GemmF32Args& p, hipStream_t s) {
   return launch_f32_skinny<1, 3, 5>(p, kF32Store, s);
 }
 
-hipError_t launch_gemm_x3(const GemmX3Args& p, int epi, hipStream_t s) {
-  if (p.M <= 0 || p.N <= 0) return hipSuccess;
-  if (p.K <= 0 || p.K % 32 != 0 || p.lda % 4 != 0 || p.ldw % 8 != 0) return hipErrorInvalidValue;
-  const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-  const dim3 grid(tiles), block(kThreads);
-  switch (epi) {
-    case kF32Store: hipLaunchKernelGGL((gemm_x3_kernel<kF32Store>), grid, block, 0, s, p); break;
-    case kF32Gelu: hipLaunchKernelGGL((gemm_x3_kernel<kF32Gelu>), grid, block, 0, s, p); break;
-    case kF32Resid: hipLaunchKernelGGL((gemm_x3_kernel<kF32Resid>), grid, block, 0, s, p); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
+hipError_t launch_gemm_x3(const GemmX3Args& x, int epi, hipStream_t s) {
+  if (x.M <= 0 || x.N <= 0) return hipSuccess;
+  if (x.K <= 0 || x.K % 32 != 0) return hipErrorInvalidValue;
+  // The stage loads' 32-bit offsets reach 2^32 bytes of A and of W: larger
+  // operands go in pieces.
+  const int most = static_cast<int>(std::min<int64_t>(1 << 30, (int64_t{1} << 32) / (int64_t{x.K} * 4)));
+  for (int n0 = 0; n0 < x.N; n0 += most)
+    for (int m0 = 0; m0 < x.M; m0 += most) {
+      GemmF32Args p;
+      // Rows of K / 32 pieces of 128 bytes: the fp32 kernel's pitches.
+      p.A = reinterpret_cast<const float*>(x.A) + static_cast<size_t>(m0) * x.K;
+      p.W = reinterpret_cast<const float*>(x.W) + static_cast<size_t>(n0) * x.K;
+      p.lda = p.ldw = p.K = x.K;
+      p.c_unscale = x.w_unscale;
+      p.bias = x.bias ? x.bias + n0 : nullptr;
+      p.C = x.C + static_cast<size_t>(m0) * x.ldc + n0;
+      p.ldc = x.ldc;
+      p.M = std::min(most, x.M - m0);
+      p.N = std::min(most, x.N - n0);
+      if (!f32_tile_ok(p)) return hipErrorInvalidValue;
+      const hipError_t e = launch_x3_tile(p, epi, s);
+      if (e != hipSuccess) return e;
+    }
+  return hipSuccess;
 }
 
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epi, hipStream_t s) {
@@ -605,10 +533,10 @@ hipError_t launch_gemm_f32(const GemmF32Args& p, int epi, hipStream_t s) {
   const long tiles16 = static_cast<long>((p.M + 15) / 16) * ((p.N + 15) / 16);
   if (f32_skinny_ok(p) && p.K >= 512 && tiles16 <= device_cus()) return launch_f32_skinny<1, 1, 10>(p, epi, s);
   if (f32_tile_ok(p)) {
-    switch (f32_tile_of(p.M, p.N)) {
-      case 0: return launch_f32_tile<1, 1>(p, epi, s);
-      case 1: return launch_f32_tile<2, 2>(p, epi, s);
-      default: return launch_f32_tile<4, 2>(p, epi, s);
+    switch (tile_of(p.M, p.N, 3, kF32Cost)) {
+      case 0: return launch_f32_tile<false, 1, 1>(p, epi, s);
+      case 1: return launch_f32_tile<false, 2, 2>(p, epi, s);
+      default: return launch_f32_tile<false, 4, 2>(p, epi, s);
     }
   }
   const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);

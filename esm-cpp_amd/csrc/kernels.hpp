@@ -108,7 +108,7 @@ int gemm_i8_tile_rows(int M, int N, int K, int epi, int cus);
 int device_cus();
 // K splits of a kEpiF32 launch with a workspace (1: none): grids that leave
 // CUs idle split K when the estimated time of the split grid plus its dequant
-// pass beats the unsplit one's. *rows receives the tile code to use.
+// pass beats the unsplit one's. *rows receives the tile height to use.
 // fused: the partial planes are summed by the kernel that reads the result
 // (launch_layernorm_quant_split) instead of a pass of their own, which then
 // costs only that kernel's extra reads.
@@ -136,6 +136,7 @@ struct GemmF32Args {
   float* C = nullptr;
   int ldc = 0;
   int M = 0, N = 0, K = 0;
+  float c_unscale = 1.0f;  // set by launch_gemm_x3 (its w_unscale)
 };
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epilogue, hipStream_t s);
 // C = A W^T + bias for N <= 48 (the tied vocabulary decoder), fp32 MFMA, one
@@ -145,16 +146,14 @@ hipError_t launch_gemm_narrow(const GemmF32Args& p, hipStream_t s);
 // FP32-accurate GEMM on fp16 MFMA ("split-fp16"): every operand x is carried
 // as hi = fp16(x) and lo = fp16(x - hi), and every product as hi*hi + lo*hi +
 // hi*lo (22 significant bits per operand; the dropped lo*lo term is below
-// 2^-22 relative), accumulated in fp32. A is fp32 and split on the fly; W
-// arrives pre-split as two fp16 planes [N, ldw] holding W * 2^w_shift (the
-// shift keeps the lo parts of small weights out of the fp16 subnormal
-// range), which the epilogue undoes exactly. K % 32 == 0.
+// 2^-22 relative), accumulated in fp32. A [M, K] and W [N, K] arrive split
+// (W holds W * 2^w_shift, which keeps the lo parts of small weights out of the
+// fp16 subnormal range and which the epilogue undoes exactly): a row is K / 32
+// pieces of 128 bytes, the 32 hi parts of k = 32 b .. + 32 and then their lo
+// parts. 16-byte aligned, K % 32 == 0.
 struct GemmX3Args {
-  const float* A = nullptr;
-  int lda = 0;
-  const uint16_t* w_hi = nullptr;
-  const uint16_t* w_lo = nullptr;
-  int ldw = 0;
+  const uint16_t* A = nullptr;
+  const uint16_t* W = nullptr;
   float w_unscale = 1.0f;  // 2^-w_shift
   const float* bias = nullptr;
   float* C = nullptr;
@@ -231,6 +230,12 @@ hipError_t launch_layernorm(float* x, const float* resid, const float* gamma,
 hipError_t launch_layernorm_quant_tensor(float* x, const float* gamma, const float* beta, float eps, int rows, int d,
                                          const float* absmax, int8_t* q, int ldq, float* scales, hipStream_t s,
                                          int round16 = 0);
+// The same LayerNorm written as the split-fp16 GEMM's A rows (GemmX3Args).
+// d % 32 == 0, d <= 2560.
+hipError_t launch_layernorm_x3(float* x, const float* resid, const float* gamma, const float* beta, float eps,
+                               uint16_t* out, int rows, int d, hipStream_t s);
+// n fp32 values (rows of a multiple of 32) -> those rows.
+hipError_t launch_split_rows(const float* x, size_t n, uint16_t* out, hipStream_t s);
 // LayerNorm (with the same optional residual add) fused with per-token
 // symmetric int8 quantisation.
 hipError_t launch_layernorm_quant(float* x, const float* resid, const float* gamma,

@@ -103,6 +103,24 @@ def test_w8a8_lm_dense_split_matches_fp32_mfma(dev, w650_small, small_batch):
     np.testing.assert_allclose(split, f32, rtol=0, atol=1e-5 * scale)
 
 
+@pytest.mark.parametrize("T", [1, 33, 1101, 7603, 16001])
+def test_lm_dense_split_tiles(dev, T):
+    """The split-fp16 dense at row counts that take each of its tiles, one row
+    past them: against the fp32-MFMA dense to fp32 rounding noise (both sum
+    1,280 products in fp32; 1e-5 of the logit range, as above), and the same
+    bits where the LayerNorm output is split by a pass of its own because the
+    hidden states are wanted too."""
+    cfg = syn.EsmConfig("lm-head-only", 0, 1280, 20, 5120)
+    m = eg.Model(dev, syn.make_weights(cfg, seed=5, int8=True), int8=True)
+    b = syn.batch_from_lengths([T] if T > 2 else [3], seed=T)
+    split = m.forward_packed(b.ids, b.cu)
+    assert np.array_equal(m.forward_hidden_states(b.ids, b.cu)[0], split)
+    m.set_lm_dense_split(False)
+    f32 = m.forward_packed(b.ids, b.cu)
+    m.free()
+    assert np.abs(split - f32).max() <= 1e-5 * np.abs(f32).max()
+
+
 @pytest.mark.parametrize("per_token", [False, True])
 def test_gemm_tile_rows_do_not_change_logits(dev, w650_small, small_batch, per_token):
     """The INT8 GEMM's 64-, 128-, 256- and 320-row tiles (and the automatic
