@@ -369,16 +369,25 @@ __device__ __forceinline__ void split8(const float (&p)[8], f16x8* hi, f16x8* lo
 // registers of the chunk in flight leave three workgroups a CU.
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // any fp32 address
 
-template <bool LONG, bool F32>
-__global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
+//
+// QB: 16-query blocks per wave, so 64 QB queries per item: 2 (128-query
+// items), or 1 where a batch has few of those. NBUF chunk buffers: with one
+// workgroup or less on a CU nothing else covers the chunk loads' latency, so
+// the QB 1 form has the loads of three chunks in flight instead of one. 20
+// heads: one sequence of 66 tokens 10.2 -> 8.6 us, of 301 18.7 -> 15.3, of 512
+// 26.7 -> 20.4; past one 64-query item a CU the smaller items' extra key reads
+// cost more (8 x 256 tokens, 640 items: 22.8 -> 25.6).
+template <bool LONG, bool F32, int QB, int NBUF>
+__global__ __launch_bounds__(256, F32 ? 3 : QB == 1 ? 2 : 4) void attn_x3_kernel(
     const uint32_t* __restrict__ q, int ldq, const uint16_t* __restrict__ kh, const uint16_t* __restrict__ kl,
     const uint16_t* __restrict__ vh, const uint16_t* __restrict__ vl, int ldp, const float* __restrict__ fq,
     const float* __restrict__ fk, const float* __restrict__ fv, int ldf, float q_prescale, float s2,
     const int* __restrict__ cu, const AttnWork* __restrict__ work, float* __restrict__ out, int ld_out,
     float* __restrict__ part_max) {
-  // Two chunk buffers, each [K hi | K lo | V hi | V lo] planes of 64 rows x
-  // 128 bytes.
-  __shared__ __attribute__((aligned(1024))) uint8_t sbuf[2 * kChunkBytes];
+  // Chunk buffers, each [K hi | K lo | V hi | V lo] planes of 32 rows x 128
+  // bytes.
+  static_assert(NBUF == 2 || (NBUF == 4 && !F32), "two buffers, or four with direct loads");
+  __shared__ __attribute__((aligned(1024))) uint8_t sbuf[NBUF * kChunkBytes];
 
   const AttnWork w = work[blockIdx.x];
   const int start = cu[w.seq];
@@ -394,7 +403,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lr = lane & 15, lg = lane >> 4;
-  const int qbase = w.q0 + wave * 32;
+  const int qbase = w.q0 + wave * 16 * QB;
   const bool active = qbase < L;  // wave-uniform
 
   // Chunk loads: wave p moves plane p (K hi, K lo, V hi, V lo) as eight 1 KB
@@ -422,7 +431,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
   // block qb, positions [lg*8, lg*8+8) and [32+lg*8, 32+lg*8+8). The Q words
   // are loaded first and chunk 0 right behind them, so both round trips
   // overlap.
-  f16x8 qh[2][2], ql[2][2];
+  f16x8 qh[QB][2], ql[QB][2];
   f32x4u kr[2], vr[2];  // F32: the next chunk's dims of this thread
   // F32: this thread's row and 16-byte plane chunk of a key chunk.
   const int crow = tid >> 3, cc = tid & 7;
@@ -450,9 +459,9 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
   if constexpr (F32) {
     // Positions 32 half + 8 lg .. + 8 are dims 16 half + 4 lg .. + 4 and those
     // + 32, paired.
-    f32x4u x[2][2][2];
+    f32x4u x[QB][2][2];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
+    for (int qb = 0; qb < QB; ++qb) {
       const float* qp = fq + static_cast<size_t>(start + min(qbase + qb * 16 + lr, L - 1)) * ldf + hoff + 4 * lg;
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
@@ -462,7 +471,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
     }
     load_f32(0);
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
+    for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         uint32_t h[4], l[4];
@@ -474,9 +483,9 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
       }
     store_f32(0);
   } else {
-    uint4 qw[2][2][2];
+    uint4 qw[QB][2][2];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
+    for (int qb = 0; qb < QB; ++qb) {
       const int qi = min(qbase + qb * 16 + lr, L - 1);
       const uint32_t* qp = q + static_cast<size_t>(start + qi) * ldq + hoff;
 #pragma unroll
@@ -485,20 +494,26 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
         qw[qb][half][1] = *reinterpret_cast<const uint4*>(qp + half * 32 + lg * 8 + 4);
       }
     }
-    load_chunk(0, 0);
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
+    for (int c = 0; c < NBUF - 1; ++c)
+      if (c * KCX < L) load_chunk(c * KCX, c);
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
       for (int half = 0; half < 2; ++half) unpack8(qw[qb][half][0], qw[qb][half][1], &qh[qb][half], &ql[qb][half]);
   }
 
-  f32x4 o[2][4];
+  f32x4 o[QB][4];
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb)
+  for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
     for (int db = 0; db < 4; ++db) o[qb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float mrun[2] = {-INFINITY, -INFINITY};
-  float lrun[2] = {0.f, 0.f};
+  float mrun[QB], lrun[QB];
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    mrun[qb] = -INFINITY;
+    lrun[qb] = 0.f;
+  }
 
   // Fragment offsets inside a plane. K: row kb*16 + lr, chunks lg and 4 + lg
   // (kb*16 leaves the swizzle unchanged). V (transposing reads): row
@@ -516,15 +531,22 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
   // so no key needs masking.
   auto chunk = [&](int kc0, int nkeys, int buf, auto fullc_tag) {
     constexpr bool FULLC = decltype(fullc_tag)::value;
-    // This wave's loads of the chunk have landed; the barrier publishes
-    // everyone's and retires the previous chunk's reads of the other buffer,
-    // which then receives the next chunk, in flight during this one.
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (kc0 + KCX < L) {
+    // This wave's loads of the chunk have landed (those of the next NBUF - 2
+    // may still be in flight; vector memory operations complete in order); the
+    // barrier publishes everyone's and retires the previous chunk's reads of
+    // its buffer, which then receives chunk + NBUF - 1.
+    constexpr int kLoads = KCX / 8;  // a wave's loads per chunk
+    if (NBUF == 4 && kc0 + 2 * KCX < L)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * kLoads) : "memory");
+    else if (NBUF == 4 && kc0 + KCX < L)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kLoads) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kc0 + (NBUF - 1) * KCX < L) {
       if constexpr (F32)
         load_f32(kc0 + KCX);
       else
-        load_chunk(kc0 + KCX, buf ^ 1);
+        load_chunk(kc0 + (NBUF - 1) * KCX, (buf + NBUF - 1) % NBUF);
     }
     if (!active) return;
     const uint8_t* sKh = sbuf + buf * kChunkBytes;
@@ -533,7 +555,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
     const uint8_t* sVl = sKh + 3 * kPlaneBytes;
 
     const int nkb = FULLC ? KCX / 16 : (nkeys + 15) >> 4;
-    f32x4 s[KCX / 16][2];
+    f32x4 s[KCX / 16][QB];
 #pragma unroll
     for (int kb = 0; kb < KCX / 16; ++kb) {
       if (kb < nkb) {
@@ -542,7 +564,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
         const f16x8 kl0 = *reinterpret_cast<const f16x8*>(sKl + kb * 2048 + koff0);
         const f16x8 kl1 = *reinterpret_cast<const f16x8*>(sKl + kb * 2048 + koff1);
 #pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
+        for (int qb = 0; qb < QB; ++qb) {
           f32x4 acc = mma16(kh0, qh[qb][0], f32x4{0.f, 0.f, 0.f, 0.f});
           acc = mma16(kl0, qh[qb][0], acc);
           acc = mma16(kh0, ql[qb][0], acc);
@@ -557,9 +579,9 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
     // running max and the rescale of O happen first; the probabilities are
     // then formed, summed and split per key-block pair inside the PV loop, so
     // only one pair's fp16 fragments are live at a time.
-    float mnew[2], al[2];
+    float mnew[QB], al[QB];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) {
+    for (int qb = 0; qb < QB; ++qb) {
       float cmax = -INFINITY;
 #pragma unroll
       for (int kb = 0; kb < KCX / 16; ++kb) {
@@ -598,10 +620,10 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
 #pragma unroll
     for (int kp = 0; kp < KCX / 32; ++kp) {
       if (2 * kp < nkb) {
-        f16x8 pfh[2], pfl[2];
+        f16x8 pfh[QB], pfl[QB];
         const bool two = FULLC || 2 * kp + 1 < nkb;
 #pragma unroll
-        for (int qb = 0; qb < 2; ++qb) {
+        for (int qb = 0; qb < QB; ++qb) {
           float pr[8];
           float psum = 0.f;
 #pragma unroll
@@ -626,7 +648,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
           const f16x8 vfh = f16x8{vah[0], vah[1], vah[2], vah[3], vbh[0], vbh[1], vbh[2], vbh[3]};
           const f16x8 vfl = f16x8{val[0], val[1], val[2], val[3], vbl[0], vbl[1], vbl[2], vbl[3]};
 #pragma unroll
-          for (int qb = 0; qb < 2; ++qb) {
+          for (int qb = 0; qb < QB; ++qb) {
             f32x4 acc = mma16(vfh, pfh[qb], o[qb][db]);
             acc = mma16(vfl, pfh[qb], acc);
             o[qb][db] = mma16(vfh, pfl[qb], acc);
@@ -638,16 +660,13 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
 
   // Whole chunks, then the sequence's partial last chunk (if any).
   int kc0 = 0, buf = 0;
-  for (; kc0 + KCX <= L; kc0 += KCX, buf ^= 1) {
+  for (; kc0 + KCX <= L; kc0 += KCX, buf = (buf + 1) % NBUF) {
     chunk(kc0, KCX, buf, std::true_type{});
     // The other buffer's last reads ended before this chunk's barrier.
     if constexpr (F32)
       if (kc0 + KCX < L) store_f32(buf ^ 1);
   }
-  if (kc0 < L) {
-    chunk(kc0, L - kc0, buf, std::false_type{});
-    buf ^= 1;
-  }
+  if (kc0 < L) chunk(kc0, L - kc0, buf, std::false_type{});
 
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // every wave is done with the chunks
   if (!active) {
@@ -655,14 +674,14 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
     return;
   }
   // Output: rows of o[qb][db] are positions db*16 + 4 lg .. +4, i.e. dims i,
-  // i + 32, i + 1, i + 33 for i = 8 db + 2 lg. Each wave puts its 32 x 64
+  // i + 32, i + 1, i + 33 for i = 8 db + 2 lg. Each wave puts its 16 QB x 64
   // tile in natural order into its own 8 KB of the chunk buffers (free after
   // the barrier above), 256-byte rows with 16-byte unit u at u ^ (row % 16),
   // then stores whole rows: 16 lanes x 16 bytes per query.
   uint8_t* stage = sbuf + wave * 8192;
   auto soff = [](int row, int dim) { return row * 256 + (((dim >> 2) ^ (row & 15)) << 4) + ((dim & 3) << 2); };
 #pragma unroll
-  for (int qb = 0; qb < 2; ++qb) {
+  for (int qb = 0; qb < QB; ++qb) {
     float lt = lrun[qb];
     lt += __shfl_xor(lt, 16, kWave);
     lt += __shfl_xor(lt, 32, kWave);
@@ -678,7 +697,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : 4) void attn_x3_kernel(
   const int unit = lane & 15;
   float m = 0.0f;
 #pragma unroll
-  for (int r4 = 0; r4 < 8; ++r4) {
+  for (int r4 = 0; r4 < 4 * QB; ++r4) {
     const int row = r4 * 4 + (lane >> 4);
     const float4 val = *reinterpret_cast<const float4*>(stage + soff(row, unit * 4));
     const int qi = qbase + row;
@@ -896,31 +915,51 @@ hipError_t launch_attention_mfma(const uint16_t* q, const uint16_t* k,
 
 hipError_t launch_attention_x3(const uint32_t* q, int ldq, const uint16_t* kh, const uint16_t* kl, const uint16_t* vh,
                                const uint16_t* vl, int ldp, float q_prescale, const int* cu_seqlens,
-                               const AttnWork* work, int num_work, float* out, int ld_out, int max_len,
+                               const AttnWork* work, int num_work, int q_tile, float* out, int ld_out, int max_len,
                                hipStream_t s, float* part_max) {
   if (num_work <= 0) return hipSuccess;
   const float s2 = kLog2e / q_prescale;
-  if (max_len > kAttnLongSeq)
-    hipLaunchKernelGGL((attn_x3_kernel<true, false>), dim3(num_work), dim3(256), 0, s, q, ldq, kh, kl, vh, vl, ldp,
-                       nullptr, nullptr, nullptr, 0, q_prescale, s2, cu_seqlens, work, out, ld_out, part_max);
+#define ESM_ATTN_X3(...)                                                                                              \
+  hipLaunchKernelGGL((attn_x3_kernel<__VA_ARGS__>), dim3(num_work), dim3(256), 0, s, q, ldq, kh, kl, vh, vl, ldp,     \
+                     nullptr, nullptr, nullptr, 0, q_prescale, s2, cu_seqlens, work, out, ld_out, part_max)
+  if (q_tile == kAttnX3SmallQTile)
+    ESM_ATTN_X3(true, false, 1, 4);
+  else if (q_tile != kAttnMfmaQTile)
+    return hipErrorInvalidValue;
+  else if (max_len > kAttnLongSeq)
+    ESM_ATTN_X3(true, false, 2, 2);
   else
-    hipLaunchKernelGGL((attn_x3_kernel<false, false>), dim3(num_work), dim3(256), 0, s, q, ldq, kh, kl, vh, vl, ldp,
-                       nullptr, nullptr, nullptr, 0, q_prescale, s2, cu_seqlens, work, out, ld_out, part_max);
+    ESM_ATTN_X3(false, false, 2, 2);
+#undef ESM_ATTN_X3
   return hipGetLastError();
 }
 
 hipError_t launch_attention_x3_f32(const float* q, const float* k, const float* v, int ld, float q_prescale,
-                                   const int* cu_seqlens, const AttnWork* work, int num_work, float* out, int ld_out,
-                                   int max_len, hipStream_t s) {
+                                   const int* cu_seqlens, const AttnWork* work, int num_work, int q_tile, float* out,
+                                   int ld_out, int max_len, hipStream_t s) {
   if (num_work <= 0) return hipSuccess;
   const float s2 = kLog2e / q_prescale;
-  if (max_len > kAttnLongSeq)
-    hipLaunchKernelGGL((attn_x3_kernel<true, true>), dim3(num_work), dim3(256), 0, s, nullptr, 0, nullptr, nullptr,
-                       nullptr, nullptr, 0, q, k, v, ld, q_prescale, s2, cu_seqlens, work, out, ld_out, nullptr);
+#define ESM_ATTN_X3(...)                                                                                              \
+  hipLaunchKernelGGL((attn_x3_kernel<__VA_ARGS__>), dim3(num_work), dim3(256), 0, s, nullptr, 0, nullptr, nullptr,    \
+                     nullptr, nullptr, 0, q, k, v, ld, q_prescale, s2, cu_seqlens, work, out, ld_out, nullptr)
+  if (q_tile == kAttnX3SmallQTile)
+    ESM_ATTN_X3(true, true, 1, 2);
+  else if (q_tile != kAttnMfmaQTile)
+    return hipErrorInvalidValue;
+  else if (max_len > kAttnLongSeq)
+    ESM_ATTN_X3(true, true, 2, 2);
   else
-    hipLaunchKernelGGL((attn_x3_kernel<false, true>), dim3(num_work), dim3(256), 0, s, nullptr, 0, nullptr, nullptr,
-                       nullptr, nullptr, 0, q, k, v, ld, q_prescale, s2, cu_seqlens, work, out, ld_out, nullptr);
+    ESM_ATTN_X3(false, true, 2, 2);
+#undef ESM_ATTN_X3
   return hipGetLastError();
+}
+
+int attention_x3_q_tile(const int* cu, int batch, int heads) {
+  // 64-query items while there is at most one a CU (figures at attn_x3_kernel).
+  long items = 0;
+  for (int b = 0; b < batch; ++b)
+    items += static_cast<long>((cu[b + 1] - cu[b] + kAttnX3SmallQTile - 1) / kAttnX3SmallQTile) * heads;
+  return items <= device_cus() ? kAttnX3SmallQTile : kAttnMfmaQTile;
 }
 
 hipError_t launch_attention_f32(const float* q, const float* k, const float* v,

@@ -758,13 +758,14 @@ extern "C" int esm_gfx950_attention_varlen(esm_gfx950_ctx* ctx, const float* q, 
     int* d_cu;
     AttnWork* d_work;
     int nwork;
-    ESM_TRY(stage_attention_meta(ctx, cu_seqlens, batch_size, num_heads, kAttnMfmaQTile, 0, &d_cu, &d_work, &nwork,
-                                 true));
+    const int q_tile = attention_x3_q_tile(cu_seqlens, batch_size, num_heads);
+    ESM_TRY(stage_attention_meta(ctx, cu_seqlens, batch_size, num_heads, q_tile, 0, &d_cu, &d_work, &nwork, true));
     int max_len = 0;
     for (int b = 0; b < batch_size; ++b) max_len = std::max(max_len, cu_seqlens[b + 1] - cu_seqlens[b]);
     int slot;
     ESM_TRY(ctx->time_begin("attention", &slot));
-    ESM_HIP(ctx, launch_attention_x3_f32(q, k, v, ld, kQPrescale, d_cu, d_work, nwork, out, ld, max_len, ctx->stream));
+    ESM_HIP(ctx, launch_attention_x3_f32(q, k, v, ld, kQPrescale, d_cu, d_work, nwork, q_tile, out, ld, max_len,
+                                         ctx->stream));
     ESM_TRY(ctx->time_end(slot));
     ESM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return ESM_GFX950_OK;
@@ -964,6 +965,7 @@ struct esm_gfx950_model {
     hipStream_t stream = nullptr;    // null: the context stream
     int rope_len = 0;                // rows currently in the device rope tables
     int T = 0, B = 0, nwork = 0, t0 = 0;
+    int q_tile = 0;                  // queries per attention work item
     int maxL = 0;                    // longest sequence of the staged part
     size_t x86_score_floats = 0;     // attention_x86_score_floats of the staged part
   };
@@ -1510,7 +1512,7 @@ class ObsRun {
 bool ln_tensor_quant_ok(int d) { return d % 4 == 0 && d <= 2560; }
 
 int layer_int8(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const DevLayer& L, int round16, const Arena& a,
-               const Meta& md, int T, int nwork, int max_len, const float* resid_in, ObsRun* ob, int cus,
+               const Meta& md, int T, int nwork, int q_tile, int max_len, const float* resid_in, ObsRun* ob, int cus,
                const SplitResid* split_in = nullptr, SplitResid* split_out = nullptr) {
   const auto& c = m->cfg;
   const int d = c.hidden_size, f = c.intermediate_size, H = c.num_heads, dh = c.head_dim;
@@ -1623,7 +1625,7 @@ int layer_int8(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const DevLayer& L
       // FFN buffer, dead here) and one workgroup reduces them.
       float* part = !tok && static_cast<size_t>(nwork) * 4 <= Tf ? a.inter : nullptr;
       ESM_HIP(ctx, launch_attention_x3(w, 3 * d, h16 + 2 * d, h16 + 3 * d, h16 + 4 * d, h16 + 5 * d, 6 * d, kQPrescale,
-                                       md.cu, md.work, nwork, a.attn, d, max_len, s, part));
+                                       md.cu, md.work, nwork, q_tile, a.attn, d, max_len, s, part));
       if (part)
         ESM_HIP(ctx, launch_max_of(part, static_cast<size_t>(nwork) * 4, amax_attn, s));
       else if (!tok)
@@ -2102,8 +2104,11 @@ int stage_part(esm_gfx950_ctx* ctx, esm_gfx950_model* m, esm_gfx950_model::Part&
   // The x86-exact attention takes 64-query tiles, longest sequences first.
   const bool mfma_attn = c.weights_int8 && c.attention_mode != ESM_GFX950_ATTN_MODE_FP32 &&
                          m->numerics == ESM_GFX950_NUMERICS_DEFAULT;
+  const int q_tile = !mfma_attn ? kAttnF32QTile
+                     : c.attention_mode == ESM_GFX950_ATTN_MODE_F16X3 ? attention_x3_q_tile(mh.cu, B, H)
+                                                                       : kAttnMfmaQTile;
   std::vector<AttnWork> work;
-  build_work(mh.cu, B, H, mfma_attn ? kAttnMfmaQTile : kAttnF32QTile, &work, mfma_attn);
+  build_work(mh.cu, B, H, q_tile, &work, mfma_attn);
   if (work.size() > mh.work_cap)
     return ctx->fail(ESM_GFX950_INTERNAL, "batch_upload: attention work list (" + std::to_string(work.size()) +
                                               " items) exceeds its metadata region (" +
@@ -2121,6 +2126,7 @@ int stage_part(esm_gfx950_ctx* ctx, esm_gfx950_model* m, esm_gfx950_model::Part&
   P.t0 = t0;
   P.maxL = maxL;
   P.nwork = static_cast<int>(work.size());
+  P.q_tile = q_tile;
   P.x86_score_floats = attention_x86_score_floats(mh.cu, B, m->cfg.num_heads);
   return ESM_GFX950_OK;
 }
@@ -2174,7 +2180,7 @@ int forward_part(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const esm_gfx95
       const bool last = li + 1 == m->layers.size();
       // A captured forward keeps every layer's hidden state whole: no split-K
       // partial sums left for the next layer (int32 sums, same bits).
-      ESM_TRY(layer_int8(ctx, m, L, round16, a, md, T, nwork, P.maxL, pending, ob, cus, &pending_split,
+      ESM_TRY(layer_int8(ctx, m, L, round16, a, md, T, nwork, P.q_tile, P.maxL, pending, ob, cus, &pending_split,
                          last || cap ? nullptr : &split_out));
       pending = nullptr;  // fc2 added its output into hidden (or left split partials)
       pending_split = split_out;

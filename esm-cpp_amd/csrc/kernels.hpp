@@ -188,20 +188,24 @@ hipError_t launch_attention_mfma(const uint16_t* q, const uint16_t* k,
 // vh) and lo planes (kl, vl), row stride ldp elements, 16-byte aligned rows.
 // out is written in natural dim order. Softmax logits are (q.k) / q_prescale.
 // max_len: the batch's longest sequence; past kAttnLongSeq tokens the
-// long-sequence variant runs (same results, bit for bit).
+// long-sequence variant runs (same results, bit for bit). q_tile: queries per
+// work item, kAttnMfmaQTile or kAttnX3SmallQTile (the same bits);
+// attention_x3_q_tile picks it for a batch (host cu).
 // part_max (optional, 4 * num_work floats): each item's four waves' largest
 // |output|; launch_max_of over them gives the output's maximum.
 constexpr int kAttnLongSeq = 256;
+constexpr int kAttnX3SmallQTile = 64;
+int attention_x3_q_tile(const int* cu, int batch, int heads);
 hipError_t launch_attention_x3(const uint32_t* q, int ldq, const uint16_t* kh, const uint16_t* kl, const uint16_t* vh,
                                const uint16_t* vl, int ldp, float q_prescale, const int* cu_seqlens,
-                               const AttnWork* work, int num_work, float* out, int ld_out, int max_len,
+                               const AttnWork* work, int num_work, int q_tile, float* out, int ld_out, int max_len,
                                hipStream_t s, float* part_max = nullptr);
 // The same attention on fp32 q, k, v rows (token t, head h at base + t * ld +
 // h * 64), split inside the kernel: the results of splitting them into that
 // layout first, bit for bit.
 hipError_t launch_attention_x3_f32(const float* q, const float* k, const float* v, int ld, float q_prescale,
-                                   const int* cu_seqlens, const AttnWork* work, int num_work, float* out, int ld_out,
-                                   int max_len, hipStream_t s);
+                                   const int* cu_seqlens, const AttnWork* work, int num_work, int q_tile, float* out,
+                                   int ld_out, int max_len, hipStream_t s);
 // Exact fp32 path for any head_dim <= 128 (fp32 MFMA, softmax sum in double).
 hipError_t launch_attention_f32(const float* q, const float* k, const float* v,
                                 int ld, int head_dim, const int* cu_seqlens,

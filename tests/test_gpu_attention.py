@@ -265,3 +265,29 @@ def test_x3_splits_any_fp32_rows(dev, oracle, lengths, shift):
         outs.append(out.numpy())
     assert np.array_equal(outs[0], outs[1])
     np.testing.assert_allclose(outs[0], want, rtol=1e-5, atol=1e-5)
+
+
+def test_x3_small_items_are_bit_identical(dev):
+    """A batch with few (sequence, head, query) items takes 64-query items with
+    four chunk buffers, the same sequences inside a larger batch 128-query
+    ones: the same bits, at the op and through the forward, for lengths around
+    the 32-key chunks (one to twelve of them) and the item sizes."""
+    H, r = 2, rng(7)
+    few, many = [1, 32, 33, 64, 65, 97, 129, 370], [128] * 1400
+    cu = cu_from_lengths(few + many)
+    T, t = int(cu[-1]), sum(few)
+    q, k, v = _qkv(r, T, H, 64)
+    outs = []
+    for n, end in ((len(few), t), (len(few) + len(many), T)):
+        out = dev.empty((end, H * 64), np.float32)
+        dev.attention_varlen(dev.array(q[:end]), dev.array(k[:end]), dev.array(v[:end]), cu[:n + 1], H, 64, out,
+                             eg.ATTN_F16X3_MFMA)
+        outs.append(out.numpy()[:t])
+    assert np.array_equal(outs[0], outs[1])
+    cfg = syn.EsmConfig("two-heads", 1, 128, 2, 512)
+    m = eg.Model(dev, syn.make_weights(cfg, seed=9, int8=True), int8=True)
+    batch = syn.batch_from_lengths([max(3, n) for n in few + many], seed=4)
+    t = int(batch.cu[len(few)])
+    small = m.forward_packed(batch.ids[:t], batch.cu[:len(few) + 1])
+    assert np.array_equal(small, m.forward_packed(batch.ids, batch.cu)[:t])
+    m.free()
