@@ -36,6 +36,18 @@ constexpr int kKPitch = 64 * 2 + 16;    // bytes per key row of K (bf16)
 constexpr int kVPitch = KC * 2 + 16;    // bytes per dim row of V^T (fp16)
 constexpr float kLog2e = 1.4426950408889634f;
 
+// Maximum / sum over the four lanes with the same lane % 16.
+__device__ __forceinline__ float quad_max(float v) {
+  const LanePair p = lane_xor16(v);
+  const LanePair q = lane_xor32(fmaxf(p.a, p.b));
+  return fmaxf(q.a, q.b);
+}
+__device__ __forceinline__ float quad_sum(float v) {
+  const LanePair p = lane_xor16(v);
+  const LanePair q = lane_xor32(p.a + p.b);
+  return q.a + q.b;
+}
+
 __device__ __forceinline__ uint16_t bf16_to_f16_bits(uint16_t b) {
   return f32_to_f16_bits(bf16_bits_to_f32(b));
 }
@@ -172,8 +184,7 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
           }
         }
       }
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 16, kWave));
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 32, kWave));
+      cmax = quad_max(cmax);
       const float mnew = fmaxf(mrun[qb], cmax);
       const float alpha = exp2f(mrun[qb] - mnew);
       mrun[qb] = mnew;
@@ -224,8 +235,7 @@ __global__ __launch_bounds__(256) void attn_mfma_kernel(
 #pragma unroll
   for (int qb = 0; qb < 2; ++qb) {
     float lt = lrun[qb];
-    lt += __shfl_xor(lt, 16, kWave);
-    lt += __shfl_xor(lt, 32, kWave);
+    lt = quad_sum(lt);
     const float inv = 1.0f / lt;
     const int qi = qbase + qb * 16 + lr;
     if (qi < L) {
@@ -599,8 +609,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : QB == 1 ? 2 : 4) void attn_x3_kernel
           }
         }
       }
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 16, kWave));
-      cmax = fmaxf(cmax, __shfl_xor(cmax, 32, kWave));
+      cmax = quad_max(cmax);
       mnew[qb] = fmaxf(mrun[qb], cmax);
       // The running sum takes its rescale in one fused step with the chunk's
       // first probabilities, lrun = fma(lrun, alpha, psum), in both variants,
@@ -683,8 +692,7 @@ __global__ __launch_bounds__(256, F32 ? 3 : QB == 1 ? 2 : 4) void attn_x3_kernel
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     float lt = lrun[qb];
-    lt += __shfl_xor(lt, 16, kWave);
-    lt += __shfl_xor(lt, 32, kWave);
+    lt = quad_sum(lt);
     const float inv = 1.0f / lt;
     const int row = qb * 16 + lr;
 #pragma unroll
@@ -832,8 +840,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
 #pragma unroll
       for (int i = 0; i < 4; ++i) mx = fmaxf(mx, k0 + 16 * b + 4 * i + lg < L ? s[b][i] : -INFINITY);
   }
-  mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-  mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+  mx = quad_max(mx);
 
   double sum = 0.0;
   f32x4 acc[DB];

@@ -44,10 +44,10 @@ __device__ __forceinline__ float red16(const float (&v)[16]) {
 // the group gets the result). IEEE addition is commutative, so lane j and
 // lane j ^ m forming a + b and b + a agree bit for bit.
 __device__ __forceinline__ float red16_lanes(float v) {
-  const float t3 = v + __shfl_xor(v, 8, 16);
-  const float t6 = t3 + __shfl_xor(t3, 4, 16);
-  const float t8 = t6 + __shfl_xor(t6, 2, 16);
-  return t8 + __shfl_xor(t8, 1, 16);
+  const float t3 = v + lane_dpp<0x128>(v);    // lane ^ 8: rotation by 8
+  const float t6 = t3 + lane_dpp<0x124>(t3);  // lane ^ 4 (its value, by a rotation by 4)
+  const float t8 = t6 + lane_dpp<0x4e>(t6);   // lane ^ 2
+  return t8 + lane_dpp<0xb1>(t8);             // lane ^ 1
 }
 
 // glibc's expf (the std::exp of the reference's x86 attention on its last
