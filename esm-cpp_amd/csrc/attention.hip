@@ -292,20 +292,6 @@ static_assert(2 * kChunkBytes >= 4 * 8192, "each wave's 32 x 64 fp32 output tile
 __device__ __forceinline__ int swz_k(int row) { return (row >> 1) & 7; }
 __device__ __forceinline__ int swz_v(int row) { return 2 * ((row >> 1) & 3); }
 
-// One 16-byte-per-lane global -> LDS load: a wave-uniform global base plus a
-// 32-bit lane offset, into the wave-uniform LDS byte address lds (M0).
-__device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32_t lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0v)
-               : "memory", "m0");
-#endif
-}
-
-__device__ __forceinline__ uint32_t lds_byte_addr(const void* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
-}
-
 // Low (sel_lo) or high (sel_hi) 16-bit halves of two words, packed: the hi
 // or lo fp16 parts of two consecutive values.
 constexpr uint32_t kSelLo = 0x05040100u, kSelHi = 0x07060302u;
@@ -377,8 +363,6 @@ __device__ __forceinline__ void split8(const float (&p)[8], f16x8* hi, f16x8* lo
 // re-read every operand: 64 sequences around 120 tokens (20 heads) took 76 us
 // in three packing launches plus 35 here, 41 us without them. The 16
 // registers of the chunk in flight leave three workgroups a CU.
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // any fp32 address
-
 //
 // QB: 16-query blocks per wave, so 64 QB queries per item: 2 (128-query
 // items), or 1 where a batch has few of those. NBUF chunk buffers: with one
@@ -763,12 +747,20 @@ __device__ __forceinline__ f32x4 transpose4(f32x4 x) {
 // One query per lane with scalar dot products (two passes of serial loads,
 // 1,840 waves for 16 sequences of 22-202 tokens, 20 heads of 16) took 351 us
 // on that batch, this form 29 us; one 66-token sequence 114 and 13 us.
-template <int DH, int KB, bool VEC>
+//
+// IT: the first pass keeps its scores in registers for sequences of at most 16
+// KB IT keys (the launcher passes IT only when every sequence is that short),
+// and the second pass forms no QK product; 0: the second pass forms them again.
+// That and addresses made of a uniform base and one lane offset per operand
+// (whole key blocks need no clamp) took those two from 29 and 13 us to 17
+// and 7.6.
+template <int DH, int KB, bool VEC, int IT>
 __global__ __launch_bounds__(256) void attn_f32_kernel(
     const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, int ld, int dh, const int* __restrict__ cu,
     const AttnWork* __restrict__ work, float* __restrict__ out, int ld_out) {
   constexpr int DB = DH / 16;  // 16-dim blocks
+  constexpr int KS = 16 * KB;  // keys per step
   const AttnWork w = work[blockIdx.x];
   const int start = cu[w.seq];
   const int L = cu[w.seq + 1] - start;
@@ -780,18 +772,18 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
   const float* kbase = k + base;
   const float* vbase = v + base;
 
-  // Dims 16 c + 4 lg .. + 4 of a row; dims past dh read as zero.
-  // (transpose4 then leaves dims 16 c + 4 j + lg in element j.)
-  auto load_dims = [&](const float* row, int c) {
+  // Dims 16 c + 4 lg .. + 4 of the row at base[off]; dims past dh read as
+  // zero. (transpose4 then leaves dims 16 c + 4 j + lg in element j.)
+  auto load_dims = [&](const float* row, uint32_t off, int c) {
     const int d0 = 16 * c + 4 * lg;
     if constexpr (VEC) {  // dh % 4 == 0
-      const f32x4 x = *reinterpret_cast<const f32x4*>(row + (d0 < dh ? d0 : 0));
+      const f32x4 x = *reinterpret_cast<const f32x4*>(row + (off + (d0 < dh ? d0 : 0)));
       return d0 < dh ? x : f32x4{0.f, 0.f, 0.f, 0.f};
     } else {
       f32x4 x;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const float y = row[d0 + j < dh ? d0 + j : 0];
+        const float y = row[off + (d0 + j < dh ? d0 + j : 0)];
         x[j] = d0 + j < dh ? y : 0.0f;
       }
       return x;
@@ -801,20 +793,23 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
   {
     const float* qp = q + base + static_cast<size_t>(min(q0 + lr, L - 1)) * ld;
 #pragma unroll
-    for (int c = 0; c < DB; ++c) qf[c] = transpose4(load_dims(qp, c));
+    for (int c = 0; c < DB; ++c) qf[c] = transpose4(load_dims(qp, 0, c));
   }
   // Scores of KB key blocks from key k0: element i of block b is key
-  // k0 + 16 b + 4 i + lg. Rows past the sequence repeat its last key.
+  // k0 + 16 b + 4 i + lg. Rows past the sequence (!FULL) repeat its last key.
   const int krow = 4 * (lr & 3) + (lr >> 2);
-  auto load_k = [&](int k0, f32x4(&kf)[KB][DB]) {
+  auto scores = [&](int k0, f32x4(&s)[KB], auto full) {
+    constexpr bool FULL = decltype(full)::value;
+    const float* kp = kbase + static_cast<size_t>(k0) * ld;
+    f32x4 kf[KB][DB];
 #pragma unroll
     for (int b = 0; b < KB; ++b) {
-      const float* kp = kbase + static_cast<size_t>(min(k0 + 16 * b + krow, L - 1)) * ld;
+      const int r = FULL ? krow : min(krow, L - 1 - k0 - 16 * b);  // may point before the block, not the sequence
 #pragma unroll
-      for (int c = 0; c < DB; ++c) kf[b][c] = load_dims(kp, c);
+      for (int c = 0; c < DB; ++c)
+        kf[b][c] = FULL ? load_dims(kp + 16 * b * ld, static_cast<uint32_t>(r * ld), c)
+                        : load_dims(kp + (16 * b + r) * ld, 0, c);
     }
-  };
-  auto scores = [&](f32x4(&kf)[KB][DB], f32x4(&s)[KB]) {
 #pragma unroll
     for (int b = 0; b < KB; ++b) {
       s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -829,48 +824,46 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
         for (int b = 0; b < KB; ++b)
           s[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[b][c][j], qf[c][j], s[b], 0, 0, 0);
   };
-
   float mx = -INFINITY;
-  for (int k0 = 0; k0 < L; k0 += 16 * KB) {
-    f32x4 kf[KB][DB], s[KB];
-    load_k(k0, kf);
-    scores(kf, s);
+  auto maximum = [&](int k0, f32x4(&s)[KB], auto full) {
+    scores(k0, s, full);
 #pragma unroll
     for (int b = 0; b < KB; ++b)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) mx = fmaxf(mx, k0 + 16 * b + 4 * i + lg < L ? s[b][i] : -INFINITY);
-  }
-  mx = quad_max(mx);
-
+      for (int i = 0; i < 4; ++i)
+        mx = fmaxf(mx, decltype(full)::value || k0 + 16 * b + 4 * i + lg < L ? s[b][i] : -INFINITY);
+  };
   double sum = 0.0;
   f32x4 acc[DB];
 #pragma unroll
   for (int c = 0; c < DB; ++c) acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int k0 = 0; k0 < L; k0 += 16 * KB) {
-    f32x4 kf[KB][DB], s[KB];
-    load_k(k0, kf);
+  auto weigh = [&](int k0, f32x4(&s)[KB], auto full) {
+    constexpr bool FULL = decltype(full)::value;
     // V of key k0 + 16 b + 4 j + lg, dim 16 c + lr. Keys past the sequence
     // read as zero (their weight is zero, but zero times infinity is not).
+    const float* vp = vbase + static_cast<size_t>(k0) * ld;
     float vf[KB][4][DB];
 #pragma unroll
     for (int b = 0; b < KB; ++b)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int key = k0 + 16 * b + 4 * j + lg;
-        const float* vp = vbase + static_cast<size_t>(min(key, L - 1)) * ld;
+        const int r = 16 * b + 4 * j;  // + lg
+        const bool ok = FULL || k0 + r + lg < L;
+        const int rc = FULL ? lg : min(lg, L - 1 - k0 - r);
 #pragma unroll
         for (int c = 0; c < DB; ++c) {
           const int d = 16 * c + lr;
-          const float x = vp[d < dh ? d : 0];
-          vf[b][j][c] = key < L && d < dh ? x : 0.0f;
+          const float x = FULL ? (vp + r * ld)[static_cast<uint32_t>(lg * ld + (d < dh ? d : 0))]
+                               : (vp + (r + rc) * ld)[d < dh ? d : 0];
+          vf[b][j][c] = ok && d < dh ? x : 0.0f;
         }
       }
-    scores(kf, s);
+    if constexpr (IT == 0) scores(k0, s, full);
 #pragma unroll
     for (int b = 0; b < KB; ++b) {
       f32x4 e;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) e[i] = k0 + 16 * b + 4 * i + lg < L ? expf(s[b][i] - mx) : 0.0f;
+      for (int i = 0; i < 4; ++i) e[i] = FULL || k0 + 16 * b + 4 * i + lg < L ? expf(s[b][i] - mx) : 0.0f;
       sum += (static_cast<double>(e[0]) + e[1]) + (static_cast<double>(e[2]) + e[3]);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -878,6 +871,28 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
         for (int c = 0; c < DB; ++c)
           acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[b][j][c], e[j], acc[c], 0, 0, 0);
     }
+  };
+  auto step = [&](int k0, f32x4(&s)[KB], auto& f) {
+    if (k0 + KS <= L)
+      f(k0, s, std::true_type{});
+    else
+      f(k0, s, std::false_type{});
+  };
+
+  if constexpr (IT > 0) {
+    f32x4 s[IT][KB];
+#pragma unroll
+    for (int t = 0; t < IT; ++t)
+      if (t * KS < L) step(t * KS, s[t], maximum);
+    mx = quad_max(mx);
+#pragma unroll
+    for (int t = 0; t < IT; ++t)
+      if (t * KS < L) step(t * KS, s[t], weigh);
+  } else {
+    f32x4 s[KB];
+    for (int k0 = 0; k0 < L; k0 += KS) step(k0, s, maximum);
+    mx = quad_max(mx);
+    for (int k0 = 0; k0 < L; k0 += KS) step(k0, s, weigh);
   }
   sum += __shfl_xor(sum, 16, kWave);
   sum += __shfl_xor(sum, 32, kWave);
@@ -972,7 +987,7 @@ int attention_x3_q_tile(const int* cu, int batch, int heads) {
 hipError_t launch_attention_f32(const float* q, const float* k, const float* v,
                                 int ld, int head_dim, const int* cu_seqlens,
                                 const AttnWork* work, int num_work, float* out,
-                                int ld_out, hipStream_t s) {
+                                int ld_out, int max_len, hipStream_t s) {
   if (num_work <= 0) return hipSuccess;
   if (head_dim <= 0 || head_dim > 128) return hipErrorInvalidValue;
   const dim3 grid(num_work), block(256);
@@ -980,25 +995,27 @@ hipError_t launch_attention_f32(const float* q, const float* k, const float* v,
   const uintptr_t bits = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
                          reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(out);
   const bool vec = head_dim % 4 == 0 && ld % 4 == 0 && ld_out % 4 == 0 && bits % 16 == 0;
-#define ESM_ATTN_F32(DH, KB)                                                                                      \
+#define ESM_ATTN_F32(DH, KB, IT)                                                                                  \
   do {                                                                                                            \
     if (vec)                                                                                                      \
-      hipLaunchKernelGGL((attn_f32_kernel<DH, KB, true>), grid, block, 0, s, q, k, v, ld, head_dim, cu_seqlens,   \
-                         work, out, ld_out);                                                                      \
+      hipLaunchKernelGGL((attn_f32_kernel<DH, KB, true, IT>), grid, block, 0, s, q, k, v, ld, head_dim,           \
+                         cu_seqlens, work, out, ld_out);                                                          \
     else                                                                                                          \
-      hipLaunchKernelGGL((attn_f32_kernel<DH, KB, false>), grid, block, 0, s, q, k, v, ld, head_dim, cu_seqlens,  \
-                         work, out, ld_out);                                                                      \
+      hipLaunchKernelGGL((attn_f32_kernel<DH, KB, false, IT>), grid, block, 0, s, q, k, v, ld, head_dim,          \
+                         cu_seqlens, work, out, ld_out);                                                          \
   } while (0)
   // Key blocks in flight: as many as keep the K and V fragments within about
-  // 128 registers.
-  if (head_dim <= 16)
-    ESM_ATTN_F32(16, 4);
-  else if (head_dim <= 32)
-    ESM_ATTN_F32(32, 4);
-  else if (head_dim <= 64)
-    ESM_ATTN_F32(64, 2);
-  else
-    ESM_ATTN_F32(128, 1);
+  // 128 registers. Scores are kept up to 256 keys: 64 registers.
+  const bool keep = max_len <= 256;
+  if (head_dim <= 16) {
+    if (keep) ESM_ATTN_F32(16, 4, 4); else ESM_ATTN_F32(16, 4, 0);
+  } else if (head_dim <= 32) {
+    if (keep) ESM_ATTN_F32(32, 4, 4); else ESM_ATTN_F32(32, 4, 0);
+  } else if (head_dim <= 64) {
+    if (keep) ESM_ATTN_F32(64, 2, 8); else ESM_ATTN_F32(64, 2, 0);
+  } else {
+    ESM_ATTN_F32(128, 1, 0);
+  }
 #undef ESM_ATTN_F32
   return hipGetLastError();
 }

@@ -701,7 +701,7 @@ extern "C" int esm_gfx950_rope_apply_varlen(esm_gfx950_ctx* ctx, float* x, const
   ESM_TRY(ctx->get_scratch(static_cast<size_t>(T) * 4, &s));
   ESM_HIP(ctx, hipMemcpyAsync(s, pos.data(), static_cast<size_t>(T) * 4, hipMemcpyHostToDevice, ctx->stream));
   ESM_HIP(ctx, launch_rope_f32(x, num_heads * head_dim, static_cast<int*>(s), T, num_heads, head_dim, cos, sin,
-                               head_dim, 1.0f, ctx->stream));
+                               head_dim, 1.0f, 0, ctx->stream));
   ESM_HIP(ctx, hipStreamSynchronize(ctx->stream));
   return ESM_GFX950_OK;
 }
@@ -746,7 +746,9 @@ extern "C" int esm_gfx950_attention_varlen(esm_gfx950_ctx* ctx, const float* q, 
     int nwork;
     ESM_TRY(stage_attention_meta(ctx, cu_seqlens, batch_size, num_heads, kAttnF32QTile, 0, &d_cu, &d_work, &nwork,
                                  false));
-    ESM_HIP(ctx, launch_attention_f32(q, k, v, ld, head_dim, d_cu, d_work, nwork, out, ld, ctx->stream));
+    int max_len = 0;
+    for (int b = 0; b < batch_size; ++b) max_len = std::max(max_len, cu_seqlens[b + 1] - cu_seqlens[b]);
+    ESM_HIP(ctx, launch_attention_f32(q, k, v, ld, head_dim, d_cu, d_work, nwork, out, ld, max_len, ctx->stream));
     ESM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return ESM_GFX950_OK;
   }
@@ -1601,8 +1603,7 @@ int layer_int8(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const DevLayer& L
     g.C_f32 = a.qkv;
     g.ldc = 3 * d;
     ESM_HIP(ctx, launch_gemm_i8(g, kEpiF32, s));
-    ESM_HIP(ctx, launch_rope_f32(a.qkv, 3 * d, md.pos, T, H, dh, md.cos_t, md.sin_t, dh, g.q_scale, s));
-    ESM_HIP(ctx, launch_rope_f32(a.qkv + d, 3 * d, md.pos, T, H, dh, md.cos_t, md.sin_t, dh, 1.0f, s));
+    ESM_HIP(ctx, launch_rope_f32(a.qkv, 3 * d, md.pos, T, 2 * H, dh, md.cos_t, md.sin_t, dh, g.q_scale, H, s));
   } else {
     g.q_out = a.qb;
     g.k_out = a.kb;
@@ -1632,7 +1633,7 @@ int layer_int8(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const DevLayer& L
         ESM_HIP(ctx, launch_absmax(a.attn, static_cast<size_t>(T) * d, amax_attn, s));
     } else {
       ESM_HIP(ctx, launch_attention_f32(a.qkv, a.qkv + d, a.qkv + 2 * d, 3 * d, dh, md.cu, md.work, nwork, a.attn,
-                                        d, s));
+                                        d, max_len, s));
       if (!tok) ESM_HIP(ctx, launch_absmax(a.attn, static_cast<size_t>(T) * d, amax_attn, s));
     }
   } else {
@@ -1789,7 +1790,7 @@ int layer_int8(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const DevLayer& L
   return ESM_GFX950_OK;
 }
 
-int f32_linear(esm_gfx950_ctx* ctx, const float* A, const DevLinear& W, float* C, int M, int epi) {
+GemmF32Args f32_linear_args(const float* A, const DevLinear& W, float* C, int M) {
   GemmF32Args p;
   p.A = A;
   p.lda = W.K;
@@ -1801,12 +1802,16 @@ int f32_linear(esm_gfx950_ctx* ctx, const float* A, const DevLinear& W, float* C
   p.M = M;
   p.N = W.N;
   p.K = W.K;
-  ESM_HIP(ctx, launch_gemm_f32(p, epi, ctx->stream));
+  return p;
+}
+
+int f32_linear(esm_gfx950_ctx* ctx, const float* A, const DevLinear& W, float* C, int M, int epi) {
+  ESM_HIP(ctx, launch_gemm_f32(f32_linear_args(A, W, C, M), epi, ctx->stream));
   return ESM_GFX950_OK;
 }
 
 int layer_f32(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const DevLayer& L, int round16, const Arena& a,
-              const Meta& md, int T, int nwork, ObsRun* ob) {
+              const Meta& md, int T, int nwork, int max_len, ObsRun* ob) {
   const auto& c = m->cfg;
   const int d = c.hidden_size, H = c.num_heads, dh = c.head_dim;
   hipStream_t s = ctx->stream;
@@ -1814,10 +1819,20 @@ int layer_f32(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const DevLayer& L,
   const size_t Td = static_cast<size_t>(T) * d, Tf = static_cast<size_t>(T) * c.intermediate_size;
   ESM_HIP(ctx, launch_layernorm(a.hidden, nullptr, L.ln1_w, L.ln1_b, c.layer_norm_eps, a.ln, T, d, nullptr, s));
   if (ob) ESM_TRY(ob->capture(ctx, a.ln, Td, 0));
-  ESM_TRY(f32_linear(ctx, a.ln, L.qkv, a.qkv, T, kF32Store));
-  ESM_HIP(ctx, launch_rope_f32(a.qkv, 3 * d, md.pos, T, H, dh, md.cos_t, md.sin_t, dh, q_scale, s));
-  ESM_HIP(ctx, launch_rope_f32(a.qkv + d, 3 * d, md.pos, T, H, dh, md.cos_t, md.sin_t, dh, 1.0f, s));
-  ESM_HIP(ctx, launch_attention_f32(a.qkv, a.qkv + d, a.qkv + 2 * d, 3 * d, dh, md.cu, md.work, nwork, a.attn, d, s));
+  GemmF32Args g = f32_linear_args(a.ln, L.qkv, a.qkv, T);
+  if (gemm_f32_rope_ok(g, dh)) {
+    g.d_model = d;
+    g.pos = md.pos;
+    g.rope_cos = md.cos_t;
+    g.rope_sin = md.sin_t;
+    g.q_scale = q_scale;
+    ESM_HIP(ctx, launch_gemm_f32(g, kF32QkvRope, s));
+  } else {
+    ESM_HIP(ctx, launch_gemm_f32(g, kF32Store, s));
+    ESM_HIP(ctx, launch_rope_f32(a.qkv, 3 * d, md.pos, T, 2 * H, dh, md.cos_t, md.sin_t, dh, q_scale, H, s));
+  }
+  ESM_HIP(ctx, launch_attention_f32(a.qkv, a.qkv + d, a.qkv + 2 * d, 3 * d, dh, md.cu, md.work, nwork, a.attn, d,
+                                    max_len, s));
   if (ob) ESM_TRY(ob->capture(ctx, a.attn, Td, 0));
   ESM_TRY(f32_linear(ctx, a.attn, L.out, a.hidden, T, kF32Resid));
   ESM_HIP(ctx, launch_layernorm(a.hidden, nullptr, L.ln2_w, L.ln2_b, c.layer_norm_eps, a.ln, T, d, nullptr, s,
@@ -2185,7 +2200,7 @@ int forward_part(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const esm_gfx95
       pending = nullptr;  // fc2 added its output into hidden (or left split partials)
       pending_split = split_out;
     } else {
-      ESM_TRY(layer_f32(ctx, m, L, round16, a, md, T, nwork, ob));
+      ESM_TRY(layer_f32(ctx, m, L, round16, a, md, T, nwork, P.maxL, ob));
     }
     if (cap && li + 1 < m->layers.size()) {
       if (pending) {

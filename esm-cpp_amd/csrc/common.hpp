@@ -12,6 +12,7 @@ namespace esm_gfx950 {
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // at any fp32 address
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -86,6 +87,21 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 __device__ __forceinline__ float wave_max(float v) {
   return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+
+// One 16-byte-per-lane global -> LDS load: a wave-uniform global base plus a
+// 32-bit lane offset, into the wave-uniform LDS byte address lds (M0). The
+// compiler does not see the LDS write: whoever reads it waits (vmcnt) first.
+__device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32_t lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds);
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0v)
+               : "memory", "m0");
+#endif
+}
+
+__device__ __forceinline__ uint32_t lds_byte_addr(const void* p) {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
 }
 
 // Split-fp16 word: fp16(x) in the low half, fp16(x - fp16(x)) in the high

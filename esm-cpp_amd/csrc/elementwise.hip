@@ -715,7 +715,8 @@ __global__ void scale_kernel(float* __restrict__ x, size_t n, float s) {
 // One thread per (token, head, i < head_dim/2) rotary pair.
 __global__ void rope_f32_kernel(float* __restrict__ x, int ld, const int* __restrict__ pos,
                                 int T, int heads, int dh, const float* __restrict__ cos_tab,
-                                const float* __restrict__ sin_tab, int tab_ld, float pre_scale) {
+                                const float* __restrict__ sin_tab, int tab_ld, float pre_scale,
+                                int scaled_heads) {
   const int half = dh / 2;
   const size_t total = static_cast<size_t>(T) * heads * half;
   for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < total;
@@ -728,7 +729,8 @@ __global__ void rope_f32_kernel(float* __restrict__ x, int ld, const int* __rest
     float* xr = x + static_cast<size_t>(t) * ld + static_cast<size_t>(h) * dh;
     const float* cr = cos_tab + static_cast<size_t>(p) * tab_ld;
     const float* sr = sin_tab + static_cast<size_t>(p) * tab_ld;
-    const float x1 = xr[c] * pre_scale, x2 = xr[c + half] * pre_scale;
+    const float f = h < scaled_heads ? pre_scale : 1.0f;
+    const float x1 = xr[c] * f, x2 = xr[c + half] * f;
     // Same fused forms as the QKV GEMM epilogue's rotation.
     xr[c] = __builtin_fmaf(x1, cr[c], -(x2 * sr[c]));
     xr[c + half] = __builtin_fmaf(x2, cr[c + half], x1 * sr[c + half]);
@@ -1028,11 +1030,11 @@ hipError_t launch_scale(float* x, size_t n, float scale, hipStream_t s) {
 
 hipError_t launch_rope_f32(float* x, int ld, const int* pos, int T, int heads, int head_dim,
                            const float* cos_tab, const float* sin_tab, int tab_ld, float pre_scale,
-                           hipStream_t s) {
+                           int scaled_heads, hipStream_t s) {
   const size_t n = static_cast<size_t>(T) * heads * (head_dim / 2);
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(rope_f32_kernel, grid_for(n), dim3(256), 0, s, x, ld, pos, T, heads, head_dim, cos_tab,
-                     sin_tab, tab_ld, pre_scale);
+                     sin_tab, tab_ld, pre_scale, scaled_heads);
   return hipGetLastError();
 }
 

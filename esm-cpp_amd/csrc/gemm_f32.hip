@@ -191,17 +191,6 @@ struct F32Tile {
   static constexpr int kChains = MB * NB == 1 ? 2 : 1;
 };
 
-// One 16-byte-per-lane global -> LDS load, as in the INT8 kernel: uniform
-// base, 32-bit lane offset, LDS byte address in M0; awaited by the explicit
-// vmcnt before the barrier that publishes the stage.
-__device__ __forceinline__ void f32_dma16(const void* base, uint32_t off, uint32_t lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0v)
-               : "memory", "m0");
-#endif
-}
-
 // Output of four consecutive columns of one row, the epilogue applied.
 // X3: the sums are first multiplied by c_unscale, in one rounding with the bias.
 template <int EPI, bool X3>
@@ -223,6 +212,28 @@ __device__ __forceinline__ void f32_store4(const GemmF32Args& p, int row, int co
     for (int e = 0; e < 4; ++e)
       if (e < n) dst[e] = EPI == kF32Resid ? dst[e] + v[e] : v[e];
   }
+}
+
+// kF32QkvRope, 16-wide heads: a 16-column block is one head, the lane's four
+// columns dims 4 lg .. + 4 of it, and the other half of its rotary pairs is in
+// lane ^ 32. The products of launch_rope_f32, in its fused forms; a pass of its
+// own per layer and operand took 2.6 / 4.7 us each at 66 / 1,768 rows.
+__device__ __forceinline__ f32x4 rope16(const GemmF32Args& p, int row, int col, f32x4 v) {
+  const int n0 = __builtin_amdgcn_readfirstlane(col) & ~15;
+  if (n0 >= 2 * p.d_model) return v;
+  const int lane = threadIdx.x & 63, d0 = 4 * (lane >> 4);
+  const size_t at = static_cast<size_t>(p.pos[min(row, p.M - 1)]) * 16 + d0;
+  const f32x4 c = *reinterpret_cast<const f32x4*>(p.rope_cos + at);
+  const f32x4 s = *reinterpret_cast<const f32x4*>(p.rope_sin + at);
+  const float f = n0 < p.d_model ? p.q_scale : 1.0f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    // The swap leaves dim d0 % 8 + e's value first, its partner's second, in
+    // both halves of the wave.
+    const LanePair x = lane_xor32(v[e] * f);
+    v[e] = lane < 32 ? __builtin_fmaf(x.a, c[e], -(x.b * s[e])) : __builtin_fmaf(x.b, c[e], x.a * s[e]);
+  }
+  return v;
 }
 
 template <bool X3, int MB, int NB, int EPI>
@@ -247,12 +258,11 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
     const int row = is_a ? min(m0 + b * 8 + r, p.M - 1) : min(n0 + (b - BM / 8) * 8 + r, p.N - 1);
     goff[i] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(is_a ? p.lda : p.ldw) + c * 4) * 4u;
   }
-  const uint32_t lds0 = static_cast<uint32_t>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)smem));
+  const uint32_t lds0 = lds_byte_addr(smem);
   auto load_stage = [&](int kt, int buf) {
 #pragma unroll
     for (int i = 0; i < kPer; ++i)
-      f32_dma16((wave * kPer + i < BM / 8 ? p.A : p.W) + kt * 32, goff[i],
+      lds_dma16((wave * kPer + i < BM / 8 ? p.A : p.W) + kt * 32, goff[i],
                 lds0 + static_cast<uint32_t>(buf * kStage + (wave * kPer + i) * 1024));
   };
   const int nk = p.K / 32;
@@ -339,7 +349,17 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
     for (int j = 0; j < NB; ++j) {
       f32x4 v = acc[0][i][j];
       if constexpr (kChains == 2) v += acc[1][i][j];
-      f32_store4<EPI, X3>(p, m0 + wm * 16 * MB + 16 * i + lr, n0 + wn * 16 * NB + 16 * j + 4 * lg, v, vec_c);
+      const int row = m0 + wm * 16 * MB + 16 * i + lr, col = n0 + wn * 16 * NB + 16 * j + 4 * lg;
+      if constexpr (EPI == kF32QkvRope) {
+        // N is a multiple of 16 (gemm_f32_rope_ok), so a block is in or out.
+        if (col < p.N) {
+          if (p.bias) v += *reinterpret_cast<const f32x4u*>(p.bias + col);
+          v = rope16(p, row, col, v);
+          if (row < p.M) *reinterpret_cast<f32x4*>(p.C + static_cast<size_t>(row) * p.ldc + col) = v;
+        }
+      } else {
+        f32_store4<EPI, X3>(p, row, col, v, vec_c);
+      }
     }
 }
 
@@ -425,6 +445,12 @@ hipError_t launch_f32_tile(const GemmF32Args& p, int epi, hipStream_t s) {
   using TL = F32Tile<MB, NB>;
   const bool vec_c = f32_vec_c(p);
   const dim3 grid(((p.M + TL::BM - 1) / TL::BM) * ((p.N + TL::BN - 1) / TL::BN)), block(256);
+  if constexpr (!X3) {
+    if (epi == kF32QkvRope) {
+      hipLaunchKernelGGL((gemm_f32_tile_kernel<false, MB, NB, kF32QkvRope>), grid, block, 0, s, p, vec_c);
+      return hipGetLastError();
+    }
+  }
   ESM_F32_EPI(gemm_f32_tile_kernel, X3, MB, NB);
 }
 
@@ -524,14 +550,27 @@ hipError_t launch_gemm_x3(const GemmX3Args& x, int epi, hipStream_t s) {
   return hipSuccess;
 }
 
+namespace {
+
+// At most one 16x16-tile workgroup a CU and a K long enough to be worth
+// splitting: N = 320 at 66 rows takes 6.4 / 6.5 / 6.6 / 6.7 us skinny for K
+// = 320 / 480 / 960 / 1280 against 4.8 / 6.0 / 9.7 / 12.2 in 32x32 tiles; a
+// second round of workgroups (301 rows) 11.4 against 12.4 at K = 1280.
+bool f32_takes_skinny(const GemmF32Args& p) {
+  const long tiles16 = static_cast<long>((p.M + 15) / 16) * ((p.N + 15) / 16);
+  return f32_skinny_ok(p) && p.K >= 512 && tiles16 <= device_cus();
+}
+
+}  // namespace
+
+bool gemm_f32_rope_ok(const GemmF32Args& p, int head_dim) {
+  return head_dim == 16 && p.N % 16 == 0 && f32_vec_c(p) && f32_tile_ok(p) && !f32_takes_skinny(p);
+}
+
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epi, hipStream_t s) {
   if (p.M <= 0 || p.N <= 0) return hipSuccess;
-  // At most one 16x16-tile workgroup a CU and a K long enough to be worth
-  // splitting: N = 320 at 66 rows takes 6.4 / 6.5 / 6.6 / 6.7 us skinny for K
-  // = 320 / 480 / 960 / 1280 against 4.8 / 6.0 / 9.7 / 12.2 in 32x32 tiles; a
-  // second round of workgroups (301 rows) 11.4 against 12.4 at K = 1280.
-  const long tiles16 = static_cast<long>((p.M + 15) / 16) * ((p.N + 15) / 16);
-  if (f32_skinny_ok(p) && p.K >= 512 && tiles16 <= device_cus()) return launch_f32_skinny<1, 1, 10>(p, epi, s);
+  if (epi == kF32QkvRope && !gemm_f32_rope_ok(p, 16)) return hipErrorInvalidValue;
+  if (f32_takes_skinny(p)) return launch_f32_skinny<1, 1, 10>(p, epi, s);
   if (f32_tile_ok(p)) {
     switch (tile_of(p.M, p.N, 3, kF32Cost)) {
       case 0: return launch_f32_tile<false, 1, 1>(p, epi, s);

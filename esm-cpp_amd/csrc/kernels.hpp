@@ -126,6 +126,8 @@ enum GemmF32Epilogue : int {
   kF32Store = 0,   // C = A W^T + bias
   kF32Gelu = 1,    // C = gelu(A W^T + bias)
   kF32Resid = 2,   // C += A W^T + bias
+  kF32QkvRope = 3, // kF32Store of Q|K|V rows, Q * q_scale and RoPE on Q and K
+                   // (gemm_f32_rope_ok)
 };
 struct GemmF32Args {
   const float* A = nullptr;
@@ -137,8 +139,17 @@ struct GemmF32Args {
   int ldc = 0;
   int M = 0, N = 0, K = 0;
   float c_unscale = 1.0f;  // set by launch_gemm_x3 (its w_unscale)
+  // kF32QkvRope: columns [0, d_model) are Q, the next d_model K; positions [M]
+  // and tables [max_len, 16] as launch_rope_f32 takes them.
+  int d_model = 0;
+  const int* pos = nullptr;
+  const float* rope_cos = nullptr;
+  const float* rope_sin = nullptr;
+  float q_scale = 1.0f;
 };
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epilogue, hipStream_t s);
+// Whether the launch can take kF32QkvRope: 16-wide heads on the tiled kernel.
+bool gemm_f32_rope_ok(const GemmF32Args& p, int head_dim);
 // C = A W^T + bias for N <= 48 (the tied vocabulary decoder), fp32 MFMA, one
 // wave per 16 rows; K % 16 == 0, lda and ldw multiples of 4.
 hipError_t launch_gemm_narrow(const GemmF32Args& p, hipStream_t s);
@@ -206,11 +217,12 @@ hipError_t launch_attention_x3(const uint32_t* q, int ldq, const uint16_t* kh, c
 hipError_t launch_attention_x3_f32(const float* q, const float* k, const float* v, int ld, float q_prescale,
                                    const int* cu_seqlens, const AttnWork* work, int num_work, int q_tile, float* out,
                                    int ld_out, int max_len, hipStream_t s);
-// Exact fp32 path for any head_dim <= 128 (fp32 MFMA, softmax sum in double).
+// Exact fp32 path for any head_dim <= 128 (fp32 MFMA, softmax sum in double);
+// max_len: the batch's longest sequence (an upper bound).
 hipError_t launch_attention_f32(const float* q, const float* k, const float* v,
                                 int ld, int head_dim, const int* cu_seqlens,
                                 const AttnWork* work, int num_work, float* out,
-                                int ld_out, hipStream_t s);
+                                int ld_out, int max_len, hipStream_t s);
 constexpr int kAttnMfmaQTile = 128;
 constexpr int kAttnF32QTile = 64;
 
@@ -299,12 +311,12 @@ hipError_t launch_gelu(const float* x, float* out, size_t n, hipStream_t s);
 hipError_t launch_residual_add(float* y, const float* x, size_t n,
                                hipStream_t s);
 hipError_t launch_scale(float* x, size_t n, float scale, hipStream_t s);
-// In-place RoPE on fp32 rows: x[t*ld + h*dh + i] for h < heads, each value
-// first multiplied by pre_scale (the Q scale; 1 for K).
+// In-place RoPE on fp32 rows: x[t*ld + h*dh + i] for h < heads, the values of
+// the first scaled_heads heads first multiplied by pre_scale (the Q scale).
 hipError_t launch_rope_f32(float* x, int ld, const int* pos, int T, int heads,
                            int head_dim, const float* cos_tab,
                            const float* sin_tab, int tab_ld, float pre_scale,
-                           hipStream_t s);
+                           int scaled_heads, hipStream_t s);
 hipError_t launch_embed(const int* ids, const float* tok_scale,
                         const float* embed, int T, int d, int mask_token_id,
                         float* out, hipStream_t s);

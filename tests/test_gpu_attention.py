@@ -221,17 +221,23 @@ class _Offset:
 @pytest.mark.parametrize("dh,shift", [(4, 0), (6, 0), (16, 0), (16, 1), (20, 0), (32, 0), (36, 1), (64, 0), (100, 0),
                                       (128, 0)])
 def test_fp32_path_block_edges(dev, oracle, dh, shift):
-    """Lengths around the 16-key blocks and 64-query tiles, head widths around
-    the padded ones, operands off a 16-byte boundary; an infinite V in the
+    """Lengths around the 16-key blocks, 64-query tiles and the 256 keys up to
+    which scores are kept, head widths around the padded ones, operands off a 16-byte boundary; an infinite V in the
     last key of a partial block reaches only what its weights reach. The
     bound is the scores' rounding: q is scaled, |score| < 8, so an exponential
     moves by at most 8 * 2^-24 * dh / 4 relative, under 1e-5 at dh 128."""
-    H, lengths = 3, [1, 15, 16, 17, 63, 64, 65, 129]
+    for lengths in ([1, 15, 16, 17, 63, 64, 65, 129], [17, 17, 255, 256, 31, 32, 33], [17, 17, 257, 17, 300]):
+        _fp32_block_edges(dev, oracle, dh, shift, lengths)
+
+
+def _fp32_block_edges(dev, oracle, dh, shift, lengths):
+    H = 3
     r = rng(dh + shift)
     cu = cu_from_lengths(lengths)
     T = int(cu[-1])
     q, k, v = _qkv(r, T, H, dh)
-    v[cu[4] - 1, 1, dh - 1] = np.inf  # the last key of the 17-token sequence
+    at = lengths.index(17)
+    v[cu[at + 1] - 1, 1, dh - 1] = np.inf  # the last key of a 17-token sequence
     pad = np.zeros(shift, np.float32)
     arrs = [dev.array(np.concatenate([pad, x.ravel()])) for x in (q, k, v)]
     out = dev.empty((T * H * dh + shift,), np.float32)
