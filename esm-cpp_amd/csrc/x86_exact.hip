@@ -883,6 +883,108 @@ __global__ __launch_bounds__(256) void linear_x86_wide_kernel(const float* __res
   }
 }
 
+// The same sums on the matrix cores (K % 64 == 0, 16-byte aligned rows):
+// v_mfma_f32_16x16x4_f32 adds its four products one after the other, fused and
+// rounded each, so accumulator lane l of a 16x16 block of outputs takes k = l, l
+// + 16, l + 32 and l + 48 of every 64 in one instruction, in LinearAvx512's
+// order. A wave holds all 16 lanes of 32 x 16 outputs (128 registers), which is
+// why it is not larger; a lane's operands for 16 of those instructions are 64
+// consecutive bytes of a row. 64 x 32 outputs per workgroup, 64-wide K stages
+// moved by direct global -> LDS loads into two buffers, rows in two 128-byte
+// pieces with chunk c at c ^ row % 8. The vector FMAs above run at under half
+// the fp32 matrix rate: 1280 x 1280 at 7,562 rows 674 -> 254 us, the decoder
+// (N = 33) 62 -> 21.
+constexpr int kMfmaM = 64, kMfmaN = 32;
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void linear_x86_mfma_kernel(const float* __restrict__ A, int lda,
+                                                                 const float* __restrict__ W, int ldw,
+                                                                 const float* __restrict__ bias, float* __restrict__ C,
+                                                                 int ldc, int M, int N, int K) {
+  constexpr int kPiece = (kMfmaM + kMfmaN) * 128, kStage = 2 * kPiece;
+  constexpr int kPer = kStage / 1024 / 4;  // 1 KB loads (8 rows x 128 bytes) per wave and stage
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * kStage];
+  int m0, n0;
+  tile_origin_of(blockIdx.x, M, N, kMfmaM, kMfmaN, &m0, &n0);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // Load b of a stage: piece b / 12, row group b % 12 (eight of A, four of W);
+  // rows past the edge repeat the last one.
+  constexpr int kGroups = (kMfmaM + kMfmaN) / 8;
+  uint32_t goff[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int b = wave * kPer + i, g = b % kGroups;
+    const int r = lane >> 3, c = (lane & 7) ^ r;
+    const bool is_a = g < kMfmaM / 8;
+    const int row = is_a ? min(m0 + g * 8 + r, M - 1) : min(n0 + (g - kMfmaM / 8) * 8 + r, N - 1);
+    goff[i] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(is_a ? lda : ldw) +
+               static_cast<uint32_t>(32 * (b / kGroups) + 4 * c)) * 4u;
+  }
+  const uint32_t lds0 = lds_byte_addr(smem);
+  auto load_stage = [&](int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int b = wave * kPer + i;
+      lds_dma16((b % kGroups < kMfmaM / 8 ? A : W) + kt * 64, goff[i],
+                lds0 + static_cast<uint32_t>(buf * kStage + b * 1024));
+    }
+  };
+  // Bytes 64 lg .. + 64 of a 64-wide stage row: the lane's values of the 16
+  // accumulator lanes.
+  auto frag = [&](const uint8_t* st, int row, f32x4(&x)[4]) {
+    const uint8_t* p = st + (lg >> 1) * kPiece + (row >> 3) * 1024 + (row & 7) * 128;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      x[j] = *reinterpret_cast<const f32x4*>(p + (((4 * (lg & 1) + j) ^ (row & 7)) << 4));
+  };
+  const int nk = K / 64;
+  load_stage(0, 0);
+  f32x4 acc[2][16];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int l = 0; l < 16; ++l) acc[i][l] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int kt = 0; kt < nk; ++kt) {
+    // Stage kt has landed, and every wave is done with the other buffer.
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt + 1 < nk) load_stage(kt + 1, (kt + 1) & 1);
+    const uint8_t* st = smem + (kt & 1) * kStage;
+    f32x4 a[2][4], w[4];
+    frag(st, kMfmaM + wn * 16 + lr, w);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) frag(st, wm * 32 + i * 16 + lr, a[i]);
+#pragma unroll
+    for (int l = 0; l < 16; ++l)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        acc[i][l] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[l >> 2][l & 3], a[i][l >> 2][l & 3], acc[i][l], 0, 0, 0);
+  }
+  // Element e of the lane: row lr of its 16-row block, column 4 lg + e.
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int m = m0 + wm * 32 + i * 16 + lr;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int n = n0 + wn * 16 + 4 * lg + e;
+      float v[16];
+#pragma unroll
+      for (int l = 0; l < 16; ++l) v[l] = acc[i][l][e];
+      if (m >= M || n >= N) continue;
+      const float y = (bias ? bias[n] : 0.0f) + red16(v);
+      float* c = C + static_cast<size_t>(m) * ldc + n;
+      if constexpr (EPI == kF32Gelu) {
+        *c = gelu_x86(y);
+      } else if constexpr (EPI == kF32Resid) {
+        *c = *c + y;
+      } else {
+        *c = y;
+      }
+    }
+  }
+}
+
 int grid_for(size_t n, int block, int cap) {
   const size_t g = (n + block - 1) / block;
   return static_cast<int>(g < static_cast<size_t>(cap) ? g : cap);
@@ -1003,6 +1105,27 @@ hipError_t launch_linear_x86(const float* A, int lda, const float* W, int ldw, c
   if (M <= 0 || N <= 0) return hipSuccess;
   const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(W) % 16 == 0;
+  // The stage loads take 32-bit byte offsets.
+  constexpr uint64_t kLimit = 1ull << 32;
+  if (vec && M >= 32 && N >= 32 && K > 0 && K % 64 == 0 && static_cast<uint64_t>(M) * lda * 4 <= kLimit &&
+      static_cast<uint64_t>(N) * ldw * 4 <= kLimit) {
+    const dim3 grid(((M + kMfmaM - 1) / kMfmaM) * ((N + kMfmaN - 1) / kMfmaN)), block(256);
+    switch (epi) {
+      case kF32Store:
+        hipLaunchKernelGGL(linear_x86_mfma_kernel<kF32Store>, grid, block, 0, s, A, lda, W, ldw, bias, C, ldc, M, N,
+                           K);
+        break;
+      case kF32Gelu:
+        hipLaunchKernelGGL(linear_x86_mfma_kernel<kF32Gelu>, grid, block, 0, s, A, lda, W, ldw, bias, C, ldc, M, N, K);
+        break;
+      case kF32Resid:
+        hipLaunchKernelGGL(linear_x86_mfma_kernel<kF32Resid>, grid, block, 0, s, A, lda, W, ldw, bias, C, ldc, M, N,
+                           K);
+        break;
+      default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+  }
   if (vec && M >= 32 && N >= 32) {
     const dim3 grid((N + 31) / 32, (M + 31) / 32), block(256);
     switch (epi) {

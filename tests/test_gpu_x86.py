@@ -92,6 +92,28 @@ def test_linear_f32_avx512(dev, oracle, M, N, K):
     assert_bits(out.numpy(), oracle.x86_linear_f32(A, W, bias), f"linear {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K,scale", [
+    (32, 32, 64, 1.0), (33, 47, 64, 1.0), (64, 33, 128, 1.0), (65, 32, 192, 1.0), (129, 97, 320, 1.0),
+    (700, 65, 1280, 1.0), (65, 70, 256, 1e-19), (65, 70, 256, 1e-21), (40, 40, 128, 3e18),
+])
+def test_linear_f32_avx512_matrix_cores(dev, oracle, M, N, K, scale):
+    """K a multiple of 64 runs on the matrix cores: tile edges, one and several
+    stages, products and sums that are subnormal (scale 1e-19: partly, 1e-21:
+    all but the largest), zeros and sums that overflow, bit for bit."""
+    r = rng(M * N + K)
+    A = (scale * r.standard_normal((M, K))).astype(np.float32)
+    W = (scale * r.standard_normal((N, K))).astype(np.float32)
+    A[0, :7] = 0.0
+    W[1, 3:9] = -0.0
+    bias = np.zeros(N, np.float32) if scale < 1 else r.standard_normal(N).astype(np.float32)
+    out = dev.empty((M, N), np.float32)
+    dev.linear_f32_avx512(dev.array(A), dev.array(W), dev.array(bias), out, M, N, K)
+    want = oracle.x86_linear_f32(A, W, bias)
+    if scale == 1e-21:
+        assert np.mean(np.abs(want) < 1.2e-38) > 0.9 and np.any(want != 0)
+    assert_bits(out.numpy(), want, f"linear {M}x{N}x{K} scale {scale}")
+
+
 @pytest.mark.parametrize("dh", [16, 32, 64])
 def test_rope_and_attention_avx512(dev, oracle, dh):
     """Ragged lengths around the 16-key chunking (1, 15, 16, 17, ...) and a
