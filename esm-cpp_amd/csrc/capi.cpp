@@ -528,14 +528,21 @@ extern "C" int esm_gfx950_linear_i8_gelu_quant_r24(esm_gfx950_ctx* ctx, const in
 }
 
 namespace {
+// absmax: scratch of `slots` floats, at least one; kAbsmaxParts of them save the
+// fill and the atomics.
 int quantize_into(esm_gfx950_ctx* ctx, const float* x, int M, int K, int mode, int8_t* q, int ldq,
-                  float* scales, float* absmax_slot) {
+                  float* scales, float* absmax, int slots) {
   if (mode == ESM_GFX950_ACT_PER_TOKEN) {
     ESM_HIP(ctx, launch_quant_rows(x, 0, K, M, K, q, ldq, scales, ctx->stream));
   } else if (mode == ESM_GFX950_ACT_PER_TENSOR) {
-    ESM_HIP(ctx, launch_fill_f32(absmax_slot, 1, 0.0f, ctx->stream));
-    ESM_HIP(ctx, launch_absmax(x, static_cast<size_t>(M) * K, absmax_slot, ctx->stream));
-    ESM_HIP(ctx, launch_quant_tensor(x, K, M, K, absmax_slot, q, ldq, scales, ctx->stream));
+    int parts = 1;
+    if (slots >= kAbsmaxParts) {
+      ESM_HIP(ctx, launch_absmax_parts(x, static_cast<size_t>(M) * K, absmax, &parts, ctx->stream));
+    } else {
+      ESM_HIP(ctx, launch_fill_f32(absmax, 1, 0.0f, ctx->stream));
+      ESM_HIP(ctx, launch_absmax(x, static_cast<size_t>(M) * K, absmax, ctx->stream));
+    }
+    ESM_HIP(ctx, launch_quant_tensor(x, K, M, K, absmax, q, ldq, scales, ctx->stream, parts));
   } else {
     return ctx->fail(ESM_GFX950_INVALID_ARGUMENT, "unknown activation quantisation mode");
   }
@@ -548,8 +555,8 @@ extern "C" int esm_gfx950_quantize_act(esm_gfx950_ctx* ctx, const float* x, int 
   if (!ctx) return ESM_GFX950_INVALID_ARGUMENT;
   ESM_REQUIRE(ctx, x && q && scales && M >= 0 && K > 0 && ldq >= K, "quantize_act: bad arguments");
   void* s = nullptr;
-  ESM_TRY(ctx->get_scratch(256, &s));
-  return quantize_into(ctx, x, M, K, mode, q, ldq, scales, static_cast<float*>(s));
+  ESM_TRY(ctx->get_scratch(kAbsmaxParts * sizeof(float), &s));
+  return quantize_into(ctx, x, M, K, mode, q, ldq, scales, static_cast<float*>(s), kAbsmaxParts);
 }
 
 extern "C" int esm_gfx950_gelu_quantize_act(esm_gfx950_ctx* ctx, const float* x, int M, int K, int8_t* q, int ldq,
@@ -575,11 +582,11 @@ extern "C" int esm_gfx950_linear_i8(esm_gfx950_ctx* ctx, const float* A, const e
   const size_t qbytes = align_up(static_cast<size_t>(M) * ldq, 256);
   const size_t sbytes = align_up(static_cast<size_t>(M) * sizeof(float), 256);
   void* s = nullptr;
-  ESM_TRY(ctx->get_scratch(qbytes + sbytes + 256, &s));
+  ESM_TRY(ctx->get_scratch(qbytes + sbytes + kAbsmaxParts * sizeof(float), &s));
   auto* q = static_cast<int8_t*>(s);
   auto* scales = reinterpret_cast<float*>(static_cast<char*>(s) + qbytes);
   auto* amax = reinterpret_cast<float*>(static_cast<char*>(s) + qbytes + sbytes);
-  ESM_TRY(quantize_into(ctx, A, M, K, act_mode, q, ldq, scales, amax));
+  ESM_TRY(quantize_into(ctx, A, M, K, act_mode, q, ldq, scales, amax, kAbsmaxParts));
   return esm_gfx950_linear_i8_q(ctx, q, ldq, scales, W, bias, C, M, 0);
 }
 
@@ -606,8 +613,9 @@ extern "C" int esm_gfx950_linear_i8_noalloc(esm_gfx950_ctx* ctx, const float* A,
   char* base = static_cast<char*>(ctx->noalloc_scratch);
   auto* q = reinterpret_cast<int8_t*>(base);
   auto* scales = reinterpret_cast<float*>(base + qbytes);
-  auto* amax = reinterpret_cast<float*>(base + qbytes + sbytes);  // zeroed by quantize_into (fill kernel)
-  ESM_TRY(quantize_into(ctx, A, M, K, act_mode, q, ldq, scales, amax));
+  auto* amax = reinterpret_cast<float*>(base + qbytes + sbytes);
+  const int slots = static_cast<int>(std::min<size_t>(kAbsmaxParts, (kNoAllocScratchBytes - qbytes - sbytes) / sizeof(float)));
+  ESM_TRY(quantize_into(ctx, A, M, K, act_mode, q, ldq, scales, amax, slots));
   return esm_gfx950_linear_i8_q(ctx, q, ldq, scales, W, bias, C, M, 0);
 }
 

@@ -289,10 +289,15 @@ hipError_t launch_gelu_quant_rows_r24(const uint16_t* xh, const uint8_t* xl, int
 hipError_t launch_quant_rows(const void* x, int src_kind, int ldx, int rows,
                              int cols, int8_t* q, int ldq, float* scales,
                              hipStream_t s);
-// Per-tensor quantisation with scale = absmax/127 (absmax read on device).
+// Per-tensor quantisation with scale = absmax/127, absmax the largest of the
+// nparts device values (more than one: 16-byte aligned, a multiple of 4).
 hipError_t launch_quant_tensor(const float* x, int ldx, int rows, int cols,
                                const float* absmax, int8_t* q, int ldq,
-                               float* scales, hipStream_t s);
+                               float* scales, hipStream_t s, int nparts = 1);
+// max |x[i]| as *nparts block maxima (a multiple of 4, at most kAbsmaxParts);
+// parts need not be cleared.
+constexpr int kAbsmaxParts = 1024;
+hipError_t launch_absmax_parts(const float* x, size_t n, float* parts, int* nparts, hipStream_t s);
 hipError_t launch_absmax(const float* x, size_t n, float* absmax,
                          hipStream_t s);
 // *out = the largest of n non-negative floats x (NaNs ignored), one

@@ -167,6 +167,52 @@ def test_linear_int8_zero_sizes(dev):
     w.free()
 
 
+@pytest.mark.parametrize("M,K", [(1, 1), (1, 3), (2, 4096), (5, 6557), (33, 1284), (513, 16388), (1031, 8191)])
+@pytest.mark.parametrize("at", ["first", "last", "nan"])
+def test_per_tensor_scale_from_block_maxima(dev, M, K, at):
+    """The scale is the largest |x| wherever it stands, from one block of the
+    maximum pass to its most; NaN is left out, and an input of nothing but NaN
+    has scale 1. Scales and codes exactly."""
+    r = rng(M * 7 + K)
+    x = r.uniform(-1, 1, size=(M, K)).astype(np.float32)
+    flat = x.reshape(-1)
+    if at == "nan":
+        flat[:: max(1, flat.size // 5)] = np.nan
+    else:
+        flat[0 if at == "first" else -1] = -3.0
+    amax = np.nanmax(np.abs(flat)) if not np.isnan(flat).all() else np.float32(0)
+    scale = np.float32(amax) / np.float32(127) if amax > 0 else np.float32(1)
+    ldq = (K + 15) // 16 * 16
+    dx, dq, ds = dev.array(x), dev.empty((M, ldq), np.int8), dev.empty((M,), np.float32)
+    dev.quantize_act(dx, M, K, eg.ACT_PER_TENSOR, dq, ldq, ds)
+    assert np.array_equal(ds.numpy(), np.full(M, scale, np.float32))
+    q = dq.numpy()
+    ok = ~np.isnan(x)
+    want = np.clip(np.rint(np.where(ok, x, 0) * (np.float32(1) / scale)), -127, 127).astype(np.int8)
+    assert np.array_equal(q[:, :K][ok], want[ok]) and not q[:, K:].any()
+    for t in (dx, dq, ds):
+        t.free()
+
+
+@pytest.mark.parametrize("M", [52200, 52264])
+def test_noalloc_per_tensor_at_its_scratch_limit(dev, M):
+    """With less scratch left than the block maxima take (52,264 rows of 1,280)
+    the maximum goes through one slot: linear_i8's bits both ways."""
+    K, N = 1280, 33
+    r = rng(M)
+    A = r.standard_normal((M, K), dtype=np.float32)
+    w = dev.weight_i8(r.integers(-127, 128, size=(N, K)).astype(np.int8), np.full(N, 0.01, np.float32))
+    dA, d1, d2 = dev.array(A), dev.empty((M, N), np.float32), dev.empty((M, N), np.float32)
+    dev.linear_i8(dA, w, None, d1, M, N, K, eg.ACT_PER_TENSOR)
+    dev.linear_i8_noalloc(dA, w, None, d2, M, N, K, eg.ACT_PER_TENSOR)
+    assert np.array_equal(d1.numpy(), d2.numpy())
+    with pytest.raises(eg.Gfx950Error):
+        dev.linear_i8_noalloc(dA, w, None, d2, 52265 + 20, N, K, eg.ACT_PER_TENSOR)
+    for t in (dA, d1, d2):
+        t.free()
+    w.free()
+
+
 @pytest.mark.parametrize("M,K,ldq", [(333, 1280, 1280), (70, 5120, 5136), (41, 260, 272), (9, 5121, 5136)])
 @pytest.mark.parametrize("mode", [eg.ACT_PER_TENSOR, eg.ACT_PER_TOKEN])
 def test_quantize_act(dev, oracle, mode, M, K, ldq):
