@@ -57,6 +57,23 @@ def test_fp32_path(dev, oracle, H, dh, lengths):
     np.testing.assert_allclose(got, want, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("n", [3264, 3290])
+def test_work_list_at_the_pinned_staging_line(dev, n):
+    """20 heads x n sequences of 3: the list and offsets just inside the 1 MiB
+    of pinned staging and just past it, against the same sequences in halves."""
+    H, dh = 20, 16
+    r = rng(n)
+    T = 3 * n
+    q, k, v = _qkv(r, T, H, dh)
+    got, half = dev.empty((T, H * dh), np.float32), dev.empty((T // 2, H * dh), np.float32)
+    dev.attention_varlen(dev.array(q), dev.array(k), dev.array(v), cu_from_lengths([3] * n), H, dh, got, eg.ATTN_FP32)
+    for t0 in (0, T // 2):
+        s = slice(t0, t0 + T // 2)
+        dev.attention_varlen(dev.array(q[s]), dev.array(k[s]), dev.array(v[s]), cu_from_lengths([3] * (n // 2)), H, dh,
+                             half, eg.ATTN_FP32)
+        np.testing.assert_array_equal(got.numpy()[s], half.numpy())
+
+
 def _mfma_vs_oracle(dev, oracle, lengths, H, seed, scale_q=True, check_seqs=None):
     r = rng(seed)
     cu = cu_from_lengths(lengths)

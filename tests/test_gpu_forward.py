@@ -399,6 +399,26 @@ def test_parts_automatic_count(dev, w650_small, small_batch):
     m.free()
 
 
+def test_hidden_states_kept_buffer_and_parts(dev, w650_small, small_batch):
+    """The states' device buffer grows and stays; their copies run beside the
+    layers, in one group and in several: a model's later calls have the bits
+    of a fresh model's first."""
+    other = syn.batch_from_lengths([40, 300, 5, 77], seed=3)
+    fresh = {}
+    for name, b in (("small", small_batch), ("other", other)):
+        m = eg.Model(dev, w650_small, int8=True)
+        fresh[name] = m.forward_hidden_states(b.ids, b.cu)
+        m.free()
+    m = eg.Model(dev, w650_small, int8=True)
+    for parts in (1, 3, 1, 2):
+        m.set_parts(parts)
+        for name, b in (("other", other), ("small", small_batch), ("other", other)):
+            got = m.forward_hidden_states(b.ids, b.cu)
+            np.testing.assert_array_equal(got[0], fresh[name][0])
+            np.testing.assert_array_equal(got[1], fresh[name][1])
+    m.free()
+
+
 def test_parts_per_tensor_stays_whole(dev, w650_small, small_batch):
     """A per-tensor activation scale spans the batch: set_parts leaves such a
     batch in one group (same logits), and a batch staged in several groups
