@@ -1236,8 +1236,9 @@ int device_cus() {
 namespace {
 
 // The pipelined kernel's tiles. 64 .. 320: rows of a tile 256 columns wide,
-// but 64 is 64x64; kTile128x128 is 128x128.
+// but 64 is 64x64; kTile128x128 is 128x128 and kTile64x256 64x256.
 constexpr int kTile128x128 = 1128;
+constexpr int kTile64x256 = 1064;
 
 // A launch's estimated time in microseconds: whole rounds of workgroups over
 // the CUs at t = fixed + per_stage * stages each, and a last, partly filled
@@ -1252,11 +1253,15 @@ struct TileCost {
 };
 constexpr TileCost kTileCosts[] = {
     // 64x64: two share a CU; alone a workgroup takes 3.8 + 0.24 a stage. At
-    // 301 rows 6.2 us (N = K = 1280), 13.1 (K = 5120); the 64x256 tile it
-    // replaced took 8.2 and 21.9.
+    // 301 rows 6.2 us (N = K = 1280), 13.1 (K = 5120), where the 64x256 tile
+    // takes 8.2 and 21.9.
     {64, 64, 64, 2, 3.0, 0.42, 0.72},
-    // 128x128: the same rows and stage bytes per column as 64x256, no slower
-    // anywhere: 8.3 against 8.6 us at 2,048 rows (N = K = 1280).
+    // 64x256 and 128x128: the same MFMAs a workgroup. 128x128 loads 32 KB a
+    // stage instead of 40 and is faster over many stages: 21.1 against 22.8 us
+    // at 2,048 rows, N = 1280, K = 5120. 64x256 has the shorter epilogue and
+    // eight waves to fill the pipeline: 8.1 against 9.3 us at 500 rows,
+    // N = 5120, K = 1280, and 12.2 against 13.3 at 850 rows, N = K = 2560.
+    {kTile64x256, 64, 256, 1, 3.0, 0.445, 1.0},
     {kTile128x128, 128, 128, 1, 3.6, 0.42, 1.0},
     {128, 128, 256, 1, 4.0, 0.95, 0.75},
     {192, 192, 256, 1, 6.0, 1.28, 0.72},
@@ -1362,6 +1367,7 @@ namespace {
 hipError_t launch_v3_rows(const GemmI8Args& p, int epi, int rows, hipStream_t s) {
   switch (rows) {
     case 64: return launch_v3_tile<1, 1>(p, epi, s);
+    case kTile64x256: return launch_v3_tile<1, 4>(p, epi, s);
     case kTile128x128: return launch_v3_tile<2, 2>(p, epi, s);
     case 192: return launch_v3_tile<3>(p, epi, s);
     case 128: return launch_v3_tile<2>(p, epi, s);

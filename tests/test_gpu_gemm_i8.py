@@ -362,7 +362,9 @@ def test_linear_i8_gelu_quant_r24_rejects_bad_shapes(dev):
 @pytest.mark.parametrize("M,N,K", [
     (1, 64, 128), (70, 130, 128), (70, 130, 256), (63, 65, 384), (65, 63, 512), (130, 70, 640), (300, 1280, 768),
     (301, 5120, 1280), (1000, 130, 1280),   # 64x64, one to ten stages in four buffers
-    (2048, 1280, 1280), (1990, 1210, 5120), (1025, 3900, 256),  # 128x128
+    (2048, 1280, 1280), (1001, 3830, 1280), (333, 10240, 2560),  # 64x256
+    (2048, 1280, 5120), (1990, 1210, 5120),  # 128x128
+    (1025, 3900, 256),  # 128x256
     (4099, 5120, 1280), (2500, 3840, 1280), (4001, 2510, 2560),  # 192 rows
     (9001, 5121, 384),
 ])
