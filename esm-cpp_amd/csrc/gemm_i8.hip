@@ -3,7 +3,7 @@
 // embedding). Two kernels:
 //   - gemm_i8_v3_kernel (namespace v3 below): the main path whenever K is a
 //     multiple of 128 and rows are 16-byte aligned -- v_mfma_i32_32x32x32_i8,
-//     256x256 or 320x256 tiles, direct global -> LDS stage loads;
+//     tiles from 64x64 to 320x256, direct global -> LDS stage loads;
 //   - gemm_i8_kernel (TileCfg, described next): the general fallback for any
 //     other shape, v_mfma_i32_16x16x64_i8.
 //
@@ -345,7 +345,8 @@ __global__ __launch_bounds__(C::THREADS, 2) void gemm_i8_kernel(const GemmI8Args
 // block and 16-byte chunk (l%8) ^ (l/8) ^ (block & 1), so the LDS copy holds
 // chunk c of row r at position c ^ r ^ (block & 1). That XOR keeps the
 // 32x32x32 fragment reads (32 rows x one chunk per half-wave) on distinct
-// banks. Two 64 KB stages ping-pong with one barrier per stage: the barrier
+// banks. The stage buffers (two of the tall tiles, three or four of the small)
+// rotate with one barrier per stage, as here for two: the barrier
 // publishes stage kt (each wave waited for its own loads) and retires the
 // reads of stage kt-1, whose buffer then receives stage kt+1 while stage
 // kt's 64 MFMAs per wave run.

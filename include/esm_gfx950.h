@@ -147,11 +147,10 @@ int esm_gfx950_gemm_i8_i32(esm_gfx950_ctx* ctx, const int8_t* A, int lda, const 
                            int M, int32_t* C);
 
 /* Row height of the INT8 GEMM's workgroup tile for every later launch in the
- * process: 64, 128, 256, 320, or 0 (default) to pick per launch. The default
- * gives grids that fill the device's CUs the height whose grid needs the
- * fewer rows' worth of workgroup rounds (320 only for the plain dequant,
- * int32 and split-word outputs), and small-M grids 64, 128 or 256 rows by an
- * estimate of their time. Results do not depend on it; it exists for tuning
+ * process: 64 (64 columns wide), 128, 256, 320 (256 wide), or 0 (default) to
+ * pick per launch by an estimate of the grid's time, also among 64x256,
+ * 128x128 and 192x256 tiles (320 only for the plain dequant, int32 and
+ * split-word outputs). Results do not depend on it; it exists for tuning
  * and tests. No reference counterpart. INVALID_ARGUMENT for other values. */
 int esm_gfx950_set_gemm_tile_rows(int rows);
 
