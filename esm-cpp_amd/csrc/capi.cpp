@@ -726,6 +726,12 @@ extern "C" int esm_gfx950_rope_apply_varlen(esm_gfx950_ctx* ctx, float* x, const
 }
 
 namespace {
+// Whether n floats at a and n floats at b share memory.
+bool overlap(const float* a, const float* b, size_t n) {
+  const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+  return (x > y ? x - y : y - x) < n * sizeof(float);
+}
+
 // Uploads cu_seqlens and the work list into op scratch (after `reserve`
 // bytes used by the caller) and returns device pointers. Up to kOpMetaBytes
 // they go in one copy from the context's pinned staging, which the host does
@@ -789,19 +795,27 @@ extern "C" int esm_gfx950_attention_varlen(esm_gfx950_ctx* ctx, const float* q, 
     return ctx->fail(ESM_GFX950_INVALID_ARGUMENT, "attention_varlen: unknown precision");
   ESM_REQUIRE(ctx, head_dim == kHeadDimMfma, "attention_varlen: the MFMA path needs head_dim == 64");
   if (precision == ESM_GFX950_ATTN_F16X3_MFMA) {
-    // The kernel splits the fp32 operands itself (Q times kQPrescale).
+    // The kernel splits the fp32 operands itself (Q times kQPrescale), reading
+    // K and V while other workgroups write their output rows: an output that
+    // shares memory with them goes to scratch first. (A workgroup reads the Q
+    // rows that it writes, and those alone, so out == q needs no copy.)
+    const size_t n = static_cast<size_t>(T) * ld;
+    const bool shared = overlap(out, k, n) || overlap(out, v, n) || (out != q && overlap(out, q, n));
     int* d_cu;
     AttnWork* d_work;
     int nwork;
     const int q_tile = attention_x3_q_tile(cu_seqlens, batch_size, num_heads);
-    ESM_TRY(stage_attention_meta(ctx, cu_seqlens, batch_size, num_heads, q_tile, 0, &d_cu, &d_work, &nwork, true));
+    ESM_TRY(stage_attention_meta(ctx, cu_seqlens, batch_size, num_heads, q_tile, shared ? align_up(n * 4, 256) : 0,
+                                 &d_cu, &d_work, &nwork, true));
+    float* dst = shared ? static_cast<float*>(ctx->scratch) : out;
     int max_len = 0;
     for (int b = 0; b < batch_size; ++b) max_len = std::max(max_len, cu_seqlens[b + 1] - cu_seqlens[b]);
     int slot;
     ESM_TRY(ctx->time_begin("attention", &slot));
-    ESM_HIP(ctx, launch_attention_x3_f32(q, k, v, ld, kQPrescale, d_cu, d_work, nwork, q_tile, out, ld, max_len,
+    ESM_HIP(ctx, launch_attention_x3_f32(q, k, v, ld, kQPrescale, d_cu, d_work, nwork, q_tile, dst, ld, max_len,
                                          ctx->stream));
     ESM_TRY(ctx->time_end(slot));
+    if (shared) ESM_HIP(ctx, hipMemcpyAsync(out, dst, n * 4, hipMemcpyDeviceToDevice, ctx->stream));
     ESM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return ESM_GFX950_OK;
   }

@@ -266,8 +266,9 @@ int esm_gfx950_rope_apply_varlen(esm_gfx950_ctx* ctx, float* x, const float* cos
  * out fp32 [T, H*head_dim]. precision FP32 is the exact path (any
  * head_dim <= 128); BF16_MFMA rounds q/k to bf16 and v to fp16 on device
  * and runs the MFMA kernel (head_dim == 64); F16X3_MFMA runs the split-fp16
- * MFMA kernel on the fp32 inputs directly (head_dim == 64). cu_seqlens is a
- * HOST array. */
+ * MFMA kernel on the fp32 inputs directly (head_dim == 64). With BF16_MFMA
+ * and F16X3_MFMA out may share memory with q, k and v. cu_seqlens is a HOST
+ * array. */
 int esm_gfx950_attention_varlen(esm_gfx950_ctx* ctx, const float* q, const float* k, const float* v,
                                 const int* cu_seqlens, int batch_size, int num_heads, int head_dim,
                                 float* out, int precision);

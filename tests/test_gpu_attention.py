@@ -314,3 +314,29 @@ def test_x3_small_items_are_bit_identical(dev):
     small = m.forward_packed(batch.ids[:t], batch.cu[:len(few) + 1])
     assert np.array_equal(small, m.forward_packed(batch.ids, batch.cu)[:t])
     m.free()
+
+
+@pytest.mark.parametrize("precision", [eg.ATTN_BF16_MFMA, eg.ATTN_F16X3_MFMA])
+@pytest.mark.parametrize("at", [("q", 0), ("k", 0), ("v", 0), ("q", 5), ("k", -3), ("v", 7)])
+def test_output_over_an_input(dev, precision, at):
+    """The MFMA paths' output over one of their inputs, exactly or some rows
+    apart, equals the output elsewhere bit for bit: several query tiles a
+    sequence, so that other workgroups still read what one writes."""
+    name, rows = at
+    H, lengths = 3, [257, 1, 300, 64]
+    cu = cu_from_lengths(lengths)
+    T, ld, pad = int(cu[-1]), H * 64, 8
+    x = dict(zip("qkv", _qkv(rng(17), T, H, 64)))
+    want = dev.empty((T, ld), np.float32)
+    d = {n: dev.array(a) for n, a in x.items()}
+    dev.attention_varlen(d["q"], d["k"], d["v"], cu, H, 64, want, precision)
+    # The input inside a buffer with room for the shifted output.
+    held = dev.array(np.concatenate([np.zeros(pad * ld, np.float32), x[name].ravel(), np.zeros(pad * ld, np.float32)]))
+    base = held.ptr.value
+    ins = {n: a.ptr for n, a in d.items()}
+    ins[name] = type(held.ptr)(base + 4 * pad * ld)
+    out = type(held.ptr)(base + 4 * (pad + rows) * ld)
+    dev._check(dev.lib.esm_gfx950_attention_varlen(dev.ctx, ins["q"], ins["k"], ins["v"], cu.ctypes.data, len(lengths),
+                                                   H, 64, out, precision))
+    got = held.numpy()[(pad + rows) * ld:][:T * ld].reshape(T, ld)
+    np.testing.assert_array_equal(got, want.numpy())
