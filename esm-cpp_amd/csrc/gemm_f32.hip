@@ -7,12 +7,15 @@
 // Products are exact fp32 products accumulated in fp32, so results differ
 // from the sequential reference sum only by summation order.
 //
-// Three kernels (launch_gemm_f32 picks):
+// Three kernels (launch_gemm_f32 picks), and the decoder's:
 //   - gemm_f32_tile_kernel: aligned rows with K % 32 == 0; LDS tiles of 32x32
 //     to 128x64, direct global -> LDS stage loads;
-//   - gemm_f32_skinny_kernel: grids too small for that one (and the decoder's
-//     N <= 48): eight waves split K, operands straight into registers;
-//   - gemm_f32_kernel: any other shape (128x128 tiles through registers).
+//   - gemm_f32_pair_kernel: the same operands and the same sums bit for bit, for
+//     grids too small for that one: two waves to a 16x16 tile;
+//   - gemm_f32_kernel: any other shape (128x128 tiles through registers);
+//   - gemm_narrow_kernel: N <= 48, eight waves split K.
+// Which order a row is summed in is chosen by N, K and the alignment alone,
+// never by M: a sequence's logits do not depend on what it is batched with.
 //
 // gemm_f32_kernel's tiling: 128x128 workgroup tile, four waves of 64x64,
 // 32-wide K stages in LDS (row pitch 36 floats). Within a stage, lane group g
@@ -176,6 +179,15 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const GemmF32Args
 // split while it was staged through registers (128x128 tiles, 64-byte rows) the
 // ESM-2 650M lm dense took 58 / 62 / 409 us at 301 / 2,048 / 31,107 rows; 15 /
 // 35 / 359 here.
+//
+// The order of an output's sum depends on K alone: over kSumStages stages one
+// sum of the first and one of the second halves, the two added, and those added
+// in turn. gemm_f32_pair_kernel has the same. Sums of 160 products keep the
+// error of the eight-way split that small grids had before, at K = 1280 0.36 of
+// one long sum's standard deviation, and cost the large tiles 1% (2560 x 2560 at
+// 16,000 rows 1,488 -> 1,501 us). A second sum also keeps a 32x32 tile's wave off
+// a single chain of dependent MFMAs.
+constexpr int kSumStages = 10;
 template <int MB, int NB>
 struct F32Tile {
   static constexpr int BM = 32 * MB, BN = 32 * NB;
@@ -185,10 +197,6 @@ struct F32Tile {
   // More buffers only cost resident workgroups (1280 x 1280 at 1,000 rows,
   // 32x32 tiles: 33 us with three, 39 with five).
   static constexpr int kNStage = kStage <= 16384 ? 3 : 2;
-  // A single 16x16 block per wave would be one chain of dependent MFMAs, 52
-  // cycles each instead of the 32 they occupy the matrix core: its halves of a
-  // stage go to two accumulators.
-  static constexpr int kChains = MB * NB == 1 ? 2 : 1;
 };
 
 // Output of four consecutive columns of one row, the epilogue applied.
@@ -236,8 +244,23 @@ __device__ __forceinline__ f32x4 rope16(const GemmF32Args& p, int row, int col, 
   return v;
 }
 
+// Four consecutive columns of one row, as a wave holds a 16x16 block (lane (lr,
+// lg): row lr, columns 4 lg .. + 4; every lane reaches this).
+template <int EPI, bool X3>
+__device__ __forceinline__ void f32_out(const GemmF32Args& p, int row, int col, f32x4 v, bool vec_c) {
+  if constexpr (EPI == kF32QkvRope) {
+    // N is a multiple of 16 (gemm_f32_rope_ok), so a block is in or out.
+    if (col >= p.N) return;
+    if (p.bias) v += *reinterpret_cast<const f32x4u*>(p.bias + col);
+    v = rope16(p, row, col, v);
+    if (row < p.M) *reinterpret_cast<f32x4*>(p.C + static_cast<size_t>(row) * p.ldc + col) = v;
+  } else {
+    f32_store4<EPI, X3>(p, row, col, v, vec_c);
+  }
+}
+
 template <bool X3, int MB, int NB, int EPI>
-__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p, bool vec_c) {
+__global__ __launch_bounds__(256, MB * NB == 16 ? 1 : 3) void gemm_f32_tile_kernel(const GemmF32Args p, bool vec_c) {
   using TL = F32Tile<MB, NB>;
   constexpr int BM = TL::BM, BN = TL::BN, kPer = TL::kPer, kStage = TL::kStage, kNStage = TL::kNStage;
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kNStage * kStage];
@@ -270,14 +293,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
   for (int st = 0; st < kNStage - 1; ++st)
     if (st < nk) load_stage(st, st);
 
-  constexpr int kChains = X3 ? 1 : TL::kChains;
+  // fp32: one sum of the first and one of the second halves of the stages.
+  constexpr int kChains = X3 ? 1 : 2;
   f32x4 acc[kChains][MB][NB];
-#pragma unroll
-  for (int x = 0; x < kChains; ++x)
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-      for (int j = 0; j < NB; ++j) acc[x][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   // Row R's chunk c of a stage: block R / 8, slot c ^ (R % 8).
   const int arow = wm * 16 * MB + lr, wrow = BM + wn * 16 * NB + lr;
   using Frag = std::conditional_t<X3, f16x8, f32x4>;
@@ -285,7 +303,9 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
     return *reinterpret_cast<const Frag*>(st + (R >> 3) * 1024 + (R & 7) * 128 + (((4 * h + lg) ^ (R & 7)) << 4));
   };
   int buf = 0;
-  for (int kt = 0; kt < nk; ++kt) {
+  // first: the sums start with this stage.
+  auto stage = [&](int kt, auto first) {
+    constexpr bool FIRST = decltype(first)::value;
     // Stage kt has landed (this wave's loads, then everyone's behind the
     // barrier), and every wave is done with stage kt - 1, whose buffer
     // receives stage kt + kNStage - 1.
@@ -312,83 +332,173 @@ __global__ __launch_bounds__(256) void gemm_f32_tile_kernel(const GemmF32Args p,
       for (int i = 0; i < MB; ++i)
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
-          f32x4 c = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], ah[i], acc[0][i][j], 0, 0, 0);
+          f32x4 c = FIRST ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[0][i][j];
+          c = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], ah[i], c, 0, 0, 0);
           c = __builtin_amdgcn_mfma_f32_16x16x32_f16(wh[j], al[i], c, 0, 0, 0);
           acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(wl[j], ah[i], c, 0, 0, 0);
         }
-      continue;
-    }
-    // The chains of a single-block wave advance together; otherwise one half
-    // of the stage at a time keeps fewer fragments live.
-    if constexpr (!X3)
+    } else {
+      // A single-block wave advances both sums together: one alone is a chain
+      // of dependent MFMAs, 52 cycles each instead of the 32 they occupy the
+      // matrix core. Otherwise one half of the stage at a time keeps fewer
+      // fragments live.
+      constexpr int kPair = MB * NB == 1 ? 2 : 1;
 #pragma unroll
-    for (int h0 = 0; h0 < 2; h0 += kChains) {
-      f32x4 fa[kChains][MB], fw[kChains][NB];
+      for (int h0 = 0; h0 < 2; h0 += kPair) {
+        f32x4 fa[kPair][MB], fw[kPair][NB];
 #pragma unroll
-      for (int x = 0; x < kChains; ++x) {
+        for (int x = 0; x < kPair; ++x) {
 #pragma unroll
-        for (int i = 0; i < MB; ++i) fa[x][i] = frag(st, arow + 16 * i, h0 + x);
+          for (int i = 0; i < MB; ++i) fa[x][i] = frag(st, arow + 16 * i, h0 + x);
 #pragma unroll
-        for (int j = 0; j < NB; ++j) fw[x][j] = frag(st, wrow + 16 * j, h0 + x);
+          for (int j = 0; j < NB; ++j) fw[x][j] = frag(st, wrow + 16 * j, h0 + x);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int x = 0; x < kPair; ++x)
+#pragma unroll
+            for (int i = 0; i < MB; ++i)
+#pragma unroll
+              for (int j = 0; j < NB; ++j) {
+                const f32x4 c = FIRST && e == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[h0 + x][i][j];
+                acc[h0 + x][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[x][j][e], fa[x][i][e], c, 0, 0, 0);
+              }
       }
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int x = 0; x < kChains; ++x)
-#pragma unroll
-          for (int i = 0; i < MB; ++i)
-#pragma unroll
-            for (int j = 0; j < NB; ++j)
-              acc[x][i][j] =
-                  __builtin_amdgcn_mfma_f32_16x16x4f32(fw[x][j][e], fa[x][i][e], acc[x][i][j], 0, 0, 0);
     }
+  };
+  constexpr int kSum = X3 ? 1 << 30 : kSumStages;
+  f32x4 total[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int j = 0; j < NB; ++j) total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int kb = 0; kb < nk; kb += kSum) {
+    stage(kb, std::true_type{});
+    for (int kt = kb + 1; kt < min(kb + kSum, nk); ++kt) stage(kt, std::false_type{});
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        f32x4 v = acc[0][i][j];
+        if constexpr (!X3) v += acc[1][i][j];
+        total[i][j] += v;
+      }
   }
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
-      f32x4 v = acc[0][i][j];
-      if constexpr (kChains == 2) v += acc[1][i][j];
+      const f32x4 v = total[i][j];
       const int row = m0 + wm * 16 * MB + 16 * i + lr, col = n0 + wn * 16 * NB + 16 * j + 4 * lg;
-      if constexpr (EPI == kF32QkvRope) {
-        // N is a multiple of 16 (gemm_f32_rope_ok), so a block is in or out.
-        if (col < p.N) {
-          if (p.bias) v += *reinterpret_cast<const f32x4u*>(p.bias + col);
-          v = rope16(p, row, col, v);
-          if (row < p.M) *reinterpret_cast<f32x4*>(p.C + static_cast<size_t>(row) * p.ldc + col) = v;
-        }
-      } else {
-        f32_store4<EPI, X3>(p, row, col, v, vec_c);
-      }
+      f32_out<EPI, X3>(p, row, col, v, vec_c);
     }
 }
 
-// ---- Skinny fp32 GEMM (K % 16 == 0): a 16 MB x 16 NB output tile whose K is
-// split over the workgroup's eight waves. Each wave loads its 16-wide K steps
-// straight into registers (lane (lr, lg): k = 16 s + 4 lg .. + 4 of row lr), CH
-// steps in flight at once, and the waves' sums meet in LDS in wave order. It
-// is for grids of few tiles, where one wave's walk over all of K, a load
-// latency per step, is what the launch takes.
-constexpr int kSkinnyWaves = 8;
-template <int MB, int NB, int CH, int EPI>
-__global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_f32_skinny_kernel(const GemmF32Args p, bool vec_c) {
-  __shared__ f32x4 part[kSkinnyWaves][MB * NB][64];
+// ---- The same sums for grids of few tiles: a 16x16 output tile per workgroup
+// of two waves, one for the first and one for the second halves of the stages,
+// which leave their sums in LDS for the first wave to add up. A wave's
+// operands of a K stage are 16 bytes a lane of A and of W (lane (lr, lg): k =
+// 16 h + 4 lg .. + 4 of row lr), so it keeps a ring of D stages of its own in
+// LDS, filled by direct loads and read back lane by lane, with no barrier
+// before the two sums meet: what the launch takes is the chain of dependent
+// MFMAs and one load latency. N = 320 at 66 rows: K = 320 / 640 / 1280 in 3.3 /
+// 4.4 / 6.7 us, where 32x32 tiles take 4.9 / 7.3 / 12.5. (A ring in registers
+// took 3.6 / 4.7 / 8.6, before the sums were cut: the compiler waits for every
+// load in flight at the loop's head. A wave for each sum, its operands straight
+// into registers, took 3.3 / 4.4 / 6.8 to 7.8.)
+constexpr int kPairSums = 32;  // at most: K <= 32 kSumStages kPairSums
+template <int D, int EPI>
+__global__ __launch_bounds__(128) void gemm_f32_pair_kernel(const GemmF32Args p, bool vec_c) {
+  constexpr int kStage = 2048;  // 1 KB of A, 1 KB of W
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * D * kStage];
+  __shared__ f32x4 sums[2][kPairSums][64];
+  const int lane = threadIdx.x & 63, half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int m0 = blockIdx.x * 16, n0 = blockIdx.y * 16;
+  const float* a = p.A + static_cast<size_t>(m0) * p.lda + 16 * half;
+  const float* w = p.W + static_cast<size_t>(n0) * p.ldw + 16 * half;
+  const uint32_t aoff = (static_cast<uint32_t>(min(lr, p.M - 1 - m0)) * static_cast<uint32_t>(p.lda) + 4 * lg) * 4u;
+  const uint32_t woff = (static_cast<uint32_t>(min(lr, p.N - 1 - n0)) * static_cast<uint32_t>(p.ldw) + 4 * lg) * 4u;
+  uint8_t* ring = smem + half * D * kStage;
+  const uint32_t lds = lds_byte_addr(ring);
+  auto load = [&](int kt, int slot) {
+    lds_dma16(a + 32 * kt, aoff, lds + static_cast<uint32_t>(slot * kStage));
+    lds_dma16(w + 32 * kt, woff, lds + static_cast<uint32_t>(slot * kStage + 1024));
+  };
+  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 fa, fw;
+  auto read = [&](int slot) {
+    fa = *reinterpret_cast<const f32x4*>(ring + slot * kStage + lane * 16);
+    fw = *reinterpret_cast<const f32x4*>(ring + slot * kStage + 1024 + lane * 16);
+  };
+  const int nk = p.K / 32;
+  int slot = 0, in_sum = 0, nsum = 0;
+  auto multiply = [&] {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[e], fa[e], acc, 0, 0, 0);
+    slot = slot + 1 == D ? 0 : slot + 1;
+    if (++in_sum == kSumStages) {
+      sums[half][nsum++][lane] = acc;
+      acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      in_sum = 0;
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < D; ++u)
+    if (u < nk) load(u, u);
+  // Stage kt is read into registers, its slot refilled (once the reads are
+  // back), and then multiplied.
+  for (int kt = 0; kt + D < nk; ++kt) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (D - 1)) : "memory");
+    read(slot);
+    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa), "+v"(fw)::"memory");
+    load(kt + D, slot);
+    multiply();
+  }
+  // The last min(D, nk) stages are on their way, `later` of them after this one.
+#pragma unroll
+  for (int later = D - 1; later >= 0; --later)
+    if (later < nk) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * later) : "memory");
+      read(slot);
+      multiply();
+    }
+  if (in_sum > 0) sums[half][nsum++][lane] = acc;
+  __syncthreads();
+  if (half == 1) return;
+  f32x4 total = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int x = 0; x < nsum; ++x) total += sums[0][x][lane] + sums[1][x][lane];
+  f32_out<EPI, false>(p, m0 + lr, n0 + 4 * lg, total, vec_c);
+}
+
+// ---- Narrow fp32 GEMM (N <= 48, the tied decoder; K % 16 == 0): a 16 MB x 48
+// output tile whose K is split over the workgroup's eight waves. Each wave
+// loads its 16-wide K steps straight into registers (lane (lr, lg): k = 16 s +
+// 4 lg .. + 4 of row lr), CH steps in flight at once, and the waves' sums meet
+// in LDS in wave order.
+constexpr int kNarrowBlocks = 3;
+constexpr int kNarrowWaves = 8;
+template <int MB, int CH>
+__global__ __launch_bounds__(kNarrowWaves * 64) void gemm_narrow_kernel(const GemmF32Args p, bool vec_c) {
+  constexpr int NB = kNarrowBlocks;
+  __shared__ f32x4 part[kNarrowWaves][MB * NB][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 15, lg = lane >> 4;
-  const int m0 = blockIdx.x * 16 * MB, n0 = blockIdx.y * 16 * NB;
+  const int m0 = blockIdx.x * 16 * MB;
   const float* arow[MB];
   const float* wrow[NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i) arow[i] = p.A + static_cast<size_t>(min(m0 + 16 * i + lr, p.M - 1)) * p.lda + 4 * lg;
 #pragma unroll
-  for (int j = 0; j < NB; ++j) wrow[j] = p.W + static_cast<size_t>(min(n0 + 16 * j + lr, p.N - 1)) * p.ldw + 4 * lg;
+  for (int j = 0; j < NB; ++j) wrow[j] = p.W + static_cast<size_t>(min(16 * j + lr, p.N - 1)) * p.ldw + 4 * lg;
   f32x4 acc[MB][NB];
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < NB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const int steps = p.K / 16;
-  const int s0 = steps * wave / kSkinnyWaves, s1 = steps * (wave + 1) / kSkinnyWaves;
+  const int s0 = steps * wave / kNarrowWaves, s1 = steps * (wave + 1) / kNarrowWaves;
   for (int s = s0; s < s1; s += CH) {
     f32x4 fa[CH][MB], fw[CH][NB];
 #pragma unroll
@@ -420,8 +530,8 @@ __global__ __launch_bounds__(kSkinnyWaves * 64) void gemm_f32_skinny_kernel(cons
   if (wave >= MB * NB) return;
   f32x4 v = part[0][wave][lane];
 #pragma unroll
-  for (int w = 1; w < kSkinnyWaves; ++w) v += part[w][wave][lane];
-  f32_store4<EPI, false>(p, m0 + 16 * (wave / NB) + lr, n0 + 16 * (wave % NB) + 4 * lg, v, vec_c);
+  for (int w = 1; w < kNarrowWaves; ++w) v += part[w][wave][lane];
+  f32_store4<kF32Store, false>(p, m0 + 16 * (wave / NB) + lr, 16 * (wave % NB) + 4 * lg, v, vec_c);
 }
 
 }  // namespace
@@ -454,38 +564,69 @@ hipError_t launch_f32_tile(const GemmF32Args& p, int epi, hipStream_t s) {
   ESM_F32_EPI(gemm_f32_tile_kernel, X3, MB, NB);
 }
 
-template <int MB, int NB, int CH>
-hipError_t launch_f32_skinny(const GemmF32Args& p, int epi, hipStream_t s) {
+hipError_t launch_f32_pair(const GemmF32Args& p, int epi, hipStream_t s) {
   const bool vec_c = f32_vec_c(p);
-  const dim3 grid((p.M + 16 * MB - 1) / (16 * MB), (p.N + 16 * NB - 1) / (16 * NB)), block(kSkinnyWaves * 64);
-  ESM_F32_EPI(gemm_f32_skinny_kernel, MB, NB, CH);
+  const dim3 grid((p.M + 15) / 16, (p.N + 15) / 16), block(128);
+  constexpr int kAhead = 4;  // 16 KB of LDS; 8, 12 or 16 were no faster
+  if (epi == kF32QkvRope) {
+    hipLaunchKernelGGL((gemm_f32_pair_kernel<kAhead, kF32QkvRope>), grid, block, 0, s, p, vec_c);
+    return hipGetLastError();
+  }
+  ESM_F32_EPI(gemm_f32_pair_kernel, kAhead);
 }
 
-bool f32_skinny_ok(const GemmF32Args& p) {
-  return p.K > 0 && p.K % 16 == 0 && p.lda % 4 == 0 && p.ldw % 4 == 0;
+template <int MB, int CH>
+hipError_t launch_narrow(const GemmF32Args& p, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_narrow_kernel<MB, CH>), dim3((p.M + 16 * MB - 1) / (16 * MB)), dim3(kNarrowWaves * 64), 0, s,
+                     p, f32_vec_c(p));
+  return hipGetLastError();
 }
 
-// The stage loads take 16-byte aligned rows and 32-bit lane offsets.
+constexpr uint64_t kOffsetLimit = 1ull << 32;  // bytes that 32-bit lane offsets reach
+
+// 16-byte aligned rows of A and W.
+bool f32_rows_ok(const GemmF32Args& p) {
+  return p.lda % 4 == 0 && p.ldw % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.W)) % 16 == 0;
+}
+
+// The tiled kernel's (and the pair kernel's) operands: whole K stages of
+// aligned rows, W within the stage loads' offsets. A beyond them goes in pieces
+// (f32_pieces), so which order a row is summed in does not depend on M.
 bool f32_tile_ok(const GemmF32Args& p) {
-  constexpr uint64_t kLimit = 1ull << 32;
-  return p.K > 0 && p.K % 32 == 0 && p.lda % 4 == 0 && p.ldw % 4 == 0 &&
-         (reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.W)) % 16 == 0 &&
-         static_cast<uint64_t>(p.M) * p.lda * 4 <= kLimit && static_cast<uint64_t>(p.N) * p.ldw * 4 <= kLimit;
+  return p.K > 0 && p.K % 32 == 0 && f32_rows_ok(p) && static_cast<uint64_t>(p.N) * p.ldw * 4 <= kOffsetLimit &&
+         static_cast<uint64_t>(p.lda) * 4 <= kOffsetLimit;
+}
+
+// Runs launch on pieces of rows of A that 32-bit offsets reach.
+template <class F>
+hipError_t f32_pieces(const GemmF32Args& p, F launch) {
+  const int most = static_cast<int>(std::min<uint64_t>(1 << 30, kOffsetLimit / (static_cast<uint64_t>(p.lda) * 4)));
+  for (int m0 = 0; m0 < p.M; m0 += most) {
+    GemmF32Args q = p;
+    q.A += static_cast<size_t>(m0) * p.lda;
+    q.C += static_cast<size_t>(m0) * p.ldc;
+    if (q.pos) q.pos += m0;
+    q.M = std::min(most, p.M - m0);
+    const hipError_t e = launch(q);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 // Tiles 0 .. n - 1 of {32x32, 64x64, 128x64, 128x128}: the one whose grid
-// takes the least time, (the most tiles any CU gets + 1/2) x the tile's
-// outputs x its cost per output. The costs are those of many rounds; the half
-// tile is the last round, in which a CU's few remaining workgroups leave its
-// matrix cores waiting.
-int tile_of(int M, int N, int n, const double* cost) {
+// takes the least time, (the most tiles any CU gets + the ends of its work, in
+// tiles) x the tile's outputs x its cost per output.
+template <class Ends>
+int tile_of(int M, int N, int n, const double* cost, Ends ends) {
   static constexpr int kBM[4] = {32, 64, 128, 128}, kBN[4] = {32, 64, 64, 128};
   const int cus = device_cus();
   int best = 0;
   double best_t = 0.0;
   for (int t = 0; t < n; ++t) {
     const long tiles = static_cast<long>((M + kBM[t] - 1) / kBM[t]) * ((N + kBN[t] - 1) / kBN[t]);
-    const double c = (static_cast<double>((tiles + cus - 1) / cus) + 0.5) * kBM[t] * kBN[t] * cost[t];
+    const long most = (tiles + cus - 1) / cus;
+    const double c = (static_cast<double>(most) + ends(most)) * kBM[t] * kBN[t] * cost[t];
     if (t == 0 || c < best_t) {
       best = t;
       best_t = c;
@@ -494,19 +635,30 @@ int tile_of(int M, int N, int n, const double* cost) {
   return best;
 }
 
-// fp32: 2560 x 2560 at 16,000 rows takes 1,727 / 1,529 / 1,498 us. The choice
-// follows the measured order at 1280 x 1280: 33 / 44 / 48 us at 1,000 rows, 56 /
-// 62 / 79 at 1,768, 94 / 84 / 81 at 3,000, 224 / 199 / 230 at 7,777, 457 / 393 /
-// 389 at 16,000. (64x32 and 128x128 tiles were never more than 8% faster.)
-constexpr double kF32Cost[3] = {1.17, 1.02, 1.0};
+// fp32: the first loads and the last stores of a CU's tiles take about three K
+// stages, and a CU with a single tile leaves its matrix cores waiting longer.
+// 32x32 / 64x64 / 128x64 tiles: 2560 x 2560 at 16,000 rows 1,718 / 1,535 / 1,506
+// us; 1280 x 1280 at 1,000 rows 32 / 44 / 49 us, at 1,768 53 / 62 / 80, at 3,000
+// 86 / 86 / 81, at 7,777 214 / 202 / 197, at 16,000 429 / 396 / 391. Over 20 row
+// counts of 66 .. 16,000 at nine N x K of 320 .. 3840 x 96 .. 2560 the choice is
+// 0.3% off the fastest on average, 9% at 16,000 x 320 x 320 and 8% at 16,000 x
+// 320 x 1280, where 32x32 is, and 4% at most elsewhere. (64x32 and 128x128 tiles
+// were never more than 8% faster.)
+constexpr double kF32Cost[3] = {1.14, 1.02, 1.0};
+
+int f32_tile(const GemmF32Args& p) {
+  return tile_of(p.M, p.N, 3, kF32Cost, [&](long most) { return 3.0 * 32 / p.K + (most == 1 ? 0.2 : 0.0); });
+}
 
 // Split-fp16, bound by the stage traffic: 1280 x 1280 takes 15 / 21 / 35 / 48 us
 // at 301 rows, 45 / 35 / 38 / 50 at 2,048, 148 / 103 / 91 / 110 at 7,562, - / 423
 // / 376 / 359 at 31,107; 2560 x 2560 at 7,562 rows 617 / 358 / 339 / 305.
+// The last round, in which a CU's few remaining workgroups wait for their loads,
+// counts for half a tile.
 constexpr double kX3Cost[4] = {2.2, 1.18, 1.07, 1.0};
 
 hipError_t launch_x3_tile(const GemmF32Args& p, int epi, hipStream_t s) {
-  switch (tile_of(p.M, p.N, 4, kX3Cost)) {
+  switch (tile_of(p.M, p.N, 4, kX3Cost, [](long) { return 0.5; })) {
     case 0: return launch_f32_tile<true, 1, 1>(p, epi, s);
     case 1: return launch_f32_tile<true, 2, 2>(p, epi, s);
     case 2: return launch_f32_tile<true, 4, 2>(p, epi, s);
@@ -518,65 +670,64 @@ hipError_t launch_x3_tile(const GemmF32Args& p, int epi, hipStream_t s) {
 
 hipError_t launch_gemm_narrow(const GemmF32Args& p, hipStream_t s) {
   if (p.M <= 0 || p.N <= 0) return hipSuccess;
-  if (p.N > 48 || !f32_skinny_ok(p)) return hipErrorInvalidValue;
+  if (p.N > 16 * kNarrowBlocks || p.K <= 0 || p.K % 16 != 0 || !f32_rows_ok(p)) return hipErrorInvalidValue;
   // 32 rows a workgroup halve the reads of W once there are enough of them.
-  if (p.M > 4096) return launch_f32_skinny<2, 3, 4>(p, kF32Store, s);
-  return launch_f32_skinny<1, 3, 5>(p, kF32Store, s);
+  if (p.M > 4096) return launch_narrow<2, 4>(p, s);
+  return launch_narrow<1, 5>(p, s);
 }
 
 hipError_t launch_gemm_x3(const GemmX3Args& x, int epi, hipStream_t s) {
   if (x.M <= 0 || x.N <= 0) return hipSuccess;
   if (x.K <= 0 || x.K % 32 != 0) return hipErrorInvalidValue;
-  // The stage loads' 32-bit offsets reach 2^32 bytes of A and of W: larger
-  // operands go in pieces.
-  const int most = static_cast<int>(std::min<int64_t>(1 << 30, (int64_t{1} << 32) / (int64_t{x.K} * 4)));
-  for (int n0 = 0; n0 < x.N; n0 += most)
-    for (int m0 = 0; m0 < x.M; m0 += most) {
-      GemmF32Args p;
-      // Rows of K / 32 pieces of 128 bytes: the fp32 kernel's pitches.
-      p.A = reinterpret_cast<const float*>(x.A) + static_cast<size_t>(m0) * x.K;
-      p.W = reinterpret_cast<const float*>(x.W) + static_cast<size_t>(n0) * x.K;
-      p.lda = p.ldw = p.K = x.K;
-      p.c_unscale = x.w_unscale;
-      p.bias = x.bias ? x.bias + n0 : nullptr;
-      p.C = x.C + static_cast<size_t>(m0) * x.ldc + n0;
-      p.ldc = x.ldc;
-      p.M = std::min(most, x.M - m0);
-      p.N = std::min(most, x.N - n0);
-      if (!f32_tile_ok(p)) return hipErrorInvalidValue;
-      const hipError_t e = launch_x3_tile(p, epi, s);
-      if (e != hipSuccess) return e;
-    }
+  // Larger operands than the stage loads' offsets reach go in pieces.
+  const int most = static_cast<int>(std::min<uint64_t>(1 << 30, kOffsetLimit / (static_cast<uint64_t>(x.K) * 4)));
+  for (int n0 = 0; n0 < x.N; n0 += most) {
+    GemmF32Args p;
+    // Rows of K / 32 pieces of 128 bytes: the fp32 kernel's pitches.
+    p.A = reinterpret_cast<const float*>(x.A);
+    p.W = reinterpret_cast<const float*>(x.W) + static_cast<size_t>(n0) * x.K;
+    p.lda = p.ldw = p.K = x.K;
+    p.c_unscale = x.w_unscale;
+    p.bias = x.bias ? x.bias + n0 : nullptr;
+    p.C = x.C + n0;
+    p.ldc = x.ldc;
+    p.M = x.M;
+    p.N = std::min(most, x.N - n0);
+    if (!f32_tile_ok(p)) return hipErrorInvalidValue;
+    const hipError_t e = f32_pieces(p, [&](const GemmF32Args& q) { return launch_x3_tile(q, epi, s); });
+    if (e != hipSuccess) return e;
+  }
   return hipSuccess;
 }
 
 namespace {
 
-// At most one 16x16-tile workgroup a CU and a K long enough to be worth
-// splitting: N = 320 at 66 rows takes 6.4 / 6.5 / 6.6 / 6.7 us skinny for K
-// = 320 / 480 / 960 / 1280 against 4.8 / 6.0 / 9.7 / 12.2 in 32x32 tiles; a
-// second round of workgroups (301 rows) 11.4 against 12.4 at K = 1280.
-bool f32_takes_skinny(const GemmF32Args& p) {
+// At most two 16x16 tiles a CU, whose waves then have a SIMD each. N = 320, K =
+// 320 / 1280: 4.4 / 11.2 us at 301 rows (380 tiles) against 4.9 / 12.6 in 32x32
+// tiles, 5.5 / 15.7 at 450 rows (580 tiles) against 5.0 / 12.8.
+bool f32_takes_pair(const GemmF32Args& p) {
   const long tiles16 = static_cast<long>((p.M + 15) / 16) * ((p.N + 15) / 16);
-  return f32_skinny_ok(p) && p.K >= 512 && tiles16 <= device_cus();
+  return tiles16 <= 2 * device_cus() && p.K <= 32 * kSumStages * kPairSums;
 }
 
 }  // namespace
 
 bool gemm_f32_rope_ok(const GemmF32Args& p, int head_dim) {
-  return head_dim == 16 && p.N % 16 == 0 && f32_vec_c(p) && f32_tile_ok(p) && !f32_takes_skinny(p);
+  return head_dim == 16 && p.N % 16 == 0 && f32_vec_c(p) && f32_tile_ok(p);
 }
 
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epi, hipStream_t s) {
   if (p.M <= 0 || p.N <= 0) return hipSuccess;
   if (epi == kF32QkvRope && !gemm_f32_rope_ok(p, 16)) return hipErrorInvalidValue;
-  if (f32_takes_skinny(p)) return launch_f32_skinny<1, 1, 10>(p, epi, s);
   if (f32_tile_ok(p)) {
-    switch (tile_of(p.M, p.N, 3, kF32Cost)) {
-      case 0: return launch_f32_tile<false, 1, 1>(p, epi, s);
-      case 1: return launch_f32_tile<false, 2, 2>(p, epi, s);
-      default: return launch_f32_tile<false, 4, 2>(p, epi, s);
-    }
+    if (f32_takes_pair(p)) return launch_f32_pair(p, epi, s);
+    return f32_pieces(p, [&](const GemmF32Args& q) {
+      switch (f32_tile(q)) {
+        case 0: return launch_f32_tile<false, 1, 1>(q, epi, s);
+        case 1: return launch_f32_tile<false, 2, 2>(q, epi, s);
+        default: return launch_f32_tile<false, 4, 2>(q, epi, s);
+      }
+    });
   }
   const int tiles = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
   const dim3 grid(tiles), block(kThreads);

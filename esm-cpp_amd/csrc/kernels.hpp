@@ -147,11 +147,14 @@ struct GemmF32Args {
   const float* rope_sin = nullptr;
   float q_scale = 1.0f;
 };
+// The order of a row's sum depends on N, K and the operands' alignment, not on M.
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epilogue, hipStream_t s);
-// Whether the launch can take kF32QkvRope: 16-wide heads on the tiled kernel.
+// Whether the launch can take kF32QkvRope: 16-wide heads, the tiled kernel's
+// operands and whole 16-byte pieces of C.
 bool gemm_f32_rope_ok(const GemmF32Args& p, int head_dim);
-// C = A W^T + bias for N <= 48 (the tied vocabulary decoder), fp32 MFMA, one
-// wave per 16 rows; K % 16 == 0, lda and ldw multiples of 4.
+// C = A W^T + bias for N <= 48 (the tied vocabulary decoder), fp32 MFMA, K in
+// eight ranges; K % 16 == 0, 16-byte aligned rows of A and W. The same order of
+// a row's sum at every M.
 hipError_t launch_gemm_narrow(const GemmF32Args& p, hipStream_t s);
 
 // FP32-accurate GEMM on fp16 MFMA ("split-fp16"): every operand x is carried

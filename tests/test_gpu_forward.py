@@ -349,6 +349,32 @@ def test_config5_full_workload(dev, oracle):
     assert c >= 0.9999, c
 
 
+@pytest.mark.parametrize("which", ["8m fp32", "650m fp32 lm dense", "650m split lm dense"])
+def test_logits_do_not_depend_on_the_batch(dev, w8m, w650_small, which):
+    """The logits of about 3,200 tokens have the same bits in one, two and three
+    groups, and a sequence the same bits alone, so that every GEMM and attention
+    choice from 22 to 3,200 rows is met: the fp32 linears above all, whose sums
+    depend on their order."""
+    fp32 = which == "8m fp32"
+    m = eg.Model(dev, w8m if fp32 else w650_small, int8=not fp32, act_mode=eg.ACT_PER_TOKEN)
+    if which == "650m fp32 lm dense":
+        m.set_lm_dense_split(False)
+    lengths = [66, 22, 301, 176] + [int(n) for n in np.random.default_rng(9).integers(22, 203, size=24)]
+    batch = syn.batch_from_lengths(lengths, seed=11)
+    m.set_parts(1)
+    want = m.forward_packed(batch.ids, batch.cu)
+    for parts in (2, 3):
+        m.set_parts(parts)
+        got = m.forward_packed(batch.ids, batch.cu)
+        assert m.staged_parts() == parts
+        np.testing.assert_array_equal(got.view(np.uint32), want.view(np.uint32), err_msg=f"{parts} groups")
+    for i in range(5):
+        s = slice(int(batch.cu[i]), int(batch.cu[i + 1]))
+        got = m.forward_packed(batch.ids[s], np.array([0, lengths[i]], np.int32))
+        np.testing.assert_array_equal(got.view(np.uint32), want[s].view(np.uint32), err_msg=f"sequence {i} alone")
+    m.free()
+
+
 @pytest.mark.parametrize("parts", [2, 3, 4])
 def test_parts_match_single_stream(dev, w650_small, small_batch, parts):
     """Concurrent sequence groups on separate streams: every row depends only

@@ -135,6 +135,55 @@ def test_linear_f32_tile_edges(dev, M, N, K, shift):
     assert np.all(np.abs(got - want) <= 2.0**-24 * K * (np.abs(A64) @ np.abs(W64).T + 1))
 
 
+def _rows_do_not_depend_on_m(dev, N, K, shift, rows):
+    r = rng(N + K)
+    A = r.uniform(-1, 1, size=(max(rows), K)).astype(np.float32)
+    W = r.uniform(-1, 1, size=(N, K)).astype(np.float32)
+    b = r.uniform(-1, 1, size=N).astype(np.float32)
+    held = [dev.array(np.concatenate([np.zeros(shift, np.float32), x.ravel()])) for x in (A, W, b)]
+    at = [type(h.ptr)(h.ptr.value + 4 * shift) for h in held]
+    want = None
+    for M in sorted(rows, reverse=True):
+        out = dev.empty((M, N), np.float32)
+        dev._check(dev.lib.esm_gfx950_linear_f32(dev.ctx, at[0], at[1], at[2], out.ptr, M, N, K))
+        got = out.numpy()
+        want = got if want is None else want
+        np.testing.assert_array_equal(got.view(np.uint32), want[:M].view(np.uint32), err_msg=f"{M} rows")
+    A64, W64 = A[:64].astype(np.float64), W.astype(np.float64)
+    assert np.all(np.abs(want[:64] - (A64 @ W64.T + b)) <= 2.0**-24 * K * (np.abs(A64) @ np.abs(W64).T + 1))
+
+
+@pytest.mark.parametrize("N,K,shift", [(320, 320, 0), (960, 320, 0), (320, 1280, 0), (1280, 1280, 0), (1283, 96, 0),
+                                       (47, 32, 0), (320, 1280, 1), (320, 528, 0)])
+def test_linear_f32_rows_do_not_depend_on_their_number(dev, N, K, shift):
+    """A row of linear_f32 has the same bits whatever the row count: across
+    the two-wave 16x16 tiles, the 32x32 and the 64x64 ones, and in the general
+    kernel (operands off their 16-byte boundary, K % 32 != 0)."""
+    _rows_do_not_depend_on_m(dev, N, K, shift, [1, 17, 66, 176, 301, 1461, 3001, 8003])
+
+
+def test_linear_f32_rows_do_not_depend_on_their_number_tall_tile(dev):
+    _rows_do_not_depend_on_m(dev, 2557, 2560, 0, [17, 301, 2048, 10301])
+
+
+def test_linear_f32_past_32_bit_offsets(dev):
+    """Rows past 2^32 bytes of A: the same bits as near its start."""
+    K, N, block, M = 1024, 16, 4096, (1 << 20) + 33
+    r = rng(5)
+    A = dev.empty((M, K), np.float32)
+    src = dev.array(r.uniform(-1, 1, size=(block, K)).astype(np.float32))
+    for m0 in range(0, M, block):
+        n = min(block, M - m0)
+        dev._check(dev.lib.esm_gfx950_memcpy_d2d(dev.ctx, type(A.ptr)(A.ptr.value + m0 * K * 4), src.ptr, n * K * 4))
+    W, b = dev.array(r.uniform(-1, 1, size=(N, K)).astype(np.float32)), dev.array(np.ones(N, np.float32))
+    want, out = dev.empty((block, N), np.float32), dev.empty((M, N), np.float32)
+    dev.linear_f32(src, W, b, want, block, N, K)
+    dev.linear_f32(A, W, b, out, M, N, K)
+    got, want = out.numpy(), want.numpy()
+    for m0 in range(0, M, block):
+        np.testing.assert_array_equal(got[m0:m0 + block], want[:min(block, M - m0)], err_msg=f"row {m0}")
+
+
 def test_linear_f32_known_answer(dev):
     """Reference tests/cpp/test_kernels.cpp:88-111."""
     A = np.array([[1, 2, 3], [4, 5, 6]], np.float32)
