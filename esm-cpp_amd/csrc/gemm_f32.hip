@@ -13,7 +13,8 @@
 //   - gemm_f32_pair_kernel: the same operands and the same sums bit for bit, for
 //     grids too small for that one: two waves to a 16x16 tile;
 //   - gemm_f32_kernel: any other shape (128x128 tiles through registers);
-//   - gemm_narrow_kernel: N <= 48, eight waves split K.
+//   - gemm_narrow_kernel and gemm_narrow_rows_kernel: N <= 48, the sums of eight
+//     ranges of K, by eight waves or one after the other.
 // Which order a row is summed in is chosen by N, K and the alignment alone,
 // never by M: a sequence's logits do not depend on what it is batched with.
 //
@@ -534,6 +535,91 @@ __global__ __launch_bounds__(kNarrowWaves * 64) void gemm_narrow_kernel(const Ge
   f32_store4<kF32Store, false>(p, m0 + 16 * (wave / NB) + lr, 16 * (wave % NB) + 4 * lg, v, vec_c);
 }
 
+// The same sums for many rows (K % 32 == 0): with enough of them to fill the chip
+// K need not be split, and eight waves that each read 64 bytes of a row at a
+// time only cost. Four waves of 16 rows share stages of 32 k (A's rows and the 48
+// of W) moved and laid out as in the tiled kernel; a wave walks the eight ranges
+// of K one after the other and adds each to its total. 31,107 x 33 x 1280: 72 ->
+// 39 us, 4.1 TB/s of A; its MFMAs alone are 26. (32 rows a wave leave a CU one
+// workgroup and nothing to cover its barriers: 46 us.)
+constexpr int kNarrowRows = 64;
+__global__ __launch_bounds__(256, 2) void gemm_narrow_rows_kernel(const GemmF32Args p, bool vec_c) {
+  constexpr int NB = kNarrowBlocks, BM = kNarrowRows;
+  constexpr int kBlocks = BM / 8 + 2 * NB;
+  constexpr int kPer = (kBlocks + 3) / 4;  // the last ones move W's last row again
+  constexpr int kStage = 4 * kPer * 1024, kNStage = 3;
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kNStage * kStage];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lr = lane & 15, lg = lane >> 4;
+  const int m0 = blockIdx.x * BM;
+  const float* a = p.A + static_cast<size_t>(m0) * p.lda;
+  uint32_t goff[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int b = wave * kPer + i;
+    const int r = lane >> 3, c = (lane & 7) ^ r;
+    const bool is_a = b < BM / 8;
+    const int row = is_a ? min(b * 8 + r, p.M - 1 - m0) : min((b - BM / 8) * 8 + r, p.N - 1);
+    goff[i] = (static_cast<uint32_t>(row) * static_cast<uint32_t>(is_a ? p.lda : p.ldw) + c * 4) * 4u;
+  }
+  const uint32_t lds0 = lds_byte_addr(smem);
+  auto load_stage = [&](int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      lds_dma16((wave * kPer + i < BM / 8 ? a : p.W) + kt * 32, goff[i],
+                lds0 + static_cast<uint32_t>(buf * kStage + (wave * kPer + i) * 1024));
+  };
+  const int nk = p.K / 32;
+#pragma unroll
+  for (int st = 0; st < kNStage - 1; ++st)
+    if (st < nk) load_stage(st, st);
+  const int arow = wave * 16 + lr, wrow = BM + lr;
+  auto frag = [&](const uint8_t* st, int R, int h) {
+    return *reinterpret_cast<const f32x4*>(st + (R >> 3) * 1024 + (R & 7) * 128 + (((4 * h + lg) ^ (R & 7)) << 4));
+  };
+  f32x4 acc[NB], total[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) acc[j] = total[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int steps = 2 * nk;
+  int range = 0, end = steps / kNarrowWaves, buf = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    // As in the tiled kernel: stage kt has landed, and the buffer of stage kt - 1
+    // receives stage kt + kNStage - 1.
+    if (kt + 1 < nk)
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(kPer) : "memory");
+    else
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt + kNStage - 1 < nk) load_stage(kt + kNStage - 1, buf == 0 ? kNStage - 1 : buf - 1);
+    const uint8_t* st = smem + buf * kStage;
+    buf = buf + 1 == kNStage ? 0 : buf + 1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // The ranges that end before this step (with K < 128 some are empty: zero).
+      while (2 * kt + h == end) {
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+          total[j] = range == 0 ? acc[j] : total[j] + acc[j];
+          acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        ++range;
+        end = steps * (range + 1) / kNarrowWaves;
+      }
+      const f32x4 fa = frag(st, arow, h);
+      f32x4 fw[NB];
+#pragma unroll
+      for (int j = 0; j < NB; ++j) fw[j] = frag(st, wrow + 16 * j, h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[j][e], fa[e], acc[j], 0, 0, 0);
+    }
+  }
+  // The eighth range ends with K.
+#pragma unroll
+  for (int j = 0; j < NB; ++j)
+    f32_store4<kF32Store, false>(p, m0 + arow, 16 * j + 4 * lg, total[j] + acc[j], vec_c);
+}
+
 }  // namespace
 
 namespace {
@@ -579,6 +665,12 @@ template <int MB, int CH>
 hipError_t launch_narrow(const GemmF32Args& p, hipStream_t s) {
   hipLaunchKernelGGL((gemm_narrow_kernel<MB, CH>), dim3((p.M + 16 * MB - 1) / (16 * MB)), dim3(kNarrowWaves * 64), 0, s,
                      p, f32_vec_c(p));
+  return hipGetLastError();
+}
+
+hipError_t launch_narrow_rows(const GemmF32Args& p, hipStream_t s) {
+  hipLaunchKernelGGL(gemm_narrow_rows_kernel, dim3((p.M + kNarrowRows - 1) / kNarrowRows), dim3(256), 0, s, p,
+                     f32_vec_c(p));
   return hipGetLastError();
 }
 
@@ -671,9 +763,15 @@ hipError_t launch_x3_tile(const GemmF32Args& p, int epi, hipStream_t s) {
 hipError_t launch_gemm_narrow(const GemmF32Args& p, hipStream_t s) {
   if (p.M <= 0 || p.N <= 0) return hipSuccess;
   if (p.N > 16 * kNarrowBlocks || p.K <= 0 || p.K % 16 != 0 || !f32_rows_ok(p)) return hipErrorInvalidValue;
-  // 32 rows a workgroup halve the reads of W once there are enough of them.
-  if (p.M > 4096) return launch_narrow<2, 4>(p, s);
-  return launch_narrow<1, 5>(p, s);
+  // 16 rows a workgroup while there is one for every CU, then 32, and past one of
+  // those for every CU no K split. N = 33, K = 1280 with 16 / 32 / no split: 11.4
+  // / 18.3 / 25.8 us at 3,000 rows, 21.0 / 19.5 / 26.0 at 6,400, 30.9 / 36.7 / 26.5
+  // at 10,000, 81.0 / 71.9 / 38.6 at 31,107; K = 320 6.3 / 7.1 / 9.3, 9.9 / 7.3 /
+  // 9.4, 13.8 / 12.1 / 9.7 and 33.4 / 22.8 / 14.1.
+  const int cus = device_cus();
+  if (p.M <= 16 * cus) return launch_narrow<1, 5>(p, s);
+  if (p.M <= 32 * cus || p.K % 32 != 0) return launch_narrow<2, 4>(p, s);
+  return launch_narrow_rows(p, s);
 }
 
 hipError_t launch_gemm_x3(const GemmX3Args& x, int epi, hipStream_t s) {

@@ -375,6 +375,26 @@ def test_logits_do_not_depend_on_the_batch(dev, w8m, w650_small, which):
     m.free()
 
 
+@pytest.mark.parametrize("which", ["8m", "650m"])
+def test_decoder_rows_do_not_depend_on_the_batch(dev, w8m, w650_small, which):
+    """The decoder's three kernels (up to 16 rows a CU, up to 32, and beyond:
+    about 9,000 tokens in one group) sum a row in the same order: the logits of
+    a batch, of its first half and of single sequences have the same bits. K is
+    320 (ranges of K that end inside a stage) and 1280."""
+    w = w8m if which == "8m" else w650_small
+    m = eg.Model(dev, w, int8=which != "8m", act_mode=eg.ACT_PER_TOKEN)
+    m.set_parts(1)
+    lengths = [66, 22] + [int(n) for n in np.random.default_rng(3).integers(100, 300, size=45)]
+    batch = syn.batch_from_lengths(lengths, seed=12)
+    assert 32 * 256 < batch.total_tokens and batch.total_tokens % 64
+    want = m.forward_packed(batch.ids, batch.cu)
+    for b0, b1 in ((0, 25), (0, 1), (1, 2), (46, 47)):
+        s = slice(int(batch.cu[b0]), int(batch.cu[b1]))
+        got = m.forward_packed(batch.ids[s], (batch.cu[b0:b1 + 1] - batch.cu[b0]).astype(np.int32))
+        np.testing.assert_array_equal(got.view(np.uint32), want[s].view(np.uint32), err_msg=f"sequences {b0} .. {b1}")
+    m.free()
+
+
 @pytest.mark.parametrize("parts", [2, 3, 4])
 def test_parts_match_single_stream(dev, w650_small, small_batch, parts):
     """Concurrent sequence groups on separate streams: every row depends only
