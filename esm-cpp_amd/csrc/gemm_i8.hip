@@ -1236,10 +1236,10 @@ int device_cus() {
 
 namespace {
 
-// The pipelined kernel's tiles. 64 .. 320: rows of a tile 256 columns wide,
-// but 64 is 64x64; kTile128x128 is 128x128 and kTile64x256 64x256.
+// The pipelined kernel's tiles. 64 .. 320: rows of a tile 256 columns wide;
+// 1000 + n: n x n.
+constexpr int kTile64x64 = 1064;
 constexpr int kTile128x128 = 1128;
-constexpr int kTile64x256 = 1064;
 
 // A launch's estimated time in microseconds: whole rounds of workgroups over
 // the CUs at t = fixed + per_stage * stages each, and a last, partly filled
@@ -1256,13 +1256,13 @@ constexpr TileCost kTileCosts[] = {
     // 64x64: two share a CU; alone a workgroup takes 3.8 + 0.24 a stage. At
     // 301 rows 6.2 us (N = K = 1280), 13.1 (K = 5120), where the 64x256 tile
     // takes 8.2 and 21.9.
-    {64, 64, 64, 2, 3.0, 0.42, 0.72},
+    {kTile64x64, 64, 64, 2, 3.0, 0.42, 0.72},
     // 64x256 and 128x128: the same MFMAs a workgroup. 128x128 loads 32 KB a
     // stage instead of 40 and is faster over many stages: 21.1 against 22.8 us
     // at 2,048 rows, N = 1280, K = 5120. 64x256 has the shorter epilogue and
     // eight waves to fill the pipeline: 8.1 against 9.3 us at 500 rows,
     // N = 5120, K = 1280, and 12.2 against 13.3 at 850 rows, N = K = 2560.
-    {kTile64x256, 64, 256, 1, 3.0, 0.445, 1.0},
+    {64, 64, 256, 1, 3.0, 0.445, 1.0},
     {kTile128x128, 128, 128, 1, 3.6, 0.42, 1.0},
     {128, 128, 256, 1, 4.0, 0.95, 0.75},
     {192, 192, 256, 1, 6.0, 1.28, 0.72},
@@ -1367,8 +1367,8 @@ namespace {
 
 hipError_t launch_v3_rows(const GemmI8Args& p, int epi, int rows, hipStream_t s) {
   switch (rows) {
-    case 64: return launch_v3_tile<1, 1>(p, epi, s);
-    case kTile64x256: return launch_v3_tile<1, 4>(p, epi, s);
+    case kTile64x64: return launch_v3_tile<1, 1>(p, epi, s);
+    case 64: return launch_v3_tile<1>(p, epi, s);
     case kTile128x128: return launch_v3_tile<2, 2>(p, epi, s);
     case 192: return launch_v3_tile<3>(p, epi, s);
     case 128: return launch_v3_tile<2>(p, epi, s);
@@ -1440,7 +1440,9 @@ hipError_t launch_gemm_i8_partials(const GemmI8Args& p, int splits, int rows, hi
 }
 
 bool set_gemm_tile_rows(int rows) {
-  if (rows != 0 && rows != 64 && rows != 128 && rows != 256 && rows != 320) return false;
+  if (rows != 0 && std::none_of(std::begin(kTileCosts), std::end(kTileCosts),
+                                [&](const TileCost& c) { return c.code == rows; }))
+    return false;
   g_tile_rows.store(rows, std::memory_order_relaxed);
   return true;
 }

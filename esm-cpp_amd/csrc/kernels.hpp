@@ -94,13 +94,13 @@ hipError_t launch_gemm_i8(const GemmI8Args& p, int epilogue, hipStream_t s);
 bool gemm_i8_pipelined_ok(const GemmI8Args& p);
 // variant 1: general kernel; 2: pipelined kernel (fails on shapes it cannot take).
 hipError_t launch_gemm_i8_variant(const GemmI8Args& p, int epilogue, int variant, hipStream_t s);
-// Row height of the pipelined kernel's tile for every later launch in the
-// process: 64 (64x64), 128, 256, 320 (256 columns wide), or 0 to pick per
-// launch (gemm_i8_tile_rows). False for other values.
+// The pipelined kernel's tile for every later launch in the process: 64, 128,
+// 192, 256 or 320 rows of 256 columns, 1064 (64x64), 1128 (128x128), or 0 to pick
+// per launch (gemm_i8_tile_rows). False for other values.
 bool set_gemm_tile_rows(int rows);
 // The pipelined kernel's tile for an M x N x K launch with epilogue epi on
 // `cus` CUs (0: the current device's): the one with the least estimated time
-// (64x64, 128x128, or 128, 192, 256 or 320 rows by 256 columns), as the code
+// (320 rows only for some epilogues), as a code of set_gemm_tile_rows, which
 // launch_gemm_i8_partials takes.
 int gemm_i8_tile_rows(int M, int N, int K, int epi, int cus);
 // Compute units of the current device (queried once per device; 256 if the

@@ -162,7 +162,8 @@ def _ptr(a: np.ndarray) -> C.c_void_p:
 
 
 def set_gemm_tile_rows(rows: int):
-    """INT8 GEMM tile height for later launches: 64, 128, 256, 320 or 0 (automatic)."""
+    """INT8 GEMM tile for later launches: 64, 128, 192, 256 or 320 rows of 256
+    columns, 1064 (64x64), 1128 (128x128) or 0 (automatic)."""
     rc = load_library().esm_gfx950_set_gemm_tile_rows(int(rows))
     if rc != OK:
         raise Gfx950Error(rc, f"set_gemm_tile_rows({rows})")

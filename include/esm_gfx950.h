@@ -146,12 +146,12 @@ int esm_gfx950_weight_free(esm_gfx950_ctx* ctx, esm_gfx950_weight* w);
 int esm_gfx950_gemm_i8_i32(esm_gfx950_ctx* ctx, const int8_t* A, int lda, const esm_gfx950_weight* W,
                            int M, int32_t* C);
 
-/* Row height of the INT8 GEMM's workgroup tile for every later launch in the
- * process: 64 (64 columns wide), 128, 256, 320 (256 wide), or 0 (default) to
- * pick per launch by an estimate of the grid's time, also among 64x256,
- * 128x128 and 192x256 tiles (320 only for the plain dequant, int32 and
- * split-word outputs). Results do not depend on it; it exists for tuning
- * and tests. No reference counterpart. INVALID_ARGUMENT for other values. */
+/* The INT8 GEMM's workgroup tile for every later launch in the process: 64,
+ * 128, 192, 256 or 320 rows of 256 columns, 1064 (64x64), 1128 (128x128), or 0
+ * (default) to pick one per launch by an estimate of the grid's time (320 rows
+ * only for the plain dequant, residual, int32, split-word, 24-bit and per-tensor
+ * GELU outputs). Results do not depend on it; it exists for tuning and tests. No
+ * reference counterpart. INVALID_ARGUMENT for other values. */
 int esm_gfx950_set_gemm_tile_rows(int rows);
 
 /* K splits of the model's out-proj and fc2 INT8 GEMMs for every later launch

@@ -121,20 +121,32 @@ def test_lm_dense_split_tiles(dev, T):
     assert np.abs(split - f32).max() <= 1e-5 * np.abs(f32).max()
 
 
-@pytest.mark.parametrize("per_token", [False, True])
-def test_gemm_tile_rows_do_not_change_logits(dev, w650_small, small_batch, per_token):
-    """The INT8 GEMM's 64-, 128-, 256- and 320-row tiles (and the automatic
-    choice) give bit-identical logits: the same int32 sums and the same
-    dequant expressions, only the workgroup tiling differs."""
-    mode = eg.ACT_PER_TOKEN if per_token else eg.ACT_PER_TENSOR
-    m = eg.Model(dev, w650_small, int8=True, act_mode=mode)
+@pytest.mark.parametrize("mode,attn", [
+    (eg.ACT_PER_TENSOR, eg.ATTN_MODE_F16X3), (eg.ACT_PER_TOKEN, eg.ATTN_MODE_F16X3),
+    (eg.ACT_PER_TOKEN, eg.ATTN_MODE_FP32), (eg.ACT_PER_TOKEN, eg.ATTN_MODE_FP16),
+    (eg.ACT_PER_TOKEN, eg.ATTN_MODE_BF16), ("x86", eg.ATTN_MODE_F16X3),
+])
+def test_gemm_tile_rows_do_not_change_logits(dev, w650_small, small_batch, mode, attn):
+    """Every tile of the INT8 GEMM (and the automatic choice) gives
+    bit-identical logits, with split K too: the same int32 sums and the same
+    dequant expressions (each QKV form, residual, 24-bit, the per-tensor and x86
+    GELUs), only the workgroup tiling differs. 740 rows: ragged for every tile."""
+    m = eg.Model(dev, w650_small, int8=True, act_mode=eg.ACT_PER_TENSOR if mode == "x86" else mode,
+                 attention_mode=attn)
+    if mode == "x86":
+        m.set_numerics(eg.NUMERICS_X86_AVX512)
+    # 320 rows are never picked for the other QKV forms and the x86 GELU.
+    tall = [320] if mode != "x86" and attn == eg.ATTN_MODE_F16X3 else []
     outs = []
     try:
-        for rows in (256, 320, 64, 128, 0):
+        for rows in [256, 192, 64, 128, 1064, 1128, 0] + tall:
             eg.set_gemm_tile_rows(rows)
-            outs.append(m.forward_packed(small_batch.ids, small_batch.cu))
+            for splits in (0, 3):
+                eg.set_gemm_split_k(splits)
+                outs.append(m.forward_packed(small_batch.ids, small_batch.cu))
     finally:
         eg.set_gemm_tile_rows(0)
+        eg.set_gemm_split_k(0)
         m.free()
     for o in outs[1:]:
         assert np.array_equal(outs[0], o)

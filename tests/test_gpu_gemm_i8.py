@@ -14,9 +14,12 @@ pytestmark = pytest.mark.gpu
 import esm_gfx950 as eg
 
 
-@pytest.fixture(params=[0, 64, 128, 256, 320], ids=["rows-auto", "rows-64", "rows-128", "rows-256", "rows-320"])
+TILES = [64, 128, 192, 256, 320, 1064, 1128]  # every tile of the pipelined kernel
+
+
+@pytest.fixture(params=[0] + TILES, ids=lambda t: f"rows-{t or 'auto'}")
 def tile_rows(request):
-    """INT8 GEMM tile height (0: the per-launch choice); reset afterwards."""
+    """INT8 GEMM tile (0: the per-launch choice); reset afterwards."""
     eg.set_gemm_tile_rows(request.param)
     yield request.param
     eg.set_gemm_tile_rows(0)
@@ -153,8 +156,9 @@ def test_linear_int8_facade(dev, oracle, tile_rows, mode, M, N, K):
 
 
 def test_tile_rows_rejects_other_heights():
-    with pytest.raises(eg.Gfx950Error):
-        eg.set_gemm_tile_rows(300)
+    for bad in (300, 1, -64, 1192, 1000):
+        with pytest.raises(eg.Gfx950Error):
+            eg.set_gemm_tile_rows(bad)
 
 
 def test_linear_int8_zero_sizes(dev):
@@ -344,6 +348,32 @@ def test_linear_i8_gelu_quant_r24(dev, oracle, M, N, K, ldq):
     assert np.all(got[:, N:] == 0)
 
 
+@pytest.mark.parametrize("tile", [t for t in TILES if t != 256])
+def test_linear_i8_gelu_quant_r24_does_not_depend_on_the_tile(dev, tile):
+    """The 24-bit planes, codes and scales of every tile, at an odd row count
+    and an N that ends inside the wide tiles, equal the 256-row tile's bits (a
+    NaN row scale and bias among them)."""
+    M, N, K = 333, 1216, 256
+    r = rng(tile)
+    w = dev.weight_i8(_i8(r, (N, K)), r.uniform(0.005, 0.05, size=N).astype(np.float32))
+    a_s, bias = r.uniform(0.005, 0.05, size=M).astype(np.float32), r.standard_normal(N).astype(np.float32)
+    a_s[11], bias[1000] = np.nan, np.nan
+    dA, da, db = dev.array(_i8(r, (M, K))), dev.array(a_s), dev.array(bias)
+    outs = []
+    for t in (256, tile):
+        dh, dl = dev.empty((M, N), np.uint16), dev.empty((M + 1, N), np.uint8)
+        dq, ds = dev.array(np.full((M, N), 99, np.int8)), dev.empty((M,), np.float32)
+        eg.set_gemm_tile_rows(t)
+        try:
+            dev.linear_i8_gelu_quant_r24(dA, K, da, w, db, M, dh, dl, dq, N, ds)
+        finally:
+            eg.set_gemm_tile_rows(0)
+        outs.append((_planes_to_f32(dh.numpy(), dl.numpy()).view(np.uint32), dq.numpy(), ds.numpy().view(np.uint32)))
+    w.free()
+    for x, y in zip(*outs):
+        assert np.array_equal(x, y)
+
+
 def test_linear_i8_gelu_quant_r24_rejects_bad_shapes(dev):
     r = rng(5)
     w = dev.weight_i8(_i8(r, (96, 256)), np.ones(96, np.float32))  # N % 64 != 0
@@ -369,7 +399,8 @@ def test_linear_i8_gelu_quant_r24_rejects_bad_shapes(dev):
     (9001, 5121, 384),
 ])
 def test_automatic_tile_edges(dev, M, N, K):
-    """The tile that a launch picks by itself, at ragged edges and few K
+    """Every tile, and the one that the launch picks by itself (the comments:
+    which one that is, at the time of writing), at ragged edges and few K
     stages: the dequantised output equals the 256-row tile's bit for bit, and
     the edge rows equal the closed form fma(acc, a_scale * w_scale, bias)."""
     r = rng(M + N + K)
@@ -381,16 +412,21 @@ def test_automatic_tile_edges(dev, M, N, K):
     w = dev.weight_i8(W, s)
     dA, ds, db = dev.array(A), dev.array(a_s), dev.array(b)
     outs = []
-    for rows in (0, 256):
+    for rows in [256, 0] + TILES:
         eg.set_gemm_tile_rows(rows)
         try:
             out = dev.array(np.full((M, N), np.nan, np.float32))
             dev.linear_i8_q(dA, K, ds, w, db, out, M)
-            outs.append(out.numpy())
+            got = [out.numpy()]
+            if rows != 320:  # never picked for the erf GELU
+                dev.linear_i8_q(dA, K, ds, w, db, out, M, gelu=True)
+                got.append(out.numpy())
         finally:
             eg.set_gemm_tile_rows(0)
+        outs = outs or got
+        for x, y in zip(outs, got):
+            assert np.array_equal(x, y), rows
     w.free()
-    assert np.array_equal(outs[0], outs[1])
     for m in sorted({0, M // 2, max(0, M - 2), M - 1}):
         acc = (W.astype(np.int64) @ A[m].astype(np.int64)).astype(np.float32)  # |acc| < 2^24: exact
         want = acc.astype(np.float64) * (a_s[m] * s).astype(np.float64) + b
