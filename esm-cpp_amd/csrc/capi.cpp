@@ -696,7 +696,8 @@ extern "C" int esm_gfx950_attention_work_items(const int32_t* cu_seqlens, int ba
   const int T = cu_seqlens[batch_size] - cu_seqlens[0];
   std::vector<AttnWork> work;
   try {
-    build_work(cu_seqlens, batch_size, num_heads, mfma ? kAttnMfmaQTile : kAttnF32QTile, &work, mfma != 0);
+    build_work(cu_seqlens, batch_size, num_heads,
+               mfma == 0 ? kAttnF32QTile : mfma == 2 ? kAttnX3SmallQTile : kAttnMfmaQTile, &work, mfma != 0);
   } catch (const std::exception&) {
     return ESM_GFX950_INTERNAL;
   }

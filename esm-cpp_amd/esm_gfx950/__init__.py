@@ -188,9 +188,10 @@ def rope_build_tables(seq_len: int, head_dim: int):
     return cos[:seq_len], sin[:seq_len]
 
 
-def attention_work_items(cu: np.ndarray, num_heads: int, mfma: bool = True):
-    """(items, capacity): the attention work items a batch produces and the
-    number the model's per-batch metadata reserves (host only)."""
+def attention_work_items(cu: np.ndarray, num_heads: int, mfma: int = True):
+    """(items, capacity): the attention work items a batch produces (mfma 2: in
+    64-query tiles) and the number the model's per-batch metadata reserves
+    (host only)."""
     lib = load_library()
     cu = np.ascontiguousarray(cu, np.int32)
     items, cap = C.c_size_t(), C.c_size_t()

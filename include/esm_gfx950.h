@@ -248,9 +248,11 @@ int esm_gfx950_scale(esm_gfx950_ctx* ctx, float* x, size_t n, float scale);
 int esm_gfx950_rope_build_tables(int seq_len, int head_dim, float* cos_out, float* sin_out);
 /* Host only, no counterpart in the reference (whose AttentionVarlen
  * parallelises over (sequence, head) with no work list): the number of
- * attention work items a batch with these cu_seqlens produces (mfma != 0:
- * the MFMA kernels' per-XCD queues of 128-query tiles; 0: the fp32 kernel's
- * list) and the number the model's per-batch metadata region reserves for
+ * attention work items a batch with these cu_seqlens produces (mfma 0: the
+ * fp32 kernel's list of 64-query tiles; 2: the split-fp16 kernel's per-XCD
+ * queues of 64-query tiles, which batches of few queries take; any other
+ * value: the MFMA kernels' per-XCD queues of 128-query tiles) and the number
+ * the model's per-batch metadata region reserves for
  * them (items <= capacity for every valid batch). */
 int esm_gfx950_attention_work_items(const int32_t* cu_seqlens, int batch_size, int num_heads, int mfma,
                                     size_t* items, size_t* capacity);

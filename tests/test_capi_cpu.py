@@ -61,7 +61,7 @@ def test_attention_work_list_fits_its_metadata_region():
     for lengths in cases:
         cu = cu_from_lengths(lengths)
         for H in (1, 2, 3, 4, 5, 20, 40):
-            for mfma in (True, False):
+            for mfma in (True, False, 2):
                 items, cap = eg.attention_work_items(cu, H, mfma)
                 assert items <= cap, (lengths, H, mfma, items, cap)
     # The case the bound was derived for: d = 128, H = 2, one 1024-token
