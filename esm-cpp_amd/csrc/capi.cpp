@@ -651,6 +651,12 @@ extern "C" int esm_gfx950_linear_f32(esm_gfx950_ctx* ctx, const float* A, const 
   return ESM_GFX950_OK;
 }
 
+extern "C" int esm_gfx950_linear_f32_tile(int M, int N, int K, int* rows, int* cols) {
+  if (!rows || !cols) return ESM_GFX950_INVALID_ARGUMENT;
+  gemm_f32_tile(M, N, K, rows, cols);
+  return ESM_GFX950_OK;
+}
+
 extern "C" int esm_gfx950_layernorm(esm_gfx950_ctx* ctx, const float* x, const float* gamma,
                                     const float* beta, float eps, float* out, int num_rows, int d) {
   if (!ctx) return ESM_GFX950_INVALID_ARGUMENT;

@@ -709,16 +709,16 @@ hipError_t f32_pieces(const GemmF32Args& p, F launch) {
 // Tiles 0 .. n - 1 of {32x32, 64x64, 128x64, 128x128}: the one whose grid
 // takes the least time, (the most tiles any CU gets + the ends of its work, in
 // tiles) x the tile's outputs x its cost per output.
+constexpr int kTileRows[4] = {32, 64, 128, 128}, kTileCols[4] = {32, 64, 64, 128};
 template <class Ends>
 int tile_of(int M, int N, int n, const double* cost, Ends ends) {
-  static constexpr int kBM[4] = {32, 64, 128, 128}, kBN[4] = {32, 64, 64, 128};
   const int cus = device_cus();
   int best = 0;
   double best_t = 0.0;
   for (int t = 0; t < n; ++t) {
-    const long tiles = static_cast<long>((M + kBM[t] - 1) / kBM[t]) * ((N + kBN[t] - 1) / kBN[t]);
+    const long tiles = static_cast<long>((M + kTileRows[t] - 1) / kTileRows[t]) * ((N + kTileCols[t] - 1) / kTileCols[t]);
     const long most = (tiles + cus - 1) / cus;
-    const double c = (static_cast<double>(most) + ends(most)) * kBM[t] * kBN[t] * cost[t];
+    const double c = (static_cast<double>(most) + ends(most)) * kTileRows[t] * kTileCols[t] * cost[t];
     if (t == 0 || c < best_t) {
       best = t;
       best_t = c;
@@ -812,6 +812,18 @@ bool f32_takes_pair(const GemmF32Args& p) {
 
 bool gemm_f32_rope_ok(const GemmF32Args& p, int head_dim) {
   return head_dim == 16 && p.N % 16 == 0 && f32_vec_c(p) && f32_tile_ok(p);
+}
+
+void gemm_f32_tile(int M, int N, int K, int* rows, int* cols) {
+  GemmF32Args p;
+  p.lda = p.ldw = p.K = K;
+  p.M = M;
+  p.N = N;
+  *rows = *cols = 0;
+  if (M <= 0 || N <= 0 || !f32_tile_ok(p)) return;
+  const int t = f32_takes_pair(p) ? -1 : f32_tile(p);
+  *rows = t < 0 ? 16 : kTileRows[t];
+  *cols = t < 0 ? 16 : kTileCols[t];
 }
 
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epi, hipStream_t s) {

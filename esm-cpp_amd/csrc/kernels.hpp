@@ -149,6 +149,9 @@ struct GemmF32Args {
 };
 // The order of a row's sum depends on N, K and the operands' alignment, not on M.
 hipError_t launch_gemm_f32(const GemmF32Args& p, int epilogue, hipStream_t s);
+// The tile of C that a launch of aligned operands takes, 0 x 0 for the general
+// kernel.
+void gemm_f32_tile(int M, int N, int K, int* rows, int* cols);
 // Whether the launch can take kF32QkvRope: 16-wide heads, the tiled kernel's
 // operands and whole 16-byte pieces of C.
 bool gemm_f32_rope_ok(const GemmF32Args& p, int head_dim);

@@ -232,6 +232,11 @@ int esm_gfx950_linear_i8_noalloc(esm_gfx950_ctx* ctx, const float* A, const esm_
  * C[M, N] = A[M, K] W[N, K]^T + bias (bias may be NULL). */
 int esm_gfx950_linear_f32(esm_gfx950_ctx* ctx, const float* A, const float* W, const float* bias,
                           float* C, int M, int N, int K);
+/* Host only, no counterpart in the reference: the workgroup tile of C that
+ * esm_gfx950_linear_f32 takes for these sizes and 16-byte aligned operands
+ * (16x16, 32x32, 64x64 or 128x64), or 0x0 for its general kernel. Results do
+ * not depend on it; it exists for tests. */
+int esm_gfx950_linear_f32_tile(int M, int N, int K, int* rows, int* cols);
 /* esm::kernels::LayerNorm (kernels.h:32-33; LayerNormRef layernorm.cpp:23-44). */
 int esm_gfx950_layernorm(esm_gfx950_ctx* ctx, const float* x, const float* gamma, const float* beta,
                          float eps, float* out, int num_rows, int d);

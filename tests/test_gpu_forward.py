@@ -390,15 +390,23 @@ def test_logits_do_not_depend_on_the_batch(dev, w8m, w650_small, which):
 @pytest.mark.parametrize("which", ["8m", "650m"])
 def test_decoder_rows_do_not_depend_on_the_batch(dev, w8m, w650_small, which):
     """The decoder's three kernels (up to 16 rows a CU, up to 32, and beyond:
-    about 9,000 tokens in one group) sum a row in the same order: the logits of
+    9,005 and 17,401 tokens in one group) sum a row in the same order: the logits of
     a batch, of its first half and of single sequences have the same bits. K is
-    320 (ranges of K that end inside a stage) and 1280."""
+    320 (ranges of K that end inside a stage) and 1280. The 8M batch is long
+    enough for the 128x64 tiles of the fp32 linears, with each of their
+    epilogues (RoPE, GELU, residual)."""
     w = w8m if which == "8m" else w650_small
     m = eg.Model(dev, w, int8=which != "8m", act_mode=eg.ACT_PER_TOKEN)
     m.set_parts(1)
     lengths = [66, 22] + [int(n) for n in np.random.default_rng(3).integers(100, 300, size=45)]
+    if which == "8m":
+        lengths += [200] * 41 + [17401 - sum(lengths) - 41 * 200]
     batch = syn.batch_from_lengths(lengths, seed=12)
-    assert 32 * 256 < batch.total_tokens and batch.total_tokens % 64
+    T = batch.total_tokens
+    assert 32 * 256 < T and T % 64
+    if which == "8m":
+        for N, K in ((960, 320), (1280, 320), (320, 1280)):
+            assert eg.linear_f32_tile(T, N, K) == (128, 64)
     want = m.forward_packed(batch.ids, batch.cu)
     for b0, b1 in ((0, 25), (0, 1), (1, 2), (46, 47)):
         s = slice(int(batch.cu[b0]), int(batch.cu[b1]))
