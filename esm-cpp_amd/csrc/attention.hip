@@ -368,8 +368,8 @@ __device__ __forceinline__ void split8(const float (&p)[8], f16x8* hi, f16x8* lo
 // items), or 1 where a batch has few of those. NBUF chunk buffers: with one
 // workgroup or less on a CU nothing else covers the chunk loads' latency, so
 // the QB 1 form has the loads of three chunks in flight instead of one. 20
-// heads: one sequence of 66 tokens 10.2 -> 8.6 us, of 301 18.7 -> 15.3, of 512
-// 26.7 -> 20.4; past one 64-query item a CU the smaller items' extra key reads
+// heads: one sequence of 66 tokens 9.6 -> 8.2 us, of 301 17.1 -> 13.6, of 512
+// 23.2 -> 18.3; past one 64-query item a CU the smaller items' extra key reads
 // cost more (8 x 256 tokens, 640 items: 22.8 -> 25.6).
 template <bool LONG, bool F32, int QB, int NBUF>
 __global__ __launch_bounds__(256, F32 ? 3 : QB == 1 ? 2 : 4) void attn_x3_kernel(

@@ -2221,7 +2221,6 @@ struct HiddenCapture {
 };
 
 // The whole forward of one part on ctx->stream; logits rows [0, T).
-
 int forward_part(esm_gfx950_ctx* ctx, const esm_gfx950_model* m, const esm_gfx950_model::Part& P, float* logits,
                  ObsRun* ob = nullptr, const HiddenCapture* cap = nullptr) {
   const auto& c = m->cfg;

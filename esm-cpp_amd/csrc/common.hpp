@@ -89,9 +89,13 @@ __device__ __forceinline__ float wave_max(float v) {
   return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
-// One 16-byte-per-lane global -> LDS load: a wave-uniform global base plus a
-// 32-bit lane offset, into the wave-uniform LDS byte address lds (M0). The
-// compiler does not see the LDS write: whoever reads it waits (vmcnt) first.
+// One 16-byte-per-lane global -> LDS load: a wave-uniform global base (SGPRs)
+// plus a 32-bit lane offset, one VGPR per load instead of a 64-bit address pair,
+// into the wave-uniform LDS byte address lds (M0, with one wait state before the
+// load). From inline asm, because behind the compiler's builtin its wait
+// insertion holds the reads of one stage buffer until the loads into another
+// have landed (it cannot tell the two apart). So the compiler does not see the
+// LDS write: whoever reads it waits (vmcnt) first.
 __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32_t lds) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds);
@@ -100,6 +104,8 @@ __device__ __forceinline__ void lds_dma16(const void* base, uint32_t off, uint32
 #endif
 }
 
+// LDS byte address of a __shared__ object (one address-space cast, made once,
+// instead of a null-checked cast per load).
 __device__ __forceinline__ uint32_t lds_byte_addr(const void* p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
 }

@@ -358,10 +358,12 @@ constexpr int BK = 128;
 // Tile: BLK_M 32x32 row blocks per wave, BM = 64 * BLK_M rows (1: 64, 2: 128,
 // 3: 192, 4: 256, 5: 320), and WAVES_N waves of two column blocks, BN = 64 *
 // WAVES_N columns. Which tile a launch takes: best_tile.
-// Every launch uses two column blocks a wave: two waves per SIMD. (BLK_N 4,
-// four waves of 128x128 with the accumulators in AGPRs, reads 29% fewer LDS
-// bytes per MFMA but ran 11-27% slower: one wave per SIMD leaves the matrix
-// core idle at every barrier and LDS wait.)
+// Every launch uses two column blocks a wave. The 256-wide tiles have two waves
+// per SIMD, 128x128 and (two workgroups on a CU) 64x64 one: small grids trade the
+// second wave for more CUs. (Four waves of 128x128 on a 256x256 tile, BLK_N 4 with
+// the accumulators in AGPRs, read 29% fewer LDS bytes per MFMA but ran 11-27%
+// slower on large grids: one wave per SIMD leaves the matrix core idle at every
+// barrier and LDS wait.)
 template <int BLK_M_, int BLK_N_ = 2, int WAVES_N_ = 4>
 struct Tile {
   static constexpr int BLK_M = BLK_M_, BLK_N = BLK_N_;
@@ -381,30 +383,6 @@ struct Tile {
   static constexpr int kRopeTPitch = BM + 4;
   static_assert(kBlocks % kWaves == 0, "load blocks per wave");
 };
-
-// One 16-byte-per-lane global -> LDS load (global_load_lds_dwordx4), issued
-// from inline asm: M0 holds the wave's LDS destination (uniform), and one
-// wait state separates the M0 write from the load. Issued through the
-// compiler builtin instead, the compiler's wait insertion would hold the
-// fragment reads of the other stage buffer until these loads complete (it
-// cannot tell the two buffers apart), which serialises the double buffer.
-// Completion is awaited explicitly: s_waitcnt vmcnt(0) and a barrier before
-// a stage is read. The load is addressed as a wave-uniform base (SGPRs) plus
-// a 32-bit lane offset: one VGPR per load instead of a 64-bit address pair.
-// `lds` is the destination's LDS byte address.
-__device__ __forceinline__ void dma16_async_so(const int8_t* base, uint32_t off, uint32_t lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const uint32_t m0v = __builtin_amdgcn_readfirstlane(lds);
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(m0v)
-               : "memory", "m0");
-#endif
-}
-
-// LDS byte address of a __shared__ object (one address-space cast, made
-// once, instead of a null-checked cast per load).
-__device__ __forceinline__ uint32_t lds_addr(const void* p) {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p));
-}
 
 __device__ __forceinline__ i32x16 mfma32(i32x4 a, i32x4 b, i32x16 c) {
   return __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b, c, 0, 0, 0);
@@ -841,7 +819,7 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N, WAVES_N>::kThreads), 1) void ge
     goff[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(is_a ? p.lda : p.ldw) + c * 16;
   }
   auto gbase = [&](int i) { return wave * kPer + i < BM / 8 ? pA : pW; };
-  const uint32_t ldst = lds_addr(smem) + static_cast<uint32_t>(wave * kPer * 1024);
+  const uint32_t ldst = lds_byte_addr(smem) + static_cast<uint32_t>(wave * kPer * 1024);
   // Per-row activation scales and per-column weight scales / bias of the
   // tile, read once here instead of per element in the epilogue, every item's
   // loads issued before the first LDS write (stage_scales).
@@ -905,7 +883,7 @@ __global__ __launch_bounds__((Tile<BLK_M, BLK_N, WAVES_N>::kThreads), 1) void ge
   };
   auto load_stage = [&](int st, int buf) {
 #pragma unroll
-    for (int i = 0; i < kPer; ++i) dma16_async_so(gbase(i) + st * BK, goff[i], ldst + buf * kStage + i * 1024);
+    for (int i = 0; i < kPer; ++i) lds_dma16(gbase(i) + st * BK, goff[i], ldst + buf * kStage + i * 1024);
   };
   // Tall tiles (two buffers): stage 0 first, so that its loads and the scale
   // loads are in flight together, and the scales staged behind them; the
