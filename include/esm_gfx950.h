@@ -426,7 +426,11 @@ int esm_gfx950_forward_packed(esm_gfx950_ctx* ctx, esm_gfx950_model* model, cons
  * i, and [num_layers] the post-final-LayerNorm state in place of the last
  * layer's output. The logits equal esm_gfx950_forward_packed's (the layers
  * add fc2's output into the hidden state in its GEMM; split-K partial sums
- * are not carried across a layer boundary in this call). Synchronises. */
+ * are not carried across a layer boundary in this call). Synchronises. The
+ * states' device buffer stays with the model between calls up to 256 MiB, with
+ * a stream and an event per state and group, until the model is freed; a larger
+ * buffer is given back before the call returns. It is not part of
+ * esm_gfx950_model_arena_bytes. */
 int esm_gfx950_forward_hidden_states(esm_gfx950_ctx* ctx, esm_gfx950_model* model, const int32_t* ids,
                                      const int32_t* masks, const int32_t* cu_seqlens, int batch_size,
                                      int total_tokens, float* logits, float* hidden);
@@ -539,7 +543,8 @@ int esm_gfx950_forward_with_observer(esm_gfx950_ctx* ctx, esm_gfx950_model* mode
  * form, all-fp32 models with fp32 MFMA. INVALID_ARGUMENT when the hidden size
  * is not a multiple of 32 (no split weights). No reference counterpart. */
 int esm_gfx950_model_set_lm_dense_split(esm_gfx950_ctx* ctx, esm_gfx950_model* model, int enabled);
-/* Bytes currently held by the model's device arena (for zero-growth checks). */
+/* Bytes currently held by the model's device arena (for zero-growth checks):
+ * without the weights and esm_gfx950_forward_hidden_states' kept buffer. */
 int esm_gfx950_model_arena_bytes(const esm_gfx950_model* model, size_t* bytes);
 
 #ifdef __cplusplus
