@@ -478,6 +478,12 @@ extern "C" int esm_gfx950_set_gemm_split_k(int splits) {
   return set_gemm_split_k(splits) ? ESM_GFX950_OK : ESM_GFX950_INVALID_ARGUMENT;
 }
 
+extern "C" int esm_gfx950_linear_i8_tile(int M, int N, int K, int* tile) {
+  if (!tile || M <= 0 || N <= 0 || K <= 0) return ESM_GFX950_INVALID_ARGUMENT;
+  *tile = K % 128 == 0 ? gemm_i8_tile_rows(M, N, K, kEpiF32, 0) : 0;
+  return ESM_GFX950_OK;
+}
+
 extern "C" int esm_gfx950_set_gemm_tile_rows(int rows) {
   return set_gemm_tile_rows(rows) ? ESM_GFX950_OK : ESM_GFX950_INVALID_ARGUMENT;
 }

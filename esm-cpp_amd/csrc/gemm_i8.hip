@@ -1220,32 +1220,35 @@ constexpr int kTile64x64 = 1064;
 constexpr int kTile128x128 = 1128;
 
 // A launch's estimated time in microseconds: whole rounds of workgroups over
-// the CUs at t = fixed + per_stage * stages each, and a last, partly filled
-// round at sparse * t plus the rest in proportion to its workgroups (a round
-// that leaves CUs idle runs at a higher clock and with less L2 contention).
+// the CUs at whole * t each, t = fixed + per_stage * stages, and a last, partly
+// filled round at sparse * t plus the rest in proportion to its workgroups (a
+// round that leaves CUs idle runs at a higher clock and with less L2 contention).
 // The constants are fitted to launches of N x K = 1280..10240 x 1280..10240 at
 // 30..9,000 rows; at 5120 x 1280 and 4,099 rows, for one, it gives 39 / 36 / 44
 // / 49 us for 128, 192, 256 and 320 rows, measured 40.5 / 37.5 / 42.2 / 50.4.
 struct TileCost {
   int code, rows, cols, per_cu;
-  double fixed, per_stage, sparse;
+  double fixed, per_stage, sparse, whole;
 };
 constexpr TileCost kTileCosts[] = {
     // 64x64: two share a CU; alone a workgroup takes 3.8 + 0.24 a stage. At
     // 301 rows 6.2 us (N = K = 1280), 13.1 (K = 5120), where the 64x256 tile
     // takes 8.2 and 21.9.
-    {kTile64x64, 64, 64, 2, 3.0, 0.42, 0.72},
+    {kTile64x64, 64, 64, 2, 3.0, 0.42, 0.72, 1.0},
     // 64x256 and 128x128: the same MFMAs a workgroup. 128x128 loads 32 KB a
     // stage instead of 40 and is faster over many stages: 21.1 against 22.8 us
     // at 2,048 rows, N = 1280, K = 5120. 64x256 has the shorter epilogue and
     // eight waves to fill the pipeline: 8.1 against 9.3 us at 500 rows,
     // N = 5120, K = 1280, and 12.2 against 13.3 at 850 rows, N = K = 2560.
-    {64, 64, 256, 1, 3.0, 0.445, 1.0},
-    {kTile128x128, 128, 128, 1, 3.6, 0.42, 1.0},
-    {128, 128, 256, 1, 4.0, 0.95, 0.75},
-    {192, 192, 256, 1, 6.0, 1.28, 0.72},
-    {256, 256, 256, 1, 9.0, 1.55, 0.68},
-    {320, 320, 256, 1, 13.0, 1.6, 0.72},
+    // A round that fills the CUs takes a fifth more (N = 1280, K = 5120: 21.4 us
+    // at 160 workgroups, 24.8 at 240), so two of them lose to one of 128x256:
+    // 6,000 rows 47.6 and 50.6 us against 40.6.
+    {64, 64, 256, 1, 3.0, 0.445, 1.0, 1.2},
+    {kTile128x128, 128, 128, 1, 3.6, 0.42, 1.0, 1.2},
+    {128, 128, 256, 1, 4.0, 0.95, 0.75, 1.0},
+    {192, 192, 256, 1, 6.0, 1.28, 0.72, 1.0},
+    {256, 256, 256, 1, 9.0, 1.55, 0.68, 1.0},
+    {320, 320, 256, 1, 13.0, 1.6, 0.72, 1.0},
 };
 
 long tiles_of(int M, int N, const TileCost& c) {
@@ -1257,7 +1260,7 @@ double tile_time(const TileCost& c, long workgroups, int stages, int cus) {
   const long slots = static_cast<long>(cus) * c.per_cu;
   const long whole = workgroups / slots, rest = workgroups % slots;
   const double last = rest ? t * (c.sparse + (1.0 - c.sparse) * static_cast<double>(rest) / slots) : 0.0;
-  return static_cast<double>(whole) * t + last;
+  return static_cast<double>(whole) * t * c.whole + last;
 }
 
 // The tile with the least estimated time for `splits` ranges of K.

@@ -52,7 +52,8 @@ EXPORTED = [
     "esm_gfx950_model_set_first_block_fc1_fp16", "esm_gfx950_observer_create", "esm_gfx950_observer_free",
     "esm_gfx950_observer_clear", "esm_gfx950_observer_observe", "esm_gfx950_observer_site_count",
     "esm_gfx950_observer_site_name", "esm_gfx950_observer_percentile", "esm_gfx950_forward_with_observer",
-    "esm_gfx950_attention_work_items", "esm_gfx950_linear_f32_tile", "esm_gfx950_layernorm_avx512", "esm_gfx950_gelu_avx512",
+    "esm_gfx950_attention_work_items", "esm_gfx950_linear_f32_tile", "esm_gfx950_linear_i8_tile",
+    "esm_gfx950_layernorm_avx512", "esm_gfx950_gelu_avx512",
     "esm_gfx950_expf_glibc", "esm_gfx950_linear_f32_avx512", "esm_gfx950_rope_apply_varlen_avx512",
     "esm_gfx950_attention_varlen_avx512", "esm_gfx950_model_set_numerics", "esm_gfx950_linear_i8_noalloc",
     "esm_gfx950_model_set_ffn_intermediate_bits", "esm_gfx950_linear_i8_gelu_quant_r24",
@@ -116,6 +117,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
         "esm_gfx950_scale": (i32, [vp, vp, sz, f32]),
         "esm_gfx950_rope_build_tables": (i32, [i32, i32, vp, vp]),
         "esm_gfx950_rope_apply_varlen": (i32, [vp, vp, vp, vp, vp, i32, i32, i32]),
+        "esm_gfx950_linear_i8_tile": (i32, [i32, i32, i32, C.POINTER(C.c_int)]),
         "esm_gfx950_linear_f32_tile": (i32, [i32, i32, i32, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
         "esm_gfx950_attention_work_items": (i32, [vp, i32, i32, i32, C.POINTER(sz), C.POINTER(sz)]),
         "esm_gfx950_layernorm_avx512": (i32, [vp, vp, vp, vp, f32, vp, i32, i32]),
@@ -187,6 +189,16 @@ def rope_build_tables(seq_len: int, head_dim: int):
     if rc != OK:
         raise Gfx950Error(rc, "rope_build_tables")
     return cos[:seq_len], sin[:seq_len]
+
+
+def linear_i8_tile(M: int, N: int, K: int) -> int:
+    """The tile an INT8 linear picks by itself (a value of set_gemm_tile_rows), 0
+    for its general kernel."""
+    tile = C.c_int()
+    rc = load_library().esm_gfx950_linear_i8_tile(int(M), int(N), int(K), C.byref(tile))
+    if rc != OK:
+        raise Gfx950Error(rc, "linear_i8_tile")
+    return tile.value
 
 
 def linear_f32_tile(M: int, N: int, K: int):

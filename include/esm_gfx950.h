@@ -154,6 +154,12 @@ int esm_gfx950_gemm_i8_i32(esm_gfx950_ctx* ctx, const int8_t* A, int lda, const 
  * reference counterpart. INVALID_ARGUMENT for other values. */
 int esm_gfx950_set_gemm_tile_rows(int rows);
 
+/* Host only, no counterpart in the reference: the tile that an M x N x K INT8
+ * GEMM with plain dequant output picks by itself on the whole device, as a value
+ * of esm_gfx950_set_gemm_tile_rows, or 0 for the general kernel (K not a
+ * multiple of 128). It exists for tests. */
+int esm_gfx950_linear_i8_tile(int M, int N, int K, int* tile);
+
 /* K splits of the model's out-proj and fc2 INT8 GEMMs for every later launch
  * in the process: 0 (default) chooses per launch, 1 never splits, 2..4 split
  * that many ways. A split grid writes int32 partial sums over contiguous K

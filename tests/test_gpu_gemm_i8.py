@@ -389,20 +389,22 @@ def test_linear_i8_gelu_quant_r24_rejects_bad_shapes(dev):
     w.free()
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (1, 64, 128), (70, 130, 128), (70, 130, 256), (63, 65, 384), (65, 63, 512), (130, 70, 640), (300, 1280, 768),
-    (301, 5120, 1280), (1000, 130, 1280),   # 64x64, one to ten stages in four buffers
-    (2048, 1280, 1280), (1001, 3830, 1280), (333, 10240, 2560),  # 64x256
-    (2048, 1280, 5120), (1990, 1210, 5120),  # 128x128
-    (1025, 3900, 256),  # 128x256
-    (4099, 5120, 1280), (2500, 3840, 1280), (4001, 2510, 2560),  # 192 rows
-    (9001, 5121, 384),
+@pytest.mark.parametrize("M,N,K,tile", [
+    (1, 64, 128, 1064), (70, 130, 128, 1064), (70, 130, 256, 1064), (63, 65, 384, 1064), (65, 63, 512, 1064),
+    (130, 70, 640, 1064), (300, 1280, 768, 1064), (301, 5120, 1280, 1064),
+    (1000, 130, 1280, 1064),  # one to ten stages in four buffers
+    (2048, 1280, 1280, 64), (1001, 3830, 1280, 64), (333, 10240, 2560, 64),
+    (2048, 1280, 5120, 1128), (1990, 1210, 5120, 1128),
+    (1025, 3900, 256, 128), (5999, 1275, 5120, 128),
+    (4099, 5120, 1280, 192), (2500, 3840, 1280, 192), (4001, 2510, 2560, 192), (9001, 5121, 384, 192),
+    (1599, 7670, 2560, 256), (4601, 3840, 1280, 320),
 ])
-def test_automatic_tile_edges(dev, M, N, K):
-    """Every tile, and the one that the launch picks by itself (the comments:
-    which one that is, at the time of writing), at ragged edges and few K
-    stages: the dequantised output equals the 256-row tile's bit for bit, and
-    the edge rows equal the closed form fma(acc, a_scale * w_scale, bias)."""
+def test_automatic_tile_edges(dev, M, N, K, tile):
+    """Every tile, and the one that the launch picks by itself (tile), at ragged
+    edges and few K stages: the dequantised output equals the 256-row tile's bit
+    for bit, and the edge rows equal the closed form fma(acc, a_scale * w_scale,
+    bias)."""
+    assert eg.linear_i8_tile(M, N, K) == tile
     r = rng(M + N + K)
     A = r.integers(-127, 128, size=(M, K), dtype=np.int8)
     W = r.integers(-127, 128, size=(N, K), dtype=np.int8)
