@@ -8,7 +8,7 @@
 // from the sequential reference sum only by summation order.
 //
 // Three kernels (launch_gemm_f32 picks), and the decoder's:
-//   - gemm_f32_tile_kernel: aligned rows with K % 32 == 0; LDS tiles of 32x32
+//   - gemm_f32_tile_kernel: aligned rows with K % 16 == 0; LDS tiles of 32x32
 //     to 128x64, direct global -> LDS stage loads;
 //   - gemm_f32_pair_kernel: the same operands and the same sums bit for bit, for
 //     grids too small for that one: two waves to a 16x16 tile;
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const GemmF32Args
   }
 }
 
-// ---- Tiled fp32 GEMM (K % 32 == 0, 16-byte aligned rows): 2 x 2 waves of
+// ---- Tiled fp32 GEMM (K % 16 == 0, 16-byte aligned rows): 2 x 2 waves of
 // 16 MB x 16 NB outputs, a 32 MB x 32 NB workgroup tile.
 //
 // Staging is the INT8 kernel's: K advances 128 bytes (32 floats) a stage, one
@@ -183,7 +183,9 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_f32_kernel(const GemmF32Args
 //
 // The order of an output's sum depends on K alone: over kSumStages stages one
 // sum of the first and one of the second halves, the two added, and those added
-// in turn. gemm_f32_pair_kernel has the same. Sums of 160 products keep the
+// in turn. The last half stage of a K that is an odd multiple of 16 is a sum of its
+// own, added last, its operands read straight into registers (f32_tail).
+// gemm_f32_pair_kernel has the same. Sums of 160 products keep the
 // error of the eight-way split that small grids had before, at K = 1280 0.36 of
 // one long sum's standard deviation, and cost the large tiles 1% (2560 x 2560 at
 // 16,000 rows 1,488 -> 1,501 us). A second sum also keeps a 32x32 tile's wave off
@@ -260,7 +262,15 @@ __device__ __forceinline__ void f32_out(const GemmF32Args& p, int row, int col, 
   }
 }
 
-template <bool X3, int MB, int NB, int EPI>
+// A lane's operands of the last 16 k: 4 lg .. + 4 of them, of a row of A or W.
+__device__ __forceinline__ f32x4 f32_tail(const float* base, int ld, int row, int K) {
+  return *reinterpret_cast<const f32x4*>(base + static_cast<size_t>(row) * ld + (K - 16 + 4 * ((threadIdx.x >> 4) & 3)));
+}
+
+// TAIL: K is an odd multiple of 16 (640 x 528 at 66 / 301 / 8,000 rows 4.2 / 7.0 / 54
+// us; 48.8 / 48.8 / 93.9 in the general kernel). A kernel of its own: the same
+// test made at run time cost the others four registers and up to 10%.
+template <bool X3, int MB, int NB, bool TAIL, int EPI>
 __global__ __launch_bounds__(256, MB * NB == 16 ? 1 : 3) void gemm_f32_tile_kernel(const GemmF32Args p, bool vec_c) {
   using TL = F32Tile<MB, NB>;
   constexpr int BM = TL::BM, BN = TL::BN, kPer = TL::kPer, kStage = TL::kStage, kNStage = TL::kNStage;
@@ -386,6 +396,22 @@ __global__ __launch_bounds__(256, MB * NB == 16 ? 1 : 3) void gemm_f32_tile_kern
         total[i][j] += v;
       }
   }
+  if constexpr (TAIL) {
+    f32x4 fa[MB], fw[NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i) fa[i] = f32_tail(p.A, p.lda, min(m0 + arow + 16 * i, p.M - 1), p.K);
+#pragma unroll
+    for (int j = 0; j < NB; ++j) fw[j] = f32_tail(p.W, p.ldw, min(n0 + wrow - BM + 16 * j, p.N - 1), p.K);
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[j][e], fa[i][e], v, 0, 0, 0);
+        total[i][j] += v;
+      }
+  }
 #pragma unroll
   for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -408,8 +434,8 @@ __global__ __launch_bounds__(256, MB * NB == 16 ? 1 : 3) void gemm_f32_tile_kern
 // took 3.6 / 4.7 / 8.6, before the sums were cut: the compiler waits for every
 // load in flight at the loop's head. A wave for each sum, its operands straight
 // into registers, took 3.3 / 4.4 / 6.8 to 7.8.)
-constexpr int kPairSums = 32;  // at most: K <= 32 kSumStages kPairSums
-template <int D, int EPI>
+constexpr int kPairSums = 32;  // at most, without the last half stage's: K <= 32 kSumStages kPairSums
+template <int D, bool TAIL, int EPI>
 __global__ __launch_bounds__(128) void gemm_f32_pair_kernel(const GemmF32Args p, bool vec_c) {
   constexpr int kStage = 2048;  // 1 KB of A, 1 KB of W
   __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * D * kStage];
@@ -433,6 +459,12 @@ __global__ __launch_bounds__(128) void gemm_f32_pair_kernel(const GemmF32Args p,
     fa = *reinterpret_cast<const f32x4*>(ring + slot * kStage + lane * 16);
     fw = *reinterpret_cast<const f32x4*>(ring + slot * kStage + 1024 + lane * 16);
   };
+  // The last half stage, first to be loaded, belongs to the first wave.
+  f32x4 ta, tw;
+  if (TAIL && half == 0) {
+    ta = f32_tail(p.A, p.lda, min(m0 + lr, p.M - 1), p.K);
+    tw = f32_tail(p.W, p.ldw, min(n0 + lr, p.N - 1), p.K);
+  }
   const int nk = p.K / 32;
   int slot = 0, in_sum = 0, nsum = 0;
   auto multiply = [&] {
@@ -470,6 +502,12 @@ __global__ __launch_bounds__(128) void gemm_f32_pair_kernel(const GemmF32Args p,
   if (half == 1) return;
   f32x4 total = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int x = 0; x < nsum; ++x) total += sums[0][x][lane] + sums[1][x][lane];
+  if constexpr (TAIL) {
+    f32x4 v = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v = __builtin_amdgcn_mfma_f32_16x16x4f32(tw[e], ta[e], v, 0, 0, 0);
+    total += v;
+  }
   f32_out<EPI, false>(p, m0 + lr, n0 + 4 * lg, total, vec_c);
 }
 
@@ -636,18 +674,19 @@ bool f32_vec_c(const GemmF32Args& p) { return p.ldc % 4 == 0 && reinterpret_cast
   }                                                                                           \
   return hipGetLastError()
 
-template <bool X3, int MB, int NB>
+template <bool X3, int MB, int NB, bool TAIL = false>
 hipError_t launch_f32_tile(const GemmF32Args& p, int epi, hipStream_t s) {
   using TL = F32Tile<MB, NB>;
   const bool vec_c = f32_vec_c(p);
   const dim3 grid(((p.M + TL::BM - 1) / TL::BM) * ((p.N + TL::BN - 1) / TL::BN)), block(256);
-  if constexpr (!X3) {
+  if constexpr (!X3 && !TAIL) {
+    if (p.K % 32 != 0) return launch_f32_tile<false, MB, NB, true>(p, epi, s);
     if (epi == kF32QkvRope) {
-      hipLaunchKernelGGL((gemm_f32_tile_kernel<false, MB, NB, kF32QkvRope>), grid, block, 0, s, p, vec_c);
+      hipLaunchKernelGGL((gemm_f32_tile_kernel<false, MB, NB, false, kF32QkvRope>), grid, block, 0, s, p, vec_c);
       return hipGetLastError();
     }
   }
-  ESM_F32_EPI(gemm_f32_tile_kernel, X3, MB, NB);
+  ESM_F32_EPI(gemm_f32_tile_kernel, X3, MB, NB, TAIL);
 }
 
 hipError_t launch_f32_pair(const GemmF32Args& p, int epi, hipStream_t s) {
@@ -655,10 +694,13 @@ hipError_t launch_f32_pair(const GemmF32Args& p, int epi, hipStream_t s) {
   const dim3 grid((p.M + 15) / 16, (p.N + 15) / 16), block(128);
   constexpr int kAhead = 4;  // 16 KB of LDS; 8, 12 or 16 were no faster
   if (epi == kF32QkvRope) {
-    hipLaunchKernelGGL((gemm_f32_pair_kernel<kAhead, kF32QkvRope>), grid, block, 0, s, p, vec_c);
+    hipLaunchKernelGGL((gemm_f32_pair_kernel<kAhead, false, kF32QkvRope>), grid, block, 0, s, p, vec_c);
     return hipGetLastError();
   }
-  ESM_F32_EPI(gemm_f32_pair_kernel, kAhead);
+  if (p.K % 32 != 0) {
+    ESM_F32_EPI(gemm_f32_pair_kernel, kAhead, true);
+  }
+  ESM_F32_EPI(gemm_f32_pair_kernel, kAhead, false);
 }
 
 template <int MB, int CH>
@@ -682,11 +724,11 @@ bool f32_rows_ok(const GemmF32Args& p) {
          (reinterpret_cast<uintptr_t>(p.A) | reinterpret_cast<uintptr_t>(p.W)) % 16 == 0;
 }
 
-// The tiled kernel's (and the pair kernel's) operands: whole K stages of
+// The tiled kernel's (and the pair kernel's) operands: whole and half K stages of
 // aligned rows, W within the stage loads' offsets. A beyond them goes in pieces
 // (f32_pieces), so which order a row is summed in does not depend on M.
 bool f32_tile_ok(const GemmF32Args& p) {
-  return p.K > 0 && p.K % 32 == 0 && f32_rows_ok(p) && static_cast<uint64_t>(p.N) * p.ldw * 4 <= kOffsetLimit &&
+  return p.K > 0 && p.K % 16 == 0 && f32_rows_ok(p) && static_cast<uint64_t>(p.N) * p.ldw * 4 <= kOffsetLimit &&
          static_cast<uint64_t>(p.lda) * 4 <= kOffsetLimit;
 }
 
@@ -811,7 +853,7 @@ bool f32_takes_pair(const GemmF32Args& p) {
 }  // namespace
 
 bool gemm_f32_rope_ok(const GemmF32Args& p, int head_dim) {
-  return head_dim == 16 && p.N % 16 == 0 && f32_vec_c(p) && f32_tile_ok(p);
+  return head_dim == 16 && p.N % 16 == 0 && p.K % 32 == 0 && f32_vec_c(p) && f32_tile_ok(p);
 }
 
 void gemm_f32_tile(int M, int N, int K, int* rows, int* cols) {

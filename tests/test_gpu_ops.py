@@ -103,9 +103,11 @@ def test_linear_f32(dev, oracle, M, N, K):
 
 
 @pytest.mark.parametrize("M,N,K,tile", [
-    (16, 16, 528, 0), (1, 1, 512, 16), (17, 33, 1024, 16), (65, 47, 1280, 16), (1, 4, 32, 16), (31, 33, 64, 16),
+    (16, 16, 520, 0), (1, 1, 512, 16), (17, 33, 1024, 16), (65, 47, 1280, 16), (1, 4, 32, 16), (31, 33, 64, 16),
     (33, 31, 96, 16), (64, 64, 32, 16), (65, 130, 320, 16), (5, 18, 10240, 16), (5, 18, 10272, 32),
     (1000, 333, 64, 32), (2049, 1030, 96, 32), (4133, 640, 128, 32), (9000, 322, 32, 32),
+    (1, 1, 16, 16), (17, 33, 48, 16), (20, 321, 336, 16), (20, 47, 1296, 16), (5, 18, 10256, 32), (1000, 333, 16, 32),
+    (2049, 1030, 48, 32), (1985, 2555, 336, 64), (6301, 2555, 368, 128),
     (3001, 962, 320, 64), (1985, 2555, 352, 64), (6200, 1283, 96, 64), (6010, 1283, 640, 128), (6301, 2555, 352, 128),
 ])
 @pytest.mark.parametrize("shift", [0, 1])
@@ -113,7 +115,8 @@ def test_linear_f32_tile_edges(dev, M, N, K, tile, shift):
     """Edges of the 16x16 tiles (up to the most sums they hold) and of the
     32x32, 64x64 and 128x64 tiles (tile: rows, 0 the general kernel), an N that
     is no multiple of 4, one stage and odd stage counts, K around and past the
-    320 of one partial sum; shift 1 moves every operand off its 16-byte boundary
+    320 of one partial sum, a last half stage alone, after the 320 and after a
+    part of them; shift 1 moves every operand off its 16-byte boundary
     (the general kernel). Bound: a sum of K products, each rounding at most
     2^-24 of the sum of magnitudes, 2^-24 * K * sum |a w| at worst."""
     assert eg.linear_f32_tile(M, N, K)[0] == tile
@@ -158,11 +161,11 @@ def _rows_do_not_depend_on_m(dev, N, K, shift, rows):
 
 
 @pytest.mark.parametrize("N,K,shift", [(320, 320, 0), (960, 320, 0), (320, 1280, 0), (1280, 1280, 0), (1283, 96, 0),
-                                       (47, 32, 0), (320, 1280, 1), (320, 528, 0)])
+                                       (47, 32, 0), (320, 1280, 1), (320, 520, 0), (320, 528, 0), (1283, 336, 0)])
 def test_linear_f32_rows_do_not_depend_on_their_number(dev, N, K, shift):
     """A row of linear_f32 has the same bits whatever the row count: across
     the 16x16, 32x32, 64x64 and 128x64 tiles, and in the general kernel
-    (operands off their 16-byte boundary, K % 32 != 0)."""
+    (operands off their 16-byte boundary, K % 16 != 0)."""
     _rows_do_not_depend_on_m(dev, N, K, shift, [1, 17, 66, 176, 301, 1461, 3001, 8003])
 
 
